@@ -31,13 +31,16 @@ struct ShortRangeResult {
   double virial[9] = {}; // sum over pairs of F_ij (x) d_ij, d_ij = r_i - r_j (row-major)
 };
 
-/** Cell-list pair solver.  Charged particles are counting-sorted into cells
- *  of edge >= r_cut / s, s = 2 (or 1) cells per r_cut, at most 64 per
- *  dimension; one workgroup per cell
- *  takes its particles against the (2 s + 1)^3 neighbour cells, staged through LDS
- *  with the periodic shift applied, and accumulates each particle's force in
- *  registers (FP64).  With fewer than 3 cells along a dimension it falls
- *  back to all pairs with the minimum-image displacement. */
+/** Cell-list pair solver.  Charged particles are counting-sorted into columns
+ *  along z of edge >= r_cut (>= r_cut / 2 along an axis that holds fewer than
+ *  three of those), cut into z bins; groups of 64 particles of a column take
+ *  the particles of the columns around them (k_sr_columns).  With ELC images
+ *  the sort is into cells of edge >= r_cut / s, s = 2 (or 1), at most 64 per
+ *  dimension, and one workgroup per cell takes its particles against the
+ *  (2 s + 1)^3 neighbour cells, staged through LDS with the periodic shift
+ *  applied.  Forces accumulate in registers (FP64).  With fewer than 3 cells
+ *  along a dimension it falls back to all pairs with the minimum-image
+ *  displacement. */
 class ShortRange {
 public:
   explicit ShortRange(int device);
@@ -51,7 +54,8 @@ public:
   void compute(hipStream_t st, ShortRangeParams const &p, int64_t n, double const *pos,
                double const *q, double *force, ShortRangeResult *out);
 
-  /** Cells per dimension of the last call (1 1 1: all pairs). */
+  /** Cells of edge >= r_cut / s that the box of the last call holds per
+   *  dimension (1 1 1: all pairs); the column search merges them in x and y. */
   void cells(int out[3]) const;
 
   /** Dipolar real space (DipolarP3M::pair_force / pair_energy,

@@ -148,3 +148,39 @@ def test_tuning_with_device_real_space():
         assert err <= 1.5 * acc
     with pytest.raises(ValueError, match="tuning real space"):
         P3M(prefactor=1.0, accuracy=acc).set_tuning_real_space("host")
+
+
+@pytest.mark.parametrize("box,r_cut,n,spread", [
+    ((9., 9., 9.), 2.2, 1, 1.),          # no pair at all
+    ((9., 9., 9.), 2.2, 2, 0.1),
+    ((9., 9., 9.), 2.2, 700, 0.25),      # crowded columns: full groups of 64 and a remainder
+    ((9., 9., 9.), 2.2, 2000, 1.),
+    ((5.6, 9., 9.), 2.2, 900, 1.),       # five columns of r_cut/2 along x, three wider axes
+    ((5.6, 5.7, 5.8), 2.2, 900, 1.),     # the same along x and y; z runs longer than the box
+    ((30., 8., 7.), 2.2, 64 * 20 + 1, 1.),
+    ((140., 140., 8.), 2.0, 4000, 1.),   # 64 x 64 columns: one block per group
+    ((140., 140., 8.), 2.0, 4000, 0.05),
+])
+def test_column_pairs_match_oracle(box, r_cut, n, spread):
+    """Pair forces, energy and virial of the column kernel at the edges of
+    its home groups (1 to 64 particles of a column), reaches and block
+    shares; `spread` packs the particles into a part of the box across the
+    periodic corner.  Tolerance as above: FP64 sums of the same terms."""
+    import torch
+    from oracle import oracle as O
+    rng = np.random.default_rng(n)
+    b = np.asarray(box)
+    pos = (rng.uniform(-0.5, 0.5, (n, 3)) * spread * b) % b
+    q = np.where(np.arange(n) % 2 == 0, 1., -1.) * rng.uniform(0.5, 1.5, n)
+    p3m = _actor(box, r_cut, 1.1)
+    tp, tq = torch.tensor(pos, device="cuda"), torch.tensor(q, device="cuda")
+    tf = torch.zeros_like(tp)
+    e, vir = p3m.add_short_range_forces(tp, tq, tf, energy=True, pressure=True)
+    e_ref, f_ref, v_ref = O.real_space(pos, q, box, 1.3, 1.1, r_cut, virial=True)
+    scale = max(np.sqrt(np.mean(f_ref ** 2)), 1e-300)
+    for _ in range(2):  # with energy, then forces alone
+        assert np.sqrt(np.mean((tf.cpu().numpy() - f_ref) ** 2)) <= 1e-12 * scale
+        tf.zero_()
+        p3m.add_short_range_forces(tp, tq, tf)
+    assert abs(e - e_ref) <= 1e-12 * np.sum(np.abs(e_ref))
+    assert np.max(np.abs(vir - v_ref)) <= 1e-12 * max(np.max(np.abs(v_ref)), 1e-300)
