@@ -54,16 +54,17 @@ EXPORTED_SYMBOLS = (
     "p3m_dipolar_params_default", "p3m_dipolar_create", "p3m_dipolar_destroy",
     "p3m_dipolar_last_error", "p3m_dipolar_set_params", "p3m_dipolar_get_params",
     "p3m_dipolar_activate", "p3m_dipolar_solve", "p3m_dipolar_short_range",
-    "p3m_dipolar_get_stream", "p3m_dipolar_synchronize",
+    "p3m_dipolar_get_stream", "p3m_dipolar_wait_stream", "p3m_dipolar_synchronize",
     "p3m_dipolar_set_short_range_subdivision",
-    "p3m_synchronize", "p3m_get_stream", "p3m_last_error",
+    "p3m_synchronize", "p3m_get_stream", "p3m_wait_stream", "p3m_last_error",
     "p3m_last_global_error",
     "p3m_batch_create", "p3m_batch_destroy", "p3m_batch_add_system",
     "p3m_batch_particle_offset", "p3m_batch_system_bytes",
     "p3m_batch_working_bytes", "p3m_batch_solve",
     "p3m_batch_graph_solve", "p3m_batch_set_launch_shape", "p3m_batch_get_launch_shape",
     "p3m_batch_autotune",
-    "p3m_batch_synchronize", "p3m_batch_get_stream", "p3m_batch_profile_begin",
+    "p3m_batch_synchronize", "p3m_batch_get_stream", "p3m_batch_wait_stream",
+    "p3m_batch_profile_begin",
     "p3m_batch_profile_end", "p3m_batch_last_error", "p3m_tune_model",
     "p3m_serve_create", "p3m_serve_destroy", "p3m_serve_run",
     "p3m_serve_last_error",
@@ -176,6 +177,7 @@ def load():
     shp = C.POINTER(p3m_launch_shape)
     L.p3m_autotune.argtypes = [vp, C.c_int64, vp, vp, C.c_int, shp, dp, dp]
     L.p3m_get_stream.argtypes = [vp, C.POINTER(vp)]
+    L.p3m_wait_stream.argtypes = [vp, vp]
     L.p3m_short_range.argtypes = [vp, C.c_int64, vp, vp, C.c_uint, vp, dp, dp]
     L.p3m_short_range_cells.argtypes = [vp, C.POINTER(C.c_int)]
     L.p3m_set_short_range_subdivision.argtypes = [vp, C.c_int]
@@ -198,6 +200,7 @@ def load():
     L.p3m_dipolar_solve.argtypes = [vp, C.c_int64, vp, vp, vp, vp, C.c_uint, dp]
     L.p3m_dipolar_short_range.argtypes = [vp, C.c_int64, vp, vp, vp, vp, C.c_uint, dp]
     L.p3m_dipolar_get_stream.argtypes = [vp, C.POINTER(vp)]
+    L.p3m_dipolar_wait_stream.argtypes = [vp, vp]
     L.p3m_dipolar_synchronize.argtypes = [vp]
     L.p3m_dipolar_set_short_range_subdivision.argtypes = [vp, C.c_int]
     L.p3m_last_error.argtypes = [vp]
@@ -222,6 +225,7 @@ def load():
     L.p3m_batch_autotune.argtypes = [vp, C.c_int, ip, vp, vp, vp, C.c_int, shp, dp, dp]
     L.p3m_batch_synchronize.argtypes = [vp]
     L.p3m_batch_get_stream.argtypes = [vp, C.POINTER(vp)]
+    L.p3m_batch_wait_stream.argtypes = [vp, vp]
     L.p3m_batch_profile_begin.argtypes = [vp, C.c_int]
     L.p3m_batch_profile_end.argtypes = [vp, dp, ip]
     L.p3m_batch_last_error.argtypes = [vp]
@@ -244,13 +248,11 @@ def load():
     return L
 
 
-def wait_for_torch(stream_handle):
-    """Order the solver stream after the work torch has queued so far on its
-    current stream (the producer of the device tensors handed over)."""
+def torch_stream(device):
+    """Handle of torch's current stream on the solver's device (the producer
+    of the device tensors handed over), for the *_wait_stream calls."""
     import torch
-    if stream_handle:
-        torch.cuda.ExternalStream(stream_handle).wait_stream(
-            torch.cuda.current_stream())
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def raise_for(status, ctx=None, batch=None, server=None, dipolar=None):

@@ -140,7 +140,8 @@ class P3MBatch:
         p = _device_ptr(pos, "pos", 3 * n, self.device)
         qq = _device_ptr(q, "q", n, self.device)
         f = None if force is None else _device_ptr(force, "force", 3 * n, self.device)
-        _lib.wait_for_torch(self.stream())
+        self._check(_lib.load().p3m_batch_wait_stream(
+            self._b, _lib.torch_stream(self.device)))
         return p, qq, f
 
     def solve(self, pos, q, force=None, systems=None, energy=False,

@@ -66,6 +66,7 @@ constexpr int kCountCopies = 8; // brick counter copies (one per XCD-sized share
                                 // k_scan reads a brick's copies as two 16-byte words)
 constexpr int kBrick = 8;    // first-stencil points per brick edge
 constexpr int kFill = 4096;  // mesh elements zeroed per block
+constexpr int kStamps = 8;   // stage start times of a solve
 
 /** Per-system state read by every kernel. */
 struct SysDesc {
@@ -109,6 +110,13 @@ __device__ __forceinline__ int xcd_block() {
   int const x = b & 7, k = b >> 3;
   int const q = n >> 3, r = n & 7;
   return x * q + min(x, r) + k;
+}
+
+/** Start of a stage: its first block stores the device's wall clock (100 MHz).
+ *  An event record between two kernels costs a gap of 5.6 us on the stream, a
+ *  store none. */
+__device__ __forceinline__ void stamp_start(unsigned long long *stamp) {
+  if (stamp && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *stamp = wall_clock64();
 }
 
 struct Slot {
@@ -413,7 +421,10 @@ template <typename MT>
 __global__ __launch_bounds__(kBlock) void k_clear(SysDesc const *__restrict__ sys,
                                                   int const *__restrict__ sel,
                                                   int const *__restrict__ wt, int nsel,
-                                                  int *counts, int *err_flag, int zero_rho) {
+                                                  int *counts, int *err_flag, int zero_rho,
+                                                  unsigned long long *stamps) {
+  if (blockIdx.x == 0 && threadIdx.x < kStamps)
+    stamps[threadIdx.x] = threadIdx.x ? 0ull : static_cast<unsigned long long>(wall_clock64());
   Slot const L = locate(wt, sel, nsel);
   SysDesc const &d = sys[L.s];
   if (L.vb == 0 && threadIdx.x == 0) *err_flag = 0;
@@ -655,7 +666,9 @@ __global__ __launch_bounds__(NTH, SEGMAX == 64 ? 8 : 1) void k_spread(SysDesc co
                                                int const *__restrict__ soff,
                                                int const *__restrict__ offsets,
                                                double4 const *__restrict__ spos, int chunk,
-                                               double const *__restrict__ sums, int int_mesh) {
+                                               double const *__restrict__ sums, int int_mesh,
+    unsigned long long *stamp) {
+  stamp_start(stamp);
   using GR = GroupRows<P, NTH, SX, SY, SZ>;
   constexpr int TY = GR::TY, TZ = GR::TZ;
   constexpr int TYZ = TY * TZ;
@@ -777,7 +790,9 @@ __global__ __launch_bounds__(kBlock) void k_fft_z_r2c(SysDesc const *__restrict_
                                                       int const *__restrict__ sel,
                                                       int const *__restrict__ wt, int nsel,
                                                       cx_t<MT> const *__restrict__ tw, int nlp,
-                                                      double const *__restrict__ sums, int det) {
+                                                      double const *__restrict__ sums, int det,
+    unsigned long long *stamp) {
+  stamp_start(stamp);
   using C = cx_t<MT>;
   extern __shared__ double smem_d[];
   Slot const L = locate(wt, sel, nsel);
@@ -878,7 +893,9 @@ __global__ __launch_bounds__(kBlock) void k_fft_x_conv(SysDesc const *__restrict
                                                        int const *__restrict__ wt, int nsel,
                                                        cx_t<MT> const *__restrict__ tw, int ncol,
                                                        int want_fields, int want_energy,
-                                                       double *partials) {
+                                                       double *partials,
+    unsigned long long *stamp) {
+  stamp_start(stamp);
   using C = cx_t<MT>;
   extern __shared__ double smem_d[];
   __shared__ double red[8 * 16];
@@ -970,7 +987,9 @@ template <typename MT>
 __global__ __launch_bounds__(kBlock) void k_fft_y_inv(SysDesc const *__restrict__ sys,
                                                       int const *__restrict__ sel,
                                                       int const *__restrict__ wt, int nsel,
-                                                      cx_t<MT> const *__restrict__ tw, int ncol) {
+                                                      cx_t<MT> const *__restrict__ tw, int ncol,
+    unsigned long long *stamp) {
+  stamp_start(stamp);
   using C = cx_t<MT>;
   extern __shared__ double smem_d[];
   Slot const L = locate(wt, sel, nsel);
@@ -1054,7 +1073,9 @@ __global__ __launch_bounds__(kBlock) void k_fft_yx_conv(SysDesc const *__restric
                                                         int const *__restrict__ wt, int nsel,
                                                         cx_t<MT> const *__restrict__ tw,
                                                         int want_fields, int want_energy,
-                                                        double *partials) {
+                                                        double *partials,
+    unsigned long long *stamp) {
+  stamp_start(stamp);
   using C = cx_t<MT>;
   extern __shared__ double smem_d[];
   __shared__ double red[8 * 16];
@@ -1187,7 +1208,9 @@ template <typename MT, int NC>
 __global__ __launch_bounds__(kBlock) void k_fft_z_c2r(SysDesc const *__restrict__ sys,
                                                       int const *__restrict__ sel,
                                                       int const *__restrict__ wt, int nsel,
-                                                      cx_t<MT> const *__restrict__ tw, int nlp) {
+                                                      cx_t<MT> const *__restrict__ tw, int nlp,
+    unsigned long long *stamp) {
+  stamp_start(stamp);
   using C = cx_t<MT>;
   extern __shared__ double smem_d[];
   Slot const L = locate(wt, sel, nsel);
@@ -1326,7 +1349,9 @@ __global__ __launch_bounds__(NTH) void k_gather_plane(
     SysDesc const *__restrict__ sys, int const *__restrict__ sel, int const *__restrict__ wt,
     int nsel, int const *__restrict__ soff, int const *__restrict__ offsets,
     double4 const *__restrict__ spos, int const *__restrict__ sidx, double *__restrict__ force,
-    double const *__restrict__ sums, int chunk) {
+    double const *__restrict__ sums, int chunk,
+    unsigned long long *stamp) {
+  stamp_start(stamp);
   constexpr int T = kBrick + P - 1;
   constexpr int TYZ = T * T;
   constexpr int tile_n = T * TYZ;
@@ -1439,7 +1464,9 @@ __global__ __launch_bounds__(NTH, (NTH == 512 && sizeof(MT) == 4) ? 8 : 1) void 
     SysDesc const *__restrict__ sys, int const *__restrict__ sel, int const *__restrict__ wt,
     int nsel, int const *__restrict__ soff, int const *__restrict__ offsets,
     double4 const *__restrict__ spos, int const *__restrict__ sidx, double *__restrict__ force,
-    double const *__restrict__ sums, int chunk) {
+    double const *__restrict__ sums, int chunk,
+    unsigned long long *stamp) {
+  stamp_start(stamp);
   constexpr int T = kBrick + P - 1;
   constexpr int TYZ = T * T;
   constexpr int tile_n = T * TYZ;
@@ -1620,7 +1647,9 @@ __global__ __launch_bounds__(256) void k_gather_col(
     SysDesc const *__restrict__ sys, int const *__restrict__ sel, int const *__restrict__ wt,
     int nsel, int const *__restrict__ soff, int const *__restrict__ offsets,
     double4 const *__restrict__ spos, int const *__restrict__ sidx, double *__restrict__ force,
-    double const *__restrict__ sums, int chunk) {
+    double const *__restrict__ sums, int chunk,
+    unsigned long long *stamp) {
+  stamp_start(stamp);
   using G = ColGeo<P, W>;
   constexpr int IP = G::IP;
   constexpr int PPW = 64 / S;                // particles per wave
@@ -1762,7 +1791,9 @@ __global__ __launch_bounds__(256) void k_spread_col(SysDesc const *__restrict__ 
                                                    int const *__restrict__ wt, int nsel,
                                                    int const *__restrict__ soff,
                                                    int const *__restrict__ offsets,
-                                                   double4 const *__restrict__ spos, int chunk) {
+                                                   double4 const *__restrict__ spos, int chunk,
+    unsigned long long *stamp) {
+  stamp_start(stamp);
   using G = ColGeo<P, W>;
   constexpr int IP = G::IP;
   constexpr int PPW = 64 / S;
@@ -2108,7 +2139,8 @@ struct Lane {
   double *sums = nullptr;
   int sums_cap = 0;
   int *err_flag = nullptr;
-  double *h_sums = nullptr;
+  unsigned long long *stamps = nullptr; // kStamps stage start times, after err_flag
+  double *h_sums = nullptr; // 16 per system, then the error flag and the stage times
   unsigned long long *seeds = nullptr, *h_seeds = nullptr;
   int seeds_cap = 0;
   int *tables = nullptr, *h_tables = nullptr; // plan tables (device, pinned staging)
@@ -2142,6 +2174,12 @@ struct BatchSolver::Impl {
 };
 
 namespace {
+/** Error flag and stage times of a lane: one device block. */
+constexpr size_t kStatusBytes = sizeof(unsigned long long) * (1 + kStamps);
+unsigned long long *status_stamps(int *err_flag) {
+  return reinterpret_cast<unsigned long long *>(err_flag) + 1;
+}
+
 void free_plan(Plan &p) {
   if (p.graph) (void)hipGraphExecDestroy(p.graph);
   p = Plan{};
@@ -2150,7 +2188,8 @@ void free_plan(Plan &p) {
 void create_lane(Lane &ln) {
   hip_check(hipStreamCreateWithFlags(&ln.stream, hipStreamNonBlocking), "hipStreamCreate");
   for (auto &e : ln.ev) hip_check(hipEventCreate(&e), "hipEventCreate");
-  hip_check(hipMalloc(&ln.err_flag, sizeof(int)), "hipMalloc err");
+  hip_check(hipMalloc(&ln.err_flag, kStatusBytes), "hipMalloc err");
+  ln.stamps = status_stamps(ln.err_flag);
 }
 
 void destroy_lane(Lane &ln) {
@@ -2190,6 +2229,10 @@ BatchSolver::BatchSolver(int device, MeshPrecision precision)
     : m(new Impl), m_device(device), m_prec(precision),
       m_det(precision == MeshPrecision::FP64) {
   hip_check(hipSetDevice(device), "hipSetDevice");
+  int khz = 0;
+  hip_check(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device),
+            "hipDeviceGetAttribute");
+  if (khz > 0) m_clock_khz = khz;
   m->lanes.push_back(std::make_unique<Lane>());
   create_lane(*m->lanes[0]);
   m_stream = m->lanes[0]->stream;
@@ -2732,7 +2775,7 @@ void ensure_scratch(BatchSolver::Impl *m, Lane &ln, int64_t npart, void *externa
     dfree(ln.sums);
     hip_check(hipMalloc(&ln.sums, sizeof(double) * std::max(nsys * 16, 16)), "hipMalloc sums");
     if (ln.h_sums) (void)hipHostFree(ln.h_sums);
-    hip_check(hipHostMalloc(&ln.h_sums, sizeof(double) * (std::max(nsys * 16, 16) + 8)),
+    hip_check(hipHostMalloc(&ln.h_sums, sizeof(double) * (std::max(nsys * 16, 16) + 1 + kStamps)),
               "hipHostMalloc sums");
     ln.sums_cap = nsys * 16;
   }
@@ -2753,7 +2796,8 @@ void carve_fixed(BatchSolver::Impl *m, Lane &ln, size_t table_ints, int64_t npar
     off += align256(std::max<size_t>(bytes, 1));
     return p;
   };
-  ln.err_flag = reinterpret_cast<int *>(take(sizeof(int)));
+  ln.err_flag = reinterpret_cast<int *>(take(kStatusBytes));
+  ln.stamps = status_stamps(ln.err_flag);
   ln.sums = reinterpret_cast<double *>(take(sizeof(double) * 16 * nsys));
   ln.counts = reinterpret_cast<int *>(take(sizeof(int) * kCountCopies * nb));
   ln.offsets = reinterpret_cast<int *>(take(sizeof(int) * (nb + nsys)));
@@ -2977,11 +3021,18 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
   int const ns = p.nsel;
   C const *tw = static_cast<C const *>(m->d_tw);
   SysDesc const *sys = m->d_sys;
+  // the stage's start time, from its first launch
+  unsigned stamped = 0;
+  auto stamp = [&](int k) {
+    bool const first = !(stamped & (1u << k));
+    stamped |= 1u << k;
+    return first ? ln.stamps + k : static_cast<unsigned long long *>(nullptr);
+  };
   if (ev) (void)hipEventRecord(ev[0], st);
   bool const no_spread = (flags & kSolveNoSpread) != 0;
   bool const zero_rho = !(flags & kSolveAccumulate) && !no_spread;
   k_clear<MT><<<p.blocks_fill, kBlock, 0, st>>>(sys, p.d_sel, p.wt_fill, ns, ln.counts,
-                                                ln.err_flag, zero_rho ? 1 : 0);
+                                                ln.err_flag, zero_rho ? 1 : 0, ln.stamps);
   if (p.blocks_bin > 0) {
     k_bin<<<p.blocks_bin, kBlock, 0, st>>>(sys, p.d_sel, p.wt_bin, ns, p.soff, pa, ln.counts,
                                             ln.p_brick, ln.p_rank, p_nmp, ln.bin_part,
@@ -3009,7 +3060,7 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
                              ring_points(P.value, W.value) * sizeof(double);
           k_spread_col<P.value, MT, W.value, S.value><<<g.blocks, 256, lds, st>>>(
               sys, g.d_sel, g.wt, g.nsel, p.soff, ln.offsets,
-              static_cast<double4 const *>(ln.spos), shape.chunk);
+              static_cast<double4 const *>(ln.spos), shape.chunk, stamp(1));
         });
       });
       continue;
@@ -3021,7 +3072,7 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
                                sizeof(typename SpreadWord<MT>::type);
         auto const args = std::make_tuple(sys, g.d_sel, g.wt_sp, g.nsel, p.soff, ln.offsets,
                                           static_cast<double4 const *>(ln.spos), shape.chunk,
-                                          static_cast<double const *>(ln.sums), det ? 1 : 0);
+                                          static_cast<double const *>(ln.sums), det ? 1 : 0, stamp(1));
         auto launch = [&](auto kern) {
           std::apply([&](auto... a) { kern<<<g.blocks_sp, NT.value, lds, st>>>(a...); }, args);
         };
@@ -3045,14 +3096,14 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
     return;
   }
   k_fft_z_r2c<MT><<<p.blocks_z, kBlock, p.lds_z, st>>>(sys, p.d_sel, p.wt_z, ns, tw, p.nlp_z,
-                                                       ln.sums, det ? 1 : 0);
+                                                       ln.sums, det ? 1 : 0, ln.stamps + 2);
   if (p.blocks_y > 0)
     k_fft_y<MT><<<p.blocks_y, kBlock, p.lds_y, st>>>(sys, p.d_sel, p.wt_y, ns, tw, p.ncol_y);
   if (ev) (void)hipEventRecord(ev[3], st);
   if (p.blocks_x > 0) {
     k_fft_x_conv<MT><<<p.blocks_x, kBlock, p.lds_x, st>>>(sys, p.d_sel, p.wt_x, ns, tw, p.ncol_x,
                                                           want_force ? 1 : 0, want_sums ? 1 : 0,
-                                                          ln.conv_part);
+                                                          ln.conv_part, ln.stamps + 3);
     if (want_sums)
       k_reduce_sys<<<ns, 1024, 0, st>>>(p.d_sel, p.wt_x, ns, ln.conv_part, 8, 8, ln.sums, 1);
   }
@@ -3060,7 +3111,9 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
     double *fpart = ln.conv_part + 8 * static_cast<size_t>(p.blocks_x);
     k_fft_yx_conv<MT><<<p.blocks_f, kBlock, p.lds_f, st>>>(sys, p.d_sel, p.wt_f, ns, tw,
                                                            want_force ? 1 : 0, want_sums ? 1 : 0,
-                                                           fpart);
+                                                           fpart,
+                                                           p.blocks_x > 0 ? nullptr
+                                                                          : ln.stamps + 3);
     if (want_sums)
       k_reduce_sys<<<ns, 1024, 0, st>>>(p.d_sel, p.wt_f, ns, fpart, 8, 8, ln.sums, 1);
   }
@@ -3068,13 +3121,15 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
   if (want_force) {
     if (p.blocks_yi > 0)
       k_fft_y_inv<MT><<<p.blocks_yi, kBlock, p.lds_yi, st>>>(sys, p.d_sel, p.wt_yi, ns, tw,
-                                                              p.ncol_yi);
+                                                              p.ncol_yi, ln.stamps + 4);
+    unsigned long long *const c2r_stamp = p.blocks_yi > 0 ? nullptr : ln.stamps + 4;
     if (p.c2r_comps == 3) {
       k_fft_z_c2r<MT, 3><<<p.blocks_zc, kBlock, p.lds_zc, st>>>(sys, p.d_sel, p.wt_zc, ns, tw,
-                                                                p.nlp_zc);
+                                                                p.nlp_zc, c2r_stamp);
     } else {
       dim3 const gz(p.blocks_zc, 3);
-      k_fft_z_c2r<MT, 1><<<gz, kBlock, p.lds_zc, st>>>(sys, p.d_sel, p.wt_zc, ns, tw, p.nlp_zc);
+      k_fft_z_c2r<MT, 1><<<gz, kBlock, p.lds_zc, st>>>(sys, p.d_sel, p.wt_zc, ns, tw, p.nlp_zc,
+                                                          c2r_stamp);
     }
   }
   if (ev) (void)hipEventRecord(ev[5], st);
@@ -3088,7 +3143,7 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
             k_gather_col<P.value, MT, W.value, S.value><<<g.blocks, 256, lds, st>>>(
                 sys, g.d_sel, g.wt, g.nsel, p.soff, ln.offsets,
                 static_cast<double4 const *>(ln.spos), static_cast<int const *>(ln.sidx),
-                pa.force, static_cast<double const *>(ln.sums), shape.chunk);
+                pa.force, static_cast<double const *>(ln.sums), shape.chunk, stamp(5));
           });
         });
         continue;
@@ -3101,7 +3156,7 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
               std::make_tuple(sys, g.d_sel, g.wt, g.nsel, p.soff, ln.offsets,
                               static_cast<double4 const *>(ln.spos),
                               static_cast<int const *>(ln.sidx), pa.force,
-                              static_cast<double const *>(ln.sums), shape.chunk);
+                              static_cast<double const *>(ln.sums), shape.chunk, stamp(5));
           auto launch = [&](auto kern) {
             std::apply([&](auto... a) { kern<<<g.blocks, NT.value, lds, st>>>(a...); }, args);
           };
@@ -3142,6 +3197,36 @@ __global__ void k_finalize_device(double const *__restrict__ h, double volume, d
                          h[14] + h[15]};
     for (int k = 0; k < 9; ++k) virial[k] = v[k] * prefactor / (2. * volume);
   }
+}
+
+/** End of a synchronous solve: the sums of the selected systems, the error
+ *  flag and the stage times written to pinned host memory (layout of
+ *  Lane::h_sums), instead of one copy each. */
+__global__ void k_results(int const *__restrict__ sel, int nsel, double const *__restrict__ sums,
+                          int const *__restrict__ err_flag,
+                          unsigned long long const *__restrict__ stamps, int nsys,
+                          double *__restrict__ host) {
+  unsigned long long const now = wall_clock64();
+  for (int e = threadIdx.x; e < 16 * nsel; e += blockDim.x) {
+    int const at = 16 * sel[e >> 4] + (e & 15);
+    host[at] = sums[at];
+  }
+  double *const tail = host + 16 * nsys;
+  if (threadIdx.x == 0) *reinterpret_cast<int *>(tail) = *err_flag;
+  if (threadIdx.x < kStamps)
+    reinterpret_cast<unsigned long long *>(tail + 1)[threadIdx.x] =
+        (threadIdx.x == 6) ? now : stamps[threadIdx.x];
+}
+
+/** Stage times in ms (total, then bin .. gather) from the stage start times; a
+ *  stage that did not run starts where the next one does. */
+void stage_times(unsigned long long const *stamps, double khz, float *ms) {
+  unsigned long long t[7];
+  t[6] = stamps[6];
+  for (int k = 5; k >= 0; --k) t[k] = stamps[k] ? std::min(stamps[k], t[k + 1]) : t[k + 1];
+  ms[0] = static_cast<float>(static_cast<double>(t[6] - t[0]) / khz);
+  for (int k = 1; k <= 6; ++k)
+    ms[k] = static_cast<float>(static_cast<double>(t[k] - t[k - 1]) / khz);
 }
 
 void finalize_results(BatchSolver::Impl *m, Lane const &ln, std::vector<int> const &sel,
@@ -3196,7 +3281,7 @@ void BatchSolver::solve_on(int lane, std::vector<int> const &sel, ParticleArrays
   upload_descs(m, ln.stream);
   build_plan(m, ln, sel, m_prec, m_shape);
   ensure_scratch(m, ln, ln.plan.npart, scratch, scratch_size);
-  hipEvent_t *ev = ln.ev;
+  hipEvent_t *ev = nullptr; // profiled solves only
   if (ln.profiling && static_cast<size_t>(ln.ring_used + 1) * 8 <= ln.ring.size())
     ev = &ln.ring[8 * static_cast<size_t>(ln.ring_used++)];
   if (m_det) flags |= kSolveDeterministic;
@@ -3206,24 +3291,17 @@ void BatchSolver::solve_on(int lane, std::vector<int> const &sel, ParticleArrays
     enqueue<float>(m, ln, pa, flags, m_shape, ev, nullptr, false);
   hip_check(hipGetLastError(), "P3M solve launch");
   if (!sync) return;
-  int const ns = num_systems() * 16;
-  hip_check(hipMemcpyAsync(ln.h_sums, ln.sums, sizeof(double) * ns, hipMemcpyDeviceToHost,
-                           ln.stream),
-            "copy sums");
-  hip_check(hipMemcpyAsync(ln.h_sums + ns, ln.err_flag, sizeof(int), hipMemcpyDeviceToHost,
-                           ln.stream),
-            "copy err");
+  k_results<<<1, 256, 0, ln.stream>>>(ln.plan.d_sel, ln.plan.nsel, ln.sums, ln.err_flag,
+                                      ln.stamps, num_systems(), ln.h_sums);
+  hip_check(hipGetLastError(), "P3M results");
   hip_check(hipStreamSynchronize(ln.stream), "P3M solve");
+  double const *const tail = ln.h_sums + 16 * num_systems();
   int err = 0;
-  std::memcpy(&err, ln.h_sums + ns, sizeof(int));
+  std::memcpy(&err, tail, sizeof(int));
   if (err) throw std::runtime_error("P3M: non-finite particle position");
-  float t = 0.f;
-  (void)hipEventElapsedTime(&t, ev[0], ev[6]);
-  last_ms[0] = t;
-  for (int st = 1; st <= 6; ++st) {
-    (void)hipEventElapsedTime(&t, ev[st - 1], ev[st]);
-    last_ms[st] = t;
-  }
+  unsigned long long stamps[kStamps];
+  std::memcpy(stamps, tail + 1, sizeof(stamps));
+  stage_times(stamps, m_clock_khz, last_ms);
   if (out) finalize_results(m, ln, sel, out);
 }
 

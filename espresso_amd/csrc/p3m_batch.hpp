@@ -186,6 +186,7 @@ public:
   /** Per-stage event ring for asynchronous solves (see Solver). */
   void profile_begin(int max_solves);
   int profile_end(double *stage_ms);
+  /** Stage times of the last synchronous solve (total, bin .. gather). */
   float last_ms[8] = {};
 
   /** Capture the solve of `sel` (forces, no readback) in a hipGraph and
@@ -222,6 +223,7 @@ private:
   hipStream_t m_stream = nullptr;
   LaunchShape m_shape;
   bool m_det = false;
+  double m_clock_khz = 1e5; // wall clock of the device's stage times
 };
 
 void hip_check(hipError_t err, char const *what);

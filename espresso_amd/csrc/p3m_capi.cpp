@@ -31,8 +31,32 @@
 
 using namespace espresso_amd;
 
+/** Orders a solver's stream after another stream: one event, re-recorded at
+ *  each call (a wait refers to the record at the time it was enqueued). */
+class StreamGate {
+public:
+  StreamGate() = default;
+  StreamGate(StreamGate const &) = delete;
+  StreamGate &operator=(StreamGate const &) = delete;
+  ~StreamGate() {
+    if (m_event) (void)hipEventDestroy(m_event);
+  }
+  void wait(int device, hipStream_t waiting, hipStream_t producer) {
+    if (waiting == producer) return;
+    hip_check(hipSetDevice(device), "hipSetDevice");
+    if (!m_event)
+      hip_check(hipEventCreateWithFlags(&m_event, hipEventDisableTiming), "hipEventCreate");
+    hip_check(hipEventRecord(m_event, producer), "hipEventRecord");
+    hip_check(hipStreamWaitEvent(waiting, m_event, 0), "hipStreamWaitEvent");
+  }
+
+private:
+  hipEvent_t m_event = nullptr;
+};
+
 struct p3m_context {
   int device = 0;
+  StreamGate gate;
   std::unique_ptr<Solver> solver;
   std::unique_ptr<ShortRange> short_range; // created on first use
   int short_range_subdivision = 0;
@@ -66,6 +90,7 @@ struct p3m_context {
 
 struct p3m_dipolar {
   int device = 0;
+  StreamGate gate;
   std::unique_ptr<DipolarSolver> solver;
   p3m_dipolar_params user{};
   bool have_params = false;
@@ -77,6 +102,7 @@ struct p3m_dipolar {
 
 struct p3m_batch {
   int device = 0;
+  StreamGate gate;
   // shared with the servers built over the batch, which keep the solver
   // alive when the batch handle is destroyed before them
   std::shared_ptr<BatchSolver> solver;
@@ -1251,6 +1277,13 @@ int p3m_get_stream(p3m_context const *ctx, void **stream) {
   return P3M_OK;
 }
 
+int p3m_wait_stream(p3m_context *ctx, void *producer) {
+  if (!ctx || !ctx->solver) return P3M_ERR_INVALID;
+  return guarded(ctx, [&] {
+    ctx->gate.wait(ctx->device, ctx->solver->stream(), static_cast<hipStream_t>(producer));
+  });
+}
+
 char const *p3m_last_error(p3m_context const *ctx) {
   return ctx ? ctx->last_error.c_str() : "null context";
 }
@@ -1451,6 +1484,13 @@ int p3m_batch_get_stream(p3m_batch const *b, void **stream) {
   if (!b || !stream) return P3M_ERR_INVALID;
   *stream = static_cast<void *>(b->solver->stream());
   return P3M_OK;
+}
+
+int p3m_batch_wait_stream(p3m_batch *b, void *producer) {
+  if (!b) return P3M_ERR_INVALID;
+  return guarded(&b->last_error, [&] {
+    b->gate.wait(b->device, b->solver->stream(), static_cast<hipStream_t>(producer));
+  });
 }
 
 int p3m_batch_profile_begin(p3m_batch *b, int max_solves) {
@@ -1881,6 +1921,13 @@ int p3m_dipolar_get_stream(p3m_dipolar const *c, void **stream) {
   if (!c || !stream || !c->solver) return P3M_ERR_INVALID;
   *stream = reinterpret_cast<void *>(c->solver->stream());
   return P3M_OK;
+}
+
+int p3m_dipolar_wait_stream(p3m_dipolar *c, void *producer) {
+  if (!c || !c->solver) return P3M_ERR_INVALID;
+  return guarded(&c->last_error, [&] {
+    c->gate.wait(c->device, c->solver->stream(), static_cast<hipStream_t>(producer));
+  });
 }
 
 int p3m_dipolar_synchronize(p3m_dipolar *c) {

@@ -115,6 +115,7 @@ class _Arrays:
                  asynchronous=False):
         self.keep = []
         self.device = _is_device_tensor(pos)
+        self.device_id = device
         if self.device:
             if not getattr(q, "is_cuda", False):
                 raise TypeError("'q' must be a device tensor too")
@@ -164,9 +165,8 @@ class _Arrays:
     def order_after_torch(self, ctx):
         """Device tensors: the solver stream waits for torch's stream."""
         if self.device:
-            s = C.c_void_p()
-            _lib.raise_for(_lib.load().p3m_get_stream(ctx, C.byref(s)), ctx)
-            _lib.wait_for_torch(s.value)
+            _lib.raise_for(_lib.load().p3m_wait_stream(
+                ctx, _lib.torch_stream(self.device_id)), ctx)
 
 
 def _is_device_tensor(x):

@@ -27,6 +27,7 @@ class _Vec:
     def __init__(self, pos, dip, force=None, torque=None, device=0, asynchronous=False):
         self.keep = []
         self.device = _is_device_tensor(pos)
+        self.device_id = device
         outs = []
         if self.device:
             if int(pos.numel()) % 3:
@@ -65,9 +66,8 @@ class _Vec:
     def order_after_torch(self, ctx):
         """Device tensors: the solver stream waits for torch's stream."""
         if self.device:
-            s = C.c_void_p()
-            _lib.raise_for(_lib.load().p3m_dipolar_get_stream(ctx, C.byref(s)), dipolar=ctx)
-            _lib.wait_for_torch(s.value)
+            _lib.raise_for(_lib.load().p3m_dipolar_wait_stream(
+                ctx, _lib.torch_stream(self.device_id)), dipolar=ctx)
 
 
 class DipolarP3M:

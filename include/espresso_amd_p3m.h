@@ -348,6 +348,7 @@ int p3m_dipolar_short_range(p3m_dipolar *ctx, int64_t n, const double *pos, cons
  * cells when they hold about 40 dipoles or more), 1 or 2. */
 int p3m_dipolar_set_short_range_subdivision(p3m_dipolar *ctx, int cells_per_cutoff);
 int p3m_dipolar_get_stream(const p3m_dipolar *ctx, void **stream);
+int p3m_dipolar_wait_stream(p3m_dipolar *ctx, void *producer); /* as p3m_wait_stream */
 int p3m_dipolar_synchronize(p3m_dipolar *ctx);
 
 /* Real-space cost that timed tuning (p3m_activate with tune set) adds to
@@ -445,6 +446,10 @@ int p3m_synchronize(p3m_context *ctx);
 /* Device stream of the context (hipStream_t) for callers that enqueue
  * around the solver. */
 int p3m_get_stream(const p3m_context *ctx, void **stream);
+/* Order the context's stream after the work queued so far on `producer` (a
+ * hipStream_t of the same device, null for the default stream), the stream
+ * that makes the arrays of the next call. */
+int p3m_wait_stream(p3m_context *ctx, void *producer);
 
 const char *p3m_last_error(const p3m_context *ctx);
 const char *p3m_last_global_error(void);
@@ -496,6 +501,7 @@ int p3m_batch_autotune(p3m_batch *b, int nsel, const int *sys_ids, const double 
                        double *best_ms, double *default_ms);
 int p3m_batch_synchronize(p3m_batch *b);
 int p3m_batch_get_stream(const p3m_batch *b, void **stream);
+int p3m_batch_wait_stream(p3m_batch *b, void *producer); /* as p3m_wait_stream */
 int p3m_batch_profile_begin(p3m_batch *b, int max_solves);
 int p3m_batch_profile_end(p3m_batch *b, double *stage_ms, int *nsolves);
 const char *p3m_batch_last_error(const p3m_batch *b);
