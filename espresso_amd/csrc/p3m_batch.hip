@@ -67,6 +67,12 @@ constexpr int kCountCopies = 8; // brick counter copies (one per XCD-sized share
 constexpr int kBrick = 8;    // first-stencil points per brick edge
 constexpr int kFill = 4096;  // mesh elements zeroed per block
 constexpr int kStamps = 8;   // stage start times of a solve
+constexpr int kWideBlock = 512;    // threads of a k_fft_yx_conv_wide block
+// kz columns of a selection up to which that kernel runs: 384 blocks, three
+// component blocks to every two CUs (mesh 32 FP64: 13.1 against 22.8 us, mesh
+// 64 FP32: 19.7 against 44.8; with the chip filled by whole columns, 256
+// systems, the one-block pass does 7 line passes where this one does 12)
+constexpr int kWideColumns = 128;
 
 /** Per-system state read by every kernel. */
 struct SysDesc {
@@ -1197,8 +1203,122 @@ __global__ __launch_bounds__(kBlock) void k_fft_yx_conv(SysDesc const *__restric
   }
 }
 
+/** The fused y/x pass spread over three blocks per kz column, one per field
+ *  component, for selections with too few columns to fill the chip: each block
+ *  repeats the forward transforms and takes one component through the inverse
+ *  ones, 4 line passes instead of 7 one after the other.  A single system of
+ *  mesh 32 has 17 columns, and its pass is a chain of barriers and LDS
+ *  latencies, not bandwidth.  The arithmetic of every output is that of
+ *  k_fft_yx_conv, so that a system gives the same bits in either kernel.  The
+ *  siblings read khat, so the y component goes to a buffer of its own, ybuf,
+ *  column idx of the selection at ycol[slot] + kz pl. */
+template <typename MT>
+__global__ __launch_bounds__(kWideBlock) void k_fft_yx_conv_wide(
+    SysDesc const *__restrict__ sys, int const *__restrict__ sel, int const *__restrict__ wt,
+    int nsel, cx_t<MT> const *__restrict__ tw, int want_fields, int want_energy, double *partials,
+    cx_t<MT> *__restrict__ ybuf, int const *__restrict__ ycol, unsigned long long *stamp) {
+  stamp_start(stamp);
+  using C = cx_t<MT>;
+  extern __shared__ double smem_d[];
+  __shared__ double red[8 * 16];
+  int const ncomp = want_fields ? 3 : 1;
+  int const idx = static_cast<int>(blockIdx.x) / ncomp;
+  int const comp = static_cast<int>(blockIdx.x) - idx * ncomp;
+  int const slot = find_slot(wt, nsel, idx);
+  int const kz = idx - wt[slot];
+  SysDesc const &d = sys[sel[slot]];
+  int const Mx = d.g.M[0], My = d.g.M[1], Mz = d.g.M[2];
+  int const lsy = My + 1, lsx = Mx + 1;
+  int const plane = max(Mx * lsy, My * lsx);
+  int const pl = Mx * My;
+  FastDiv const fMy = make_fastdiv(My);
+  C *twx = reinterpret_cast<C *>(smem_d);
+  C *twy = twx + Mx;
+  C *P0 = twy + My;
+  C *P1 = P0 + plane;
+  load_twiddles(twx, tw + d.tw_off[0], Mx);
+  load_twiddles(twy, tw + d.tw_off[1], My);
+  C const *const col = static_cast<C const *>(d.khat) + (int64_t)kz * pl;
+  MT const *const G = static_cast<MT const *>(d.G) + (int64_t)kz * pl;
+  for (int e = threadIdx.x; e < pl; e += kWideBlock) {
+    int const x = fdiv(e, fMy), y = e - x * My;
+    P0[x * lsy + y] = col[e];
+  }
+  __syncthreads();
+  C *r = lds_fft(P0, P1, Mx, lsy, d.plan[1], twy, false); // along y
+  C *o = (r == P0) ? P1 : P0;
+  C *q = lds_fft_cols(r, o, My, lsy, d.plan[0], twx, false); // along x
+  C *w = (q == r) ? o : r;
+  double const wvx = d.wv[0], wvy = d.wv[1], wvz = d.wv[2];
+  if (want_energy && comp == 0) {
+    // the first kBlock threads, in k_fft_yx_conv's order of the sums
+    double acc[8] = {0., 0., 0., 0., 0., 0., 0., 0.};
+    double const wgt = (kz == 0 || 2 * kz == Mz) ? 1. : 2.;
+    double const kzv = dop_shift(kz, Mz) * wvz;
+    if (threadIdx.x < kBlock) {
+      for (int e = threadIdx.x; e < pl; e += kBlock) {
+        int const x = fdiv(e, fMy), y = e - x * My;
+        C const rh = q[x * lsy + y];
+        double const ek = static_cast<double>(G[e]) *
+                          (static_cast<double>(rh.x) * rh.x + static_cast<double>(rh.y) * rh.y);
+        double const kx = dop_shift(x, Mx) * wvx;
+        double const ky = dop_shift(y, My) * wvy;
+        double const norm_sq = kx * kx + ky * ky + kzv * kzv;
+        acc[0] += wgt * ek;
+        if (norm_sq != 0.) {
+          double const pref = wgt * ek * (-2. * (1. / norm_sq + d.hais));
+          acc[1] += pref * kx * kx;
+          acc[2] += pref * kx * ky;
+          acc[3] += pref * kx * kzv;
+          acc[4] += pref * ky * ky;
+          acc[5] += pref * ky * kzv;
+          acc[6] += pref * kzv * kzv;
+          acc[7] += wgt * ek;
+        }
+      }
+    }
+    block_sum<8>(acc, red);
+    if (threadIdx.x == 0)
+      for (int k = 0; k < 8; ++k) partials[idx * 8 + k] = acc[k];
+  }
+  if (!want_fields) return;
+  // phi, or i k_x phi, in place
+  for (int e = threadIdx.x; e < pl; e += kWideBlock) {
+    int const x = fdiv(e, fMy), y = e - x * My;
+    C const rh = q[x * lsy + y];
+    MT const gv = G[e];
+    C v = C{gv * rh.x, gv * rh.y};
+    if (comp == 0) {
+      MT const kf = static_cast<MT>(ik_shift(x, Mx, d.g.conv)) * static_cast<MT>(wvx);
+      v = C{-kf * v.y, kf * v.x};
+    }
+    q[x * lsy + y] = v;
+  }
+  __syncthreads();
+  C *a = lds_fft_cols(q, w, My, lsy, d.plan[0], twx, true);
+  C *b = (a == q) ? w : q;
+  if (comp == 1) {
+    for (int e = threadIdx.x; e < pl; e += kWideBlock) {
+      int const x = fdiv(e, fMy), y = e - x * My;
+      C const v = a[x * lsy + y];
+      MT const kf = static_cast<MT>(ik_shift(y, My, d.g.conv)) * static_cast<MT>(wvy);
+      a[x * lsy + y] = C{-kf * v.y, kf * v.x};
+    }
+    __syncthreads();
+  }
+  C *c = lds_fft(a, b, Mx, lsy, d.plan[1], twy, true);
+  C *const out = (comp == 0) ? static_cast<C *>(d.B) + (int64_t)kz * pl
+                 : (comp == 1) ? ybuf + ycol[slot] + (int64_t)kz * pl
+                               : static_cast<C *>(d.A) + (int64_t)kz * pl;
+  for (int e = threadIdx.x; e < pl; e += kWideBlock) {
+    int const x = fdiv(e, fMy), y = e - x * My;
+    out[e] = c[x * lsy + y];
+  }
+}
+
 /** inverse c2r along z of the three field components (x from B into rho,
- *  y from khat into Ey, z from A times i k_z into Ez), two half-spectrum
+ *  y from khat, or from ybuf after k_fft_yx_conv_wide, into Ey, z from A
+ *  times i k_z into Ez), two half-spectrum
  *  rows per complex line.  NC = 3: a block takes the same nlp line pairs of
  *  all three components (shared index arithmetic, six loads per element in
  *  flight, one batched LDS transform of 3 nlp lines); NC = 1: blockIdx.y
@@ -1209,6 +1329,8 @@ __global__ __launch_bounds__(kBlock) void k_fft_z_c2r(SysDesc const *__restrict_
                                                       int const *__restrict__ sel,
                                                       int const *__restrict__ wt, int nsel,
                                                       cx_t<MT> const *__restrict__ tw, int nlp,
+                                                      cx_t<MT> const *__restrict__ ybuf,
+                                                      int const *__restrict__ ycol,
     unsigned long long *stamp) {
   stamp_start(stamp);
   using C = cx_t<MT>;
@@ -1222,7 +1344,8 @@ __global__ __launch_bounds__(kBlock) void k_fft_z_c2r(SysDesc const *__restrict_
   int const Kz = d.g.Kz;
   FastDiv const fn = make_fastdiv(n), fnl = make_fastdiv(nlp);
   int const c0 = (NC == 3) ? 0 : static_cast<int>(blockIdx.y);
-  C const *S[3] = {static_cast<C const *>(d.B), static_cast<C const *>(d.khat),
+  C const *S[3] = {static_cast<C const *>(d.B),
+                   (ybuf && d.kzmajor) ? ybuf + ycol[L.slot] : static_cast<C const *>(d.khat),
                    static_cast<C const *>(d.A)};
   MT *E[3] = {static_cast<MT *>(d.rho), static_cast<MT *>(d.Ey), static_cast<MT *>(d.Ez)};
   double const wvz = d.wv[2];
@@ -2096,7 +2219,8 @@ struct Plan {
   int nsel = 0;
   int *dbuf = nullptr; // device copy of all tables below (owned by the lane)
   int *d_sel = nullptr, *wt_bin = nullptr, *wt_fill = nullptr, *wt_z = nullptr, *wt_zc = nullptr,
-      *wt_y = nullptr, *wt_x = nullptr, *wt_yi = nullptr, *wt_f = nullptr;
+      *wt_y = nullptr, *wt_x = nullptr, *wt_yi = nullptr, *wt_f = nullptr, *ycol = nullptr;
+  bool wide = false; // fused pass with a block per column and component
   int blocks_bin = 0, blocks_fill = 0, blocks_z = 0, blocks_zc = 0, blocks_y = 0, blocks_x = 0,
       blocks_yi = 0, blocks_f = 0;
   int *soff = nullptr; // per system id: first particle of the system in the lane scratch
@@ -2134,6 +2258,8 @@ struct Lane {
   double4 *spos = nullptr;
   void *own = nullptr;
   size_t own_bytes = 0;
+  void *ybuf = nullptr; // y field of the wide fused pass
+  size_t ybuf_bytes = 0;
   double *bin_part = nullptr, *conv_part = nullptr;
   int bin_cap = 0, conv_cap = 0;
   double *sums = nullptr;
@@ -2199,6 +2325,8 @@ void destroy_lane(Lane &ln) {
   dfree(ln.offsets);
   if (ln.own) (void)hipFree(ln.own);
   ln.own = nullptr;
+  if (ln.ybuf) (void)hipFree(ln.ybuf);
+  ln.ybuf = nullptr;
   dfree(ln.bin_part);
   dfree(ln.conv_part);
   dfree(ln.sums);
@@ -2520,6 +2648,7 @@ template <typename MT> void set_kernel_attrs() {
   allow_lds(k_fft_x_conv<MT>);
   allow_lds(k_fft_y_inv<MT>);
   allow_lds(k_fft_yx_conv<MT>);
+  allow_lds(k_fft_yx_conv_wide<MT>);
   for (int cao = 1; cao <= 7; ++cao)
     dispatch_cao(cao, [&](auto P) {
       for_threads([&](auto NT) {
@@ -2537,6 +2666,21 @@ template <typename MT> void set_kernel_attrs() {
         allow_lds(k_gather_col<P.value, MT, W.value, S.value>);
       });
     });
+}
+
+/** Function attributes of the current device's kernels, set once per device
+ *  and precision (some 200 runtime calls, 0.5 ms). */
+void prepare_kernels(int device, MeshPrecision prec) {
+  static std::mutex mu;
+  static std::map<std::pair<int, MeshPrecision>, bool> done;
+  std::lock_guard<std::mutex> lock(mu);
+  bool &ready = done[{device, prec}];
+  if (ready) return;
+  if (prec == MeshPrecision::FP64)
+    set_kernel_attrs<double>();
+  else
+    set_kernel_attrs<float>();
+  ready = true;
 }
 
 /** G on the half spectrum in the system's layout (FP64 arithmetic). */
@@ -2619,10 +2763,7 @@ int BatchSolver::add_system(P3MParams const &params_in, Vec3d const &box_l, doub
   hip_check(hipSetDevice(m_device), "hipSetDevice");
   quiesce(m);
   if (!m->kernels_ready) {
-    if (m_prec == MeshPrecision::FP64)
-      set_kernel_attrs<double>();
-    else
-      set_kernel_attrs<float>();
+    prepare_kernels(m_device, m_prec);
     m->kernels_ready = true;
   }
   HostSys h;
@@ -2851,6 +2992,16 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
   p.nlp_zc = pick_lines(max_mz, csz, 6, shape.zlines, budget);
   p.c2r_comps = (p.nlp_zc >= p.nlp_z) ? 3 : 1;
   if (p.c2r_comps == 1) p.nlp_zc = p.nlp_z;
+  // small selections: fewer line pairs per block until the passes have a block
+  // for every CU (mesh 32: 32 blocks of 16 pairs took 6.4 us, 128 of 4 5.4)
+  int64_t pairs = 0;
+  for (int s : sel) {
+    auto const &g = m->sys.at(s).desc.g;
+    pairs += (static_cast<int64_t>(g.M[0]) * g.M[1] + 1) / 2;
+  }
+  while (p.nlp_z > 4 && pairs < 256 * static_cast<int64_t>(p.nlp_z)) p.nlp_z = (p.nlp_z + 1) / 2;
+  while (p.nlp_zc > 4 && pairs * (p.c2r_comps == 1 ? 3 : 1) < 256 * static_cast<int64_t>(p.nlp_zc))
+    p.nlp_zc = (p.nlp_zc + 1) / 2;
   p.ncol_y = pick_lines(max_my, csz, 2, shape.ncol, budget);
   p.ncol_x = pick_lines(max_mx, csz, 4, shape.ncol, budget);
   p.ncol_yi = pick_lines(max_my, csz, 3, shape.ncol, budget);
@@ -2904,6 +3055,13 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
     return h.desc.kzmajor ? 0 : ((h.desc.g.Kz + ncyi - 1) / ncyi) * h.desc.g.M[0];
   });
   auto const ff = push_prefix([](HostSys const &h) { return h.desc.kzmajor ? h.desc.g.Kz : 0; });
+  // y field of the wide fused pass (not in the fixed scratch): at most
+  // kWideColumns planes
+  p.wide = !ln.fixed && ff.second > 0 && ff.second <= kWideColumns;
+  auto const yc = push_prefix([&p](HostSys const &h) {
+    DevGeo const &g = h.desc.g;
+    return p.wide && h.desc.kzmajor ? g.Kz * g.M[0] * g.M[1] : 0;
+  });
   struct GH {
     int cao, sel_start, nsel, wt_start, blocks, wsp_start, blocks_sp;
   };
@@ -2987,6 +3145,7 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
   p.wt_yi = p.dbuf + fyi.first;
   p.blocks_yi = fyi.second;
   p.wt_f = p.dbuf + ff.first;
+  p.ycol = p.dbuf + yc.first;
   p.blocks_f = ff.second;
   p.soff = p.dbuf + soff_start;
   p.npart = npart;
@@ -3000,6 +3159,14 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
     hip_check(hipMalloc(&ln.bin_part, sizeof(double) * 8 * std::max(p.blocks_bin, 1)),
               "hipMalloc bin partials");
     ln.bin_cap = p.blocks_bin;
+  }
+  size_t const ybytes = static_cast<size_t>(yc.second) * csz;
+  if (ybytes > ln.ybuf_bytes) {
+    if (ln.ybuf) (void)hipFree(ln.ybuf); // the stream is idle (synchronised above)
+    ln.ybuf = nullptr;
+    ln.ybuf_bytes = 0;
+    hip_check(hipMalloc(&ln.ybuf, ybytes), "hipMalloc y field");
+    ln.ybuf_bytes = ybytes;
   }
   int const conv_blocks = p.blocks_x + p.blocks_f; // split partials, then fused
   if (conv_blocks > ln.conv_cap) {
@@ -3020,6 +3187,7 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
   bool const want_sums = (flags & 6u) != 0; // energy or virial (P3M_ENERGY | P3M_PRESSURE)
   int const ns = p.nsel;
   C const *tw = static_cast<C const *>(m->d_tw);
+  C *const ybuf = p.wide ? static_cast<C *>(ln.ybuf) : nullptr;
   SysDesc const *sys = m->d_sys;
   // the stage's start time, from its first launch
   unsigned stamped = 0;
@@ -3109,11 +3277,15 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
   }
   if (p.blocks_f > 0) {
     double *fpart = ln.conv_part + 8 * static_cast<size_t>(p.blocks_x);
-    k_fft_yx_conv<MT><<<p.blocks_f, kBlock, p.lds_f, st>>>(sys, p.d_sel, p.wt_f, ns, tw,
-                                                           want_force ? 1 : 0, want_sums ? 1 : 0,
-                                                           fpart,
-                                                           p.blocks_x > 0 ? nullptr
-                                                                          : ln.stamps + 3);
+    unsigned long long *const f_stamp = p.blocks_x > 0 ? nullptr : ln.stamps + 3;
+    if (p.wide)
+      k_fft_yx_conv_wide<MT><<<p.blocks_f * (want_force ? 3 : 1), kWideBlock, p.lds_f, st>>>(
+          sys, p.d_sel, p.wt_f, ns, tw, want_force ? 1 : 0, want_sums ? 1 : 0, fpart, ybuf,
+          p.ycol, f_stamp);
+    else
+      k_fft_yx_conv<MT><<<p.blocks_f, kBlock, p.lds_f, st>>>(sys, p.d_sel, p.wt_f, ns, tw,
+                                                             want_force ? 1 : 0,
+                                                             want_sums ? 1 : 0, fpart, f_stamp);
     if (want_sums)
       k_reduce_sys<<<ns, 1024, 0, st>>>(p.d_sel, p.wt_f, ns, fpart, 8, 8, ln.sums, 1);
   }
@@ -3125,11 +3297,12 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
     unsigned long long *const c2r_stamp = p.blocks_yi > 0 ? nullptr : ln.stamps + 4;
     if (p.c2r_comps == 3) {
       k_fft_z_c2r<MT, 3><<<p.blocks_zc, kBlock, p.lds_zc, st>>>(sys, p.d_sel, p.wt_zc, ns, tw,
-                                                                p.nlp_zc, c2r_stamp);
+                                                                p.nlp_zc, ybuf, p.ycol,
+                                                                c2r_stamp);
     } else {
       dim3 const gz(p.blocks_zc, 3);
       k_fft_z_c2r<MT, 1><<<gz, kBlock, p.lds_zc, st>>>(sys, p.d_sel, p.wt_zc, ns, tw, p.nlp_zc,
-                                                          c2r_stamp);
+                                                          ybuf, p.ycol, c2r_stamp);
     }
   }
   if (ev) (void)hipEventRecord(ev[5], st);

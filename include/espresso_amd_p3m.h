@@ -376,8 +376,8 @@ int p3m_pair_force(const p3m_context *ctx, double q1q2, const double d[3], doubl
                    double out[3]);
 int p3m_pair_energy(const p3m_context *ctx, double q1q2, double dist, double *out);
 
-/* Timing of the last solve on the device (ms), from HIP events on the
- * context stream: [0] total, then per stage (bin, spread, fft_fwd,
+/* Timing of the last synchronous solve on the device (ms), from clock stamps
+ * of its stages: [0] total, then per stage (bin, spread, fft_fwd,
  * convolve, fft_bwd, gather). */
 int p3m_last_timings(const p3m_context *ctx, double *ms, int n);
 

@@ -286,3 +286,43 @@ def test_launch_shape_validation():
     b.set_launch_shape(threads=256, chunk=64, gather_threads=512)
     got = b.launch_shape()
     assert got["threads"] == 256 and got["gather_threads"] == 512
+
+
+@pytest.mark.parametrize("single", [False, True])
+def test_wide_fused_pass_matches_the_one_block_pass(single):
+    """Selections of few kz columns run the fused y/x pass with one block per
+    column and component; the same systems in a selection of many columns run
+    it with one block per column.  Meshes with unequal edges and every kind of
+    radix; both kernels do the same arithmetic, so FP64 results (deterministic
+    spread) are equal bit for bit, FP32 ones to the rounding of the spread."""
+    import torch
+    from espresso_amd import P3MBatch
+    # z edges alike, so that both selections take the same form of the z passes
+    meshes = [(8, 8, 28), (16, 12, 32), (22, 14, 30), (30, 32, 28), (48, 40, 32), (40, 44, 30),
+              (34, 26, 32), (36, 36, 30), (46, 38, 28), (28, 28, 28)]
+    rng = np.random.default_rng(17)
+    b = P3MBatch(single_precision=single)
+    pos, q = [], []
+    for k, mesh in enumerate(meshes):
+        n = 400 + 37 * k
+        box = [0.5 * m for m in mesh]
+        b.add_system(box_l=box, n=n, prefactor=1., mesh=mesh, cao=3 + k % 3, alpha=0.8, r_cut=1.5)
+        pos.append(rng.uniform(0., 1., (n, 3)) * box)
+        q.append(np.where(np.arange(n) % 2 == 0, 1., -1.))
+    tp = torch.tensor(np.concatenate(pos), device="cuda")
+    tq = torch.tensor(np.concatenate(q), device="cuda")
+    f_all = torch.zeros_like(tp)
+    e_all, v_all = b.solve(tp, tq, f_all, energy=True, pressure=True)  # 159 columns
+    at = 0
+    for k in range(len(meshes)):
+        f = torch.zeros_like(tp)
+        e, v = b.solve(tp, tq, f, systems=[k], energy=True, pressure=True)
+        one, mix = f[at:at + len(q[k])], f_all[at:at + len(q[k])]
+        at += len(q[k])
+        if single:
+            assert S.rel_rms(one.cpu().numpy(), mix.cpu().numpy()) <= 1e-5
+        else:
+            assert torch.equal(one, mix), meshes[k]
+            assert e[0] == e_all[k] and np.array_equal(v[0], v_all[k])
+        e_only, _ = b.solve(tp, tq, None, systems=[k], energy=True)
+        assert abs(e_only[0] - e[0]) <= (2e-6 if single else 1e-12) * (abs(e[0]) + len(q[k]))
