@@ -297,3 +297,29 @@ def test_actor_autotune_keeps_forces():
         p3m.add_long_range_forces(tp, tq, f)
         tol = 1e-5 if single else 1e-12
         assert S.rel_rms(f.cpu().numpy(), ref.cpu().numpy()) <= tol
+
+
+@pytest.mark.parametrize("single", [False, True])
+@pytest.mark.parametrize("n,mesh,cao", [(1, 8, 3), (3, 8, 5), (400, 8, 4), (4000, 16, 7),
+                                        (9001, 24, 1), (12000, 40, 6)])
+def test_shared_bricks_match_oracle(n, mesh, cao, single):
+    """Few crowded bricks are shared by up to 128 blocks; one brick, shares
+    without particles, and systems at the edge of the rule.  Tolerances of the
+    parity tests (FP64 1e-6, FP32 mesh 2e-5 rel-rms)."""
+    import torch
+    from espresso_amd.electrostatics import P3M
+    from oracle.oracle import OracleP3M
+    rng = np.random.default_rng(n)
+    L = 9.
+    pos = rng.uniform(0., L, (n, 3))
+    pos[: n // 3] *= 0.3  # one corner is more crowded
+    q = rng.choice([-1., 1., 0.], n)
+    q[0] = 1.
+    p = P3M(prefactor=1.2, accuracy=1e-3, mesh=mesh, cao=cao, r_cut=2., alpha=1.0, tune=False,
+            single_precision=single, check_neutrality=False)
+    p.activate(pos, q, box_l=[L] * 3)
+    f = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
+    p.add_long_range_forces(torch.tensor(pos, device="cuda"), torch.tensor(q, device="cuda"), f)
+    ref = OracleP3M([L] * 3, [mesh] * 3, cao, 1.0, 2., 1.2).forces(pos, q)
+    err = np.sqrt(np.sum((f.cpu().numpy() - ref) ** 2))
+    assert err <= (2e-5 if single else 1e-6) * max(np.sqrt(np.sum(ref ** 2)), 1e-2)
