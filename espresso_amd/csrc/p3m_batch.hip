@@ -65,7 +65,11 @@ constexpr int kChunkMax = 64; // most particles staged per brick pass (3 x chunk
 constexpr int kCountCopies = 8; // brick counter copies (one per XCD-sized share of the blocks;
                                 // k_scan reads a brick's copies as two 16-byte words)
 constexpr int kBrick = 8;    // first-stencil points per brick edge
-constexpr int kFill = 4096;  // mesh elements zeroed per block
+constexpr int kFill = 8192;  // mesh elements zeroed per block
+// systems of up to this many particles and bins are binned by one block of
+// kSmallBlock threads (bin_system): 13.8 us at 1000 particles against 23 for
+// the four launches otherwise, 35 against 26 at 10^4
+constexpr int kSmallSystem = 4096, kSmallBins = 4096, kSmallBlock = 1024;
 constexpr int kStamps = 8;   // stage start times of a solve
 constexpr int kWideBlock = 512;    // threads of a k_fft_yx_conv_wide block
 // kz columns of a selection up to which that kernel runs: 384 blocks, three
@@ -218,14 +222,23 @@ __global__ void k_influence(MT *G, int Mx, int My, int Mz, int Kz, double wx, do
 }
 
 // ---------------------------------------------------------------------------
-// particle binning (one block per 256 particles of a system)
+// particle binning: systems of up to kSmallSystem particles by one block each
+// (bin_system), larger ones by one block per 256 particles (k_bin, k_scan,
+// k_scatter)
 // ---------------------------------------------------------------------------
+/** Brick (or column bin) of a particle with first stencil point gi. */
+__device__ __forceinline__ int particle_bin(DevGeo const &g, int const gi[3]) {
+  return g.col ? ((gi[1] / g.col) * g.nb[2] + gi[2] / g.col) * g.M[0] + gi[0]
+               : ((gi[0] / kBrick) * g.nb[1] + gi[1] / kBrick) * g.nb[2] + gi[2] / kBrick;
+}
+
 __global__ __launch_bounds__(kBlock) void k_bin(SysDesc const *__restrict__ sys,
                                                 int const *__restrict__ sel,
                                                 int const *__restrict__ wt, int nsel,
                                                 int const *__restrict__ soff, ParticleArrays pa,
                                                 int *counts, int *p_brick, int *p_rank,
-                                                int *p_nmp, double *partials, int *err_flag) {
+                                                int *p_nmp, double *partials, int *err_flag,
+                                                int epoch) {
   __shared__ double red[8 * 16];
   Slot const L = locate<false>(wt, sel, nsel);
   SysDesc const &d = sys[L.s];
@@ -240,9 +253,8 @@ __global__ __launch_bounds__(kBlock) void k_bin(SysDesc const *__restrict__ sys,
       double const x[3] = {pa.pos[3 * i], pa.pos[3 * i + 1], pa.pos[3 * i + 2]};
       int nmp[3], gi[3];
       double dist[3];
-      if (!particle_coordinates_rt(d.g, d.cao, x, nmp, gi, dist)) atomicOr(err_flag, 1);
-      b = d.g.col ? ((gi[1] / d.g.col) * d.g.nb[2] + gi[2] / d.g.col) * d.g.M[0] + gi[0]
-                  : ((gi[0] / kBrick) * d.g.nb[1] + gi[1] / kBrick) * d.g.nb[2] + gi[2] / kBrick;
+      if (!particle_coordinates_rt(d.g, d.cao, x, nmp, gi, dist)) atomicExch(err_flag, epoch);
+      b = particle_bin(d.g, gi);
       // brick counters [brick][copy]: blocks take copy blockIdx.x % 8, which
       // spreads the returning atomics of one brick over eight addresses
       int const copy = static_cast<int>(blockIdx.x) & (kCountCopies - 1);
@@ -310,6 +322,7 @@ __global__ __launch_bounds__(1024) void k_scan(SysDesc const *__restrict__ sys,
   __shared__ int carry;
   __shared__ double red[16 * 8];
   int const slot = blockIdx.x;
+  if (wt_bin[slot] == wt_bin[slot + 1]) return; // binned by bin_system
   int const s = sel[slot];
   SysDesc const &d = sys[s];
   {
@@ -440,29 +453,174 @@ __global__ __launch_bounds__(kBlock) void k_scatter(SysDesc const *__restrict__ 
   sidx[slot] = static_cast<int>(li);
 }
 
-/** Start of a solve, one launch over the systems' mesh blocks: zero the
- *  charge mesh (unless it is kept), each block its share of the system's
- *  brick counters, and the first block the error flag. */
+/** Scratch of bin_system in LDS. */
+struct BinLds {
+  int count[kSmallBins]; // particles per bin, then the start of the bin
+  int key[kSmallSystem]; // bin << 14 | rank of every particle, -1 if uncharged
+  double red[8 * 16];
+  int wsum[16];
+};
+
+/** Sorts one system into its bins with one block: bins and ranks from LDS
+ *  counters, the scan of the counts, then the sorted arrays; and the system's
+ *  sums (n_q, sum q, sum q^2, dipole, sum |q|, max |q|) in a fixed order.  The
+ *  work of k_bin, k_scan and k_scatter, which for a small system are three
+ *  launches of little else than latency.  Four particles per thread and turn,
+ *  their loads in flight together. */
+__device__ void bin_system(SysDesc const &d, int s, int64_t soff, ParticleArrays const &pa,
+                           int *p_nmp, int *offsets, double4 *spos, int *sidx, double *sums,
+                           int *err_flag, int epoch, BinLds &m) {
+  constexpr int U = 4;
+  int const n = d.n, nb = d.nbricks, tid = threadIdx.x;
+  for (int e = tid; e < nb; e += kSmallBlock) m.count[e] = 0;
+  __syncthreads();
+  double v[8] = {0., 0., 0., 0., 0., 0., 0., 0.}; // v[7]: max |q|
+  bool bad = false;
+  for (int l0 = tid; l0 < n; l0 += U * kSmallBlock) {
+    double4 r[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int64_t const i = d.part_off + min(l0 + u * kSmallBlock, n - 1);
+      r[u] = double4{pa.pos[3 * i], pa.pos[3 * i + 1], pa.pos[3 * i + 2], pa.q[i]};
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int const li = l0 + u * kSmallBlock;
+      int nmp[3] = {-1, -1, -1}, key = -1;
+      double const q = r[u].w;
+      if (li < n && q != 0.) {
+        int gi[3];
+        double dist[3];
+        double const x[3] = {r[u].x, r[u].y, r[u].z};
+        if (!particle_coordinates_rt(d.g, d.cao, x, nmp, gi, dist)) bad = true;
+        int const b = particle_bin(d.g, gi);
+        key = (b << 14) | atomicAdd(&m.count[b], 1);
+        double px = x[0], py = x[1], pz = x[2];
+        if (pa.upos) {
+          double const *up = pa.upos + 3 * (d.part_off + li);
+          px = up[0];
+          py = up[1];
+          pz = up[2];
+        }
+        v[0] += 1.;
+        v[1] += q;
+        v[2] += q * q;
+        v[3] += q * px;
+        v[4] += q * py;
+        v[5] += q * pz;
+        v[6] += fabs(q);
+        v[7] = fmax(v[7], fabs(q));
+      }
+      if (li < n) {
+        m.key[li] = key;
+        if (p_nmp) {
+          p_nmp[3 * li] = nmp[0];
+          p_nmp[3 * li + 1] = nmp[1];
+          p_nmp[3 * li + 2] = nmp[2];
+        }
+      }
+    }
+  }
+  if (bad) atomicExch(err_flag, epoch);
+  int const lane = tid & 63, wid = tid >> 6;
+#pragma unroll
+  for (int k = 0; k < 7; ++k) v[k] = wave_sum(v[k]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v[7] = fmax(v[7], __shfl_xor(v[7], off, 64));
+  if (lane == 0)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) m.red[k * 16 + wid] = v[k];
+  __syncthreads(); // counts, keys and wave sums complete
+  if (tid < 8) {
+    double t = 0.;
+    for (int w = 0; w < kSmallBlock / 64; ++w)
+      t = (tid == 7) ? fmax(t, m.red[tid * 16 + w]) : t + m.red[tid * 16 + w];
+    sums[s * 16 + tid] = t;
+  }
+  // exclusive scan of the counts, kSmallBins / kSmallBlock per thread
+  constexpr int PER = kSmallBins / kSmallBlock;
+  int c[PER], mine = 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    int const b = tid * PER + k;
+    c[k] = (b < nb) ? m.count[b] : 0;
+    mine += c[k];
+  }
+  int sc = mine;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    int const t = __shfl_up(sc, off, 64);
+    if (lane >= off) sc += t;
+  }
+  if (lane == 63) m.wsum[wid] = sc;
+  __syncthreads();
+  int o = sc - mine;
+  for (int w = 0; w < wid; ++w) o += m.wsum[w];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    int const b = tid * PER + k;
+    if (b < nb) {
+      m.count[b] = o;
+      offsets[d.off_off + b] = o;
+    }
+    o += c[k];
+  }
+  if (tid == kSmallBlock - 1) offsets[d.off_off + nb] = o;
+  __syncthreads();
+  for (int l0 = tid; l0 < n; l0 += U * kSmallBlock) {
+    double4 r[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int64_t const i = d.part_off + min(l0 + u * kSmallBlock, n - 1);
+      r[u] = double4{pa.pos[3 * i], pa.pos[3 * i + 1], pa.pos[3 * i + 2], pa.q[i]};
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int const li = l0 + u * kSmallBlock;
+      int const key = (li < n) ? m.key[li] : -1;
+      if (key < 0) continue;
+      int64_t const slot = soff + m.count[key >> 14] + (key & 0x3fff);
+      spos[slot] = r[u];
+      sidx[slot] = li;
+    }
+  }
+}
+
+/** Start of a solve, one launch: nsmall blocks bin the small systems, the
+ *  others zero the charge mesh (unless it is kept), each block its share of
+ *  the system's brick counters. */
 template <typename MT>
-__global__ __launch_bounds__(kBlock) void k_clear(SysDesc const *__restrict__ sys,
-                                                  int const *__restrict__ sel,
-                                                  int const *__restrict__ wt, int nsel,
-                                                  int *counts, int *err_flag, int zero_rho,
-                                                  unsigned long long *stamps) {
+__global__ __launch_bounds__(kSmallBlock) void k_begin(
+    SysDesc const *__restrict__ sys, int const *__restrict__ sel, int const *__restrict__ wt,
+    int nsel, int const *__restrict__ small, int nsmall, int const *__restrict__ soff,
+    ParticleArrays pa, int *p_nmp, int *offsets, double4 *spos, int *sidx, double *sums,
+    int *counts, int *err_flag, int epoch, int clear_err, int zero_rho,
+    unsigned long long *stamps) {
+  extern __shared__ double smem_d[];
   if (blockIdx.x == 0 && threadIdx.x < kStamps)
     stamps[threadIdx.x] = threadIdx.x ? 0ull : static_cast<unsigned long long>(wall_clock64());
-  Slot const L = locate(wt, sel, nsel);
-  SysDesc const &d = sys[L.s];
-  if (L.vb == 0 && threadIdx.x == 0) *err_flag = 0;
-  int const nblk = wt[L.slot + 1] - wt[L.slot];
-  int const nc = d.nbricks * kCountCopies;
+  if (static_cast<int>(blockIdx.x) < nsmall) {
+    int const s = small[blockIdx.x];
+    bin_system(sys[s], s, soff[s], pa, p_nmp, offsets, spos, sidx, sums, err_flag, epoch,
+               *reinterpret_cast<BinLds *>(smem_d));
+    return;
+  }
+  int const vb = static_cast<int>(blockIdx.x) - nsmall;
+  int const slot = find_slot(wt, nsel, vb);
+  int const lb = vb - wt[slot];
+  SysDesc const &d = sys[sel[slot]];
+  if (clear_err && vb == 0 && threadIdx.x == 0) *err_flag = 0;
+  int const nblk = wt[slot + 1] - wt[slot];
+  int const nc = (d.n > kSmallSystem || d.nbricks > kSmallBins || clear_err)
+                     ? d.nbricks * kCountCopies
+                     : 0;
   int const per = (nc + nblk - 1) / nblk;
   int *c = counts + d.brick_off * kCountCopies;
-  for (int e = L.lb * per + threadIdx.x; e < min(nc, (L.lb + 1) * per); e += blockDim.x) c[e] = 0;
+  for (int e = lb * per + threadIdx.x; e < min(nc, (lb + 1) * per); e += kSmallBlock) c[e] = 0;
   if (!zero_rho) return;
   int64_t const R = (int64_t)d.g.M[0] * d.g.M[1] * d.g.M[2];
   MT *rho = static_cast<MT *>(d.rho);
-  int64_t const beg = (int64_t)L.lb * kFill;
+  int64_t const beg = (int64_t)lb * kFill;
   int64_t const end = min(beg + kFill, R);
   // 16-byte stores over the block's whole words, element stores for the
   // rest (and for a mesh that is not 16-byte aligned)
@@ -470,8 +628,8 @@ __global__ __launch_bounds__(kBlock) void k_clear(SysDesc const *__restrict__ sy
   int64_t const words =
       (reinterpret_cast<uintptr_t>(rho + beg) & 15) ? 0 : (end - beg) / kPerWord;
   int4 *w = reinterpret_cast<int4 *>(rho + beg);
-  for (int64_t e = threadIdx.x; e < words; e += blockDim.x) w[e] = int4{0, 0, 0, 0};
-  for (int64_t e = beg + words * kPerWord + threadIdx.x; e < end; e += blockDim.x) rho[e] = MT(0);
+  for (int64_t e = threadIdx.x; e < words; e += kSmallBlock) w[e] = int4{0, 0, 0, 0};
+  for (int64_t e = beg + words * kPerWord + threadIdx.x; e < end; e += kSmallBlock) rho[e] = MT(0);
 }
 
 // ---------------------------------------------------------------------------
@@ -2246,6 +2404,10 @@ struct Plan {
   int *dbuf = nullptr; // device copy of all tables below (owned by the lane)
   int *d_sel = nullptr, *wt_bin = nullptr, *wt_fill = nullptr, *wt_z = nullptr, *wt_zc = nullptr,
       *wt_y = nullptr, *wt_x = nullptr, *wt_yi = nullptr, *wt_f = nullptr, *ycol = nullptr;
+  int *wt_part = nullptr; // particle blocks of every system
+  int blocks_part = 0;
+  int *d_small = nullptr; // systems binned by bin_system
+  int nsmall = 0;
   bool wide = false; // fused pass with a block per column and component
   int blocks_bin = 0, blocks_fill = 0, blocks_z = 0, blocks_zc = 0, blocks_y = 0, blocks_x = 0,
       blocks_yi = 0, blocks_f = 0;
@@ -2291,7 +2453,8 @@ struct Lane {
   int bin_cap = 0, conv_cap = 0;
   double *sums = nullptr;
   int sums_cap = 0;
-  int *err_flag = nullptr;
+  int *err_flag = nullptr; // epoch of the last solve that met a non-finite position
+  int epoch = 0;           // solves enqueued on the lane
   unsigned long long *stamps = nullptr; // kStamps stage start times, after err_flag
   double *h_sums = nullptr; // 16 per system, then the error flag and the stage times
   unsigned long long *seeds = nullptr, *h_seeds = nullptr;
@@ -2342,6 +2505,8 @@ void create_lane(Lane &ln) {
   hip_check(hipStreamCreateWithFlags(&ln.stream, hipStreamNonBlocking), "hipStreamCreate");
   for (auto &e : ln.ev) hip_check(hipEventCreate(&e), "hipEventCreate");
   hip_check(hipMalloc(&ln.err_flag, kStatusBytes), "hipMalloc err");
+  hip_check(hipMemset(ln.err_flag, 0, kStatusBytes), "clear err"); // once, not in a solve
+  hip_check(hipStreamSynchronize(nullptr), "clear err");
   ln.stamps = status_stamps(ln.err_flag);
 }
 
@@ -2668,6 +2833,7 @@ template <typename MT> void append_twiddles(BatchSolver::Impl *m, int n, hipStre
 }
 
 template <typename MT> void set_kernel_attrs() {
+  allow_lds(k_begin<MT>);
   allow_lds(k_fft_z_r2c<MT>);
   allow_lds(k_fft_z_c2r<MT, 1>);
   allow_lds(k_fft_z_c2r<MT, 3>);
@@ -3056,9 +3222,21 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
     return std::make_pair(start, acc);
   };
   host.insert(host.end(), sel.begin(), sel.end());
-  auto const bin = push_prefix([](HostSys const &h) {
+  // small systems are binned by one block each; not on the fixed lane, whose
+  // error flag is cleared by the launch that would bin them
+  auto const small = [&ln](HostSys const &h) {
+    return !ln.fixed && h.n <= kSmallSystem && h.nbricks <= kSmallBins;
+  };
+  auto const bin = push_prefix([&small](HostSys const &h) {
+    return small(h) ? 0 : static_cast<int>(std::max<int64_t>((h.n + kBlock - 1) / kBlock, 1));
+  });
+  auto const part = push_prefix([](HostSys const &h) {
     return static_cast<int>((h.n + kBlock - 1) / kBlock);
   });
+  int const small_start = static_cast<int>(host.size());
+  for (int s : sel)
+    if (small(m->sys[s])) host.push_back(s);
+  p.nsmall = static_cast<int>(host.size()) - small_start;
   auto const fill = push_prefix([](HostSys const &h) {
     int64_t const R = (int64_t)h.desc.g.M[0] * h.desc.g.M[1] * h.desc.g.M[2];
     return static_cast<int>((R + kFill - 1) / kFill);
@@ -3167,6 +3345,9 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
               "copy plan");
   }
   p.d_sel = p.dbuf;
+  p.wt_part = p.dbuf + part.first;
+  p.blocks_part = part.second;
+  p.d_small = p.dbuf + small_start;
   p.wt_bin = p.dbuf + bin.first;
   p.blocks_bin = bin.second;
   p.wt_fill = p.dbuf + fill.first;
@@ -3236,19 +3417,22 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
   if (ev) (void)hipEventRecord(ev[0], st);
   bool const no_spread = (flags & kSolveNoSpread) != 0;
   bool const zero_rho = !(flags & kSolveAccumulate) && !no_spread;
-  k_clear<MT><<<p.blocks_fill, kBlock, 0, st>>>(sys, p.d_sel, p.wt_fill, ns, ln.counts,
-                                                ln.err_flag, zero_rho ? 1 : 0, ln.stamps);
+  ln.epoch = ln.epoch % std::numeric_limits<int>::max() + 1;
+  int const epoch = ln.epoch; // of the error flag
+  k_begin<MT><<<p.nsmall + p.blocks_fill, kSmallBlock, p.nsmall ? sizeof(BinLds) : 0, st>>>(
+      sys, p.d_sel, p.wt_fill, ns, p.d_small, p.nsmall, p.soff, pa, p_nmp, ln.offsets, ln.spos,
+      ln.sidx, ln.sums, ln.counts, ln.err_flag, epoch, ln.fixed ? 1 : 0, zero_rho ? 1 : 0,
+      ln.stamps);
   if (p.blocks_bin > 0) {
     k_bin<<<p.blocks_bin, kBlock, 0, st>>>(sys, p.d_sel, p.wt_bin, ns, p.soff, pa, ln.counts,
                                             ln.p_brick, ln.p_rank, p_nmp, ln.bin_part,
-                                            ln.err_flag);
-  }
-  k_scan<<<ns, 1024, 0, st>>>(sys, p.d_sel, p.wt_bin, ln.bin_part, ln.sums, ln.counts,
-                              ln.offsets);
-  if (p.blocks_bin > 0)
+                                            ln.err_flag, epoch);
+    k_scan<<<ns, 1024, 0, st>>>(sys, p.d_sel, p.wt_bin, ln.bin_part, ln.sums, ln.counts,
+                                ln.offsets);
     k_scatter<<<p.blocks_bin, kBlock, 0, st>>>(sys, p.d_sel, p.wt_bin, ns, p.soff, pa,
                                                 ln.p_brick, ln.p_rank, ln.counts, ln.spos,
                                                 ln.sidx);
+  }
   if (ev) (void)hipEventRecord(ev[1], st);
   bool const det = (flags & kSolveDeterministic) && !no_spread && !stop_after_spread &&
                    !(flags & (kSolveAccumulate | kSolveMeshOnly));
@@ -3411,20 +3595,21 @@ __global__ void k_finalize_device(double const *__restrict__ h, double volume, d
   }
 }
 
-/** End of a synchronous solve: the sums of the selected systems, the error
- *  flag and the stage times written to pinned host memory (layout of
- *  Lane::h_sums), instead of one copy each. */
+/** End of a synchronous solve: the sums of the selected systems (when energy
+ *  or virial are wanted), the error flag and the stage times written to
+ *  pinned host memory (layout of Lane::h_sums), instead of one copy each.
+ *  Latency of the host writes: 13 us with the sums of 256 systems. */
 __global__ void k_results(int const *__restrict__ sel, int nsel, double const *__restrict__ sums,
-                          int const *__restrict__ err_flag,
+                          int const *__restrict__ err_flag, int epoch, int want_sums,
                           unsigned long long const *__restrict__ stamps, int nsys,
                           double *__restrict__ host) {
   unsigned long long const now = wall_clock64();
-  for (int e = threadIdx.x; e < 16 * nsel; e += blockDim.x) {
+  for (int e = threadIdx.x; want_sums && e < 16 * nsel; e += blockDim.x) {
     int const at = 16 * sel[e >> 4] + (e & 15);
     host[at] = sums[at];
   }
   double *const tail = host + 16 * nsys;
-  if (threadIdx.x == 0) *reinterpret_cast<int *>(tail) = *err_flag;
+  if (threadIdx.x == 0) *reinterpret_cast<int *>(tail) = *err_flag == epoch;
   if (threadIdx.x < kStamps)
     reinterpret_cast<unsigned long long *>(tail + 1)[threadIdx.x] =
         (threadIdx.x == 6) ? now : stamps[threadIdx.x];
@@ -3503,8 +3688,10 @@ void BatchSolver::solve_on(int lane, std::vector<int> const &sel, ParticleArrays
     enqueue<float>(m, ln, pa, flags, m_shape, ev, nullptr, false);
   hip_check(hipGetLastError(), "P3M solve launch");
   if (!sync) return;
+  bool const want_sums = (flags & 6u) != 0; // energy or virial
   k_results<<<1, 256, 0, ln.stream>>>(ln.plan.d_sel, ln.plan.nsel, ln.sums, ln.err_flag,
-                                      ln.stamps, num_systems(), ln.h_sums);
+                                      ln.epoch, want_sums ? 1 : 0, ln.stamps, num_systems(),
+                                      ln.h_sums);
   hip_check(hipGetLastError(), "P3M results");
   hip_check(hipStreamSynchronize(ln.stream), "P3M solve");
   double const *const tail = ln.h_sums + 16 * num_systems();
@@ -3514,7 +3701,11 @@ void BatchSolver::solve_on(int lane, std::vector<int> const &sel, ParticleArrays
   unsigned long long stamps[kStamps];
   std::memcpy(stamps, tail + 1, sizeof(stamps));
   stage_times(stamps, m_clock_khz, last_ms);
-  if (out) finalize_results(m, ln, sel, out);
+  if (!out) return;
+  if (want_sums)
+    finalize_results(m, ln, sel, out);
+  else
+    out->assign(sel.size(), SolveResult{});
 }
 
 namespace {
@@ -3632,9 +3823,9 @@ void BatchSolver::prepare_on(int lane, std::vector<int> const &sel, double *pos,
                            hipMemcpyHostToDevice, ln.stream),
             "copy seeds");
   Plan const &p = ln.plan;
-  if (p.blocks_bin > 0)
-    k_prepare<<<p.blocks_bin, kBlock, 0, ln.stream>>>(m->d_sys, p.d_sel, p.wt_bin, p.nsel, pos,
-                                                       force, sigma, ln.seeds);
+  if (p.blocks_part > 0)
+    k_prepare<<<p.blocks_part, kBlock, 0, ln.stream>>>(m->d_sys, p.d_sel, p.wt_part, p.nsel, pos,
+                                                        force, sigma, ln.seeds);
   hip_check(hipGetLastError(), "P3M prepare launch");
 }
 

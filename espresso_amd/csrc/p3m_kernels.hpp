@@ -181,6 +181,20 @@ __device__ __forceinline__ int wrap_once(int v, int M) {
   return v;
 }
 
+/** v mod M in [0, M): one conditional addition or subtraction, a remainder only
+ *  for the rare values further away. */
+__device__ __forceinline__ int periodic_index(int v, int M) {
+  if (v < 0)
+    v += M;
+  else if (v >= M)
+    v -= M;
+  if (static_cast<unsigned>(v) >= static_cast<unsigned>(M)) {
+    v %= M;
+    if (v < 0) v += M;
+  }
+  return v;
+}
+
 // ---------------------------------------------------------------------------
 // DPP lane exchanges on FP64 values (two 32-bit moves per value).
 // ---------------------------------------------------------------------------
@@ -274,10 +288,7 @@ __device__ __forceinline__ bool particle_coordinates_rt(DevGeo const &g, int P, 
     int const n = static_cast<int>(t);
     nmp[d] = n;
     dist[d] = ca_distance(t, n);
-    int gg = n - g.marg[d];
-    gg %= g.M[d];
-    if (gg < 0) gg += g.M[d];
-    gi[d] = gg;
+    gi[d] = periodic_index(n - g.marg[d], g.M[d]);
   }
   return ok;
 }
@@ -300,10 +311,7 @@ __device__ __forceinline__ bool coordinate_1d(DevGeo const &g, int P, double x, 
   int const n = static_cast<int>(t);
   nmp = n;
   dist = ca_distance(t, n);
-  int gg = n - g.marg[d];
-  gg %= g.M[d];
-  if (gg < 0) gg += g.M[d];
-  gi = gg;
+  gi = periodic_index(n - g.marg[d], g.M[d]);
   return ok;
 }
 

@@ -323,3 +323,42 @@ def test_shared_bricks_match_oracle(n, mesh, cao, single):
     ref = OracleP3M([L] * 3, [mesh] * 3, cao, 1.0, 2., 1.2).forces(pos, q)
     err = np.sqrt(np.sum((f.cpu().numpy() - ref) ** 2))
     assert err <= (2e-5 if single else 1e-6) * max(np.sqrt(np.sum(ref ** 2)), 1e-2)
+
+
+@pytest.mark.parametrize("single", [False, True])
+@pytest.mark.parametrize("systems", [
+    ((1, 16, 3), (0, 24, 4), (63, 136, 5)),
+    ((4095, 16, 7), (4096, 32, 2)),
+    ((4097, 24, 5), (3, 8, 3), (1025, 40, 6)),
+])
+def test_small_systems_binned_by_one_block_match_oracle(systems, single):
+    """Systems (n, mesh, cao) of up to 4096 particles are binned by one block,
+    larger ones (and meshes of more than 4096 bricks) by several launches,
+    both in one selection; uncharged particles, positions outside the box, and
+    a solve with a position that is not finite, which raises and leaves the
+    next one clean.  Tolerances of the parity tests (FP64 1e-6, FP32 mesh 2e-5
+    rel-rms)."""
+    import torch
+    from espresso_amd.batch import P3MBatch
+    from oracle.oracle import OracleP3M
+    rng = np.random.default_rng(sum(s[0] for s in systems))
+    L, b, pos, q, ref = 9., P3MBatch(single_precision=single), [], [], []
+    for n, mesh, cao in systems:
+        b.add_system([L] * 3, n, 1.2, mesh, cao, 1.0, 2.)
+        pos.append(rng.uniform(-L, 2. * L, (n, 3)))
+        q.append(rng.choice([-1., 1., 0.], n))
+        q[-1][:1] = 1.
+        ref.append(np.zeros((0, 3)) if n == 0 else
+                   OracleP3M([L] * 3, [mesh] * 3, cao, 1.0, 2., 1.2).forces(pos[-1] % L, q[-1]))
+    tp = torch.tensor(np.concatenate(pos), device="cuda")
+    tq = torch.tensor(np.concatenate(q), device="cuda")
+    bad = tp.clone()
+    bad[0, 1] = float("nan")
+    f = torch.zeros_like(tp)
+    with pytest.raises(RuntimeError, match="non-finite"):
+        b.solve(bad, tq, f)
+    f.zero_()
+    b.solve(tp, tq, f)
+    ref = np.concatenate(ref)
+    err = np.sqrt(np.sum((f.cpu().numpy() - ref) ** 2))
+    assert err <= (2e-5 if single else 1e-6) * max(np.sqrt(np.sum(ref ** 2)), 1e-2)
