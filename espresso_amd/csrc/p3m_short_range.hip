@@ -349,9 +349,114 @@ __global__ __launch_bounds__(NT) void k_sr_cells(CellGrid g, int const *__restri
   }
 }
 
-/** Pair terms over columns (no ELC images).  The cells are columns of edge
- *  >= r_cut / rx (x) and r_cut / ry (y), cut into z bins of edge >= r_cut /
- *  rz, z fastest, so that the candidates of a column within reach of a home
+/** All charged pairs with the minimum-image displacement (boxes narrower
+ *  than three cells of edge r_cut); one block per NT sorted particles. */
+template <int NT, bool EV>
+__global__ __launch_bounds__(NT) void k_sr_allpairs(int nq, CellGrid g,
+                                                    double4 const *__restrict__ spos,
+                                                    int const *__restrict__ sidx,
+                                                    double prefactor, double alpha, double rc2,
+                                                    double *__restrict__ force,
+                                                    double *partials, SrImages im) {
+  __shared__ double4 tile[NT];
+  __shared__ double red[8 * 16];
+  int const i = blockIdx.x * NT + static_cast<int>(threadIdx.x);
+  bool const has = i < nq;
+  double4 const pi = has ? spos[i] : double4{0., 0., 0., 0.};
+  double const qpi = prefactor * pi.w;
+  double const two_a = 2. * alpha * std::numbers::inv_sqrtpi;
+  double fx = 0., fy = 0., fz = 0.;
+  double ev[7] = {0., 0., 0., 0., 0., 0., 0.};
+  for (int tb = 0; tb < nq; tb += NT) {
+    __syncthreads();
+    int const j = tb + static_cast<int>(threadIdx.x);
+    if (j < nq) tile[threadIdx.x] = spos[j];
+    __syncthreads();
+    if (has)
+      tile_pairs<true, EV>(tile, min(NT, nq - tb), pi, qpi, g, rc2, alpha, two_a, fx, fy, fz,
+                           ev, im, 0.);
+  }
+  if (has) {
+    double *f = force + 3 * static_cast<int64_t>(sidx[i]);
+    f[0] += fx;
+    f[1] += fy;
+    f[2] += fz;
+  }
+  if constexpr (EV) {
+    block_sum<7>(ev, red);
+    if (threadIdx.x == 0)
+      for (int k = 0; k < 7; ++k) partials[blockIdx.x * 8 + k] = ev[k];
+  }
+}
+
+/** |mu|^2 of every particle (the dipolar binning key: zero dipoles take no
+ *  part, dp3m.hpp:162); the cell counters are cleared on the way. */
+__global__ __launch_bounds__(256) void k_sr_mu2(int64_t n, double const *__restrict__ dip,
+                                                double *__restrict__ mu2,
+                                                int *__restrict__ counts, int ncells) {
+  int64_t const i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  for (int64_t c = i; c < ncells; c += (int64_t)gridDim.x * blockDim.x) counts[c] = 0;
+  if (i >= n) return;
+  double const a = dip[3 * i], b = dip[3 * i + 1], c = dip[3 * i + 2];
+  mu2[i] = a * a + b * b + c * c;
+}
+
+/** Dipoles in cell order. */
+__global__ __launch_bounds__(256) void k_sr_sort_dip(int64_t n, int const *__restrict__ total,
+                                                     int const *__restrict__ sidx,
+                                                     double const *__restrict__ dip,
+                                                     double4 *__restrict__ sdip) {
+  int64_t const s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (s >= n || s >= *total) return;
+  int64_t const i = sidx[s];
+  sdip[s] = double4{dip[3 * i], dip[3 * i + 1], dip[3 * i + 2], 0.};
+}
+
+/** Dipolar pair term (DipolarP3M::pair_force / pair_energy,
+ *  dp3m.hpp:160-235) of dipole mi with partner mj at d = r_i - r_j, r2 =
+ *  |d|^2, without the prefactor and with mi taken out of the sums over
+ *  partners: the force is v[0..2] + mi v[6], the torque mi x v[3..5]; pair
+ *  energy e with EV.  EXACT takes the library's erfc, else the rational
+ *  approximation of Abramowitz and Stegun 7.1.26. */
+template <bool EV, bool EXACT>
+__device__ __forceinline__ void dip_pair(double dx, double dy, double dz, double r2,
+                                         double4 const &mi, double4 const &mj, double alpha,
+                                         double two_a, double (&v)[7], double &e) {
+  double const rinv = nr_rsq(r2);
+  double const ad = alpha * (r2 * rinv);
+  double const ex = exp(-ad * ad);
+  double const r2i = rinv * rinv;
+  double B;
+  if constexpr (EXACT) {
+    B = (erfc(ad) * rinv + two_a * ex) * r2i;
+  } else {
+    double const tt = nr_rcp(fma(0.3275911, ad, 1.));
+    double const ep =
+        tt * (0.254829592 +
+              tt * (-0.284496736 + tt * (1.421413741 + tt * (-1.453152027 + tt * 1.061405429))));
+    B = (ep * rinv + two_a) * ex * r2i;
+  }
+  double const alpsq = alpha * alpha;
+  double const common = alpsq * two_a * ex;
+  double const Cr = r2i * (3. * B + 2. * common);
+  double const Dr = r2i * (5. * Cr + 4. * common * alpsq);
+  double const mimj = mi.x * mj.x + mi.y * mj.y + mi.z * mj.z;
+  double const mir = mi.x * dx + mi.y * dy + mi.z * dz;
+  double const mjr = mj.x * dx + mj.y * dy + mj.z * dz;
+  double const cd = mimj * Cr - mir * mjr * Dr, cj = mir * Cr, c1 = mjr * Cr;
+  v[0] += cd * dx + cj * mj.x;
+  v[1] += cd * dy + cj * mj.y;
+  v[2] += cd * dz + cj * mj.z;
+  v[3] += c1 * dx - B * mj.x;
+  v[4] += c1 * dy - B * mj.y;
+  v[5] += c1 * dz - B * mj.z;
+  v[6] += c1;
+  if constexpr (EV) e += mimj * B - mir * c1;
+}
+
+/** Pair terms over columns: Coulomb without ELC images, or dipolar (DIP, sdip
+ *  the sorted dipoles).  The cells are columns of edge >= r_cut / rx (x) and
+ *  r_cut / ry (y), cut into z bins of edge >= r_cut / rz, z fastest, so that the candidates of a column within reach of a home
  *  group are one contiguous run of the sorted particles (split at the
  *  periodic boundary).  One block of W waves per home group of 64 sorted
  *  particles of one column: lane = home particle, position and force in
@@ -367,23 +472,29 @@ __global__ __launch_bounds__(NT) void k_sr_cells(CellGrid g, int const *__restri
  *  list is emptied each time and the columns are swept once, in order).
  *  Measured (250,000 charges, 311 partners each): 0.60 ms, 73 % VALU issue,
  *  against 2.94 ms with lanes over the home particles of one r_cut/2 cell,
- *  which kept 10 of 64 lanes busy; 1000 charges: 41 against 89 us. */
-template <bool EV>
-__global__ __launch_bounds__(kColWaves * 64, EV ? 4 : 5) void k_sr_columns(
+ *  which kept 10 of 64 lanes busy; 1000 charges: 32 against 89 us.  50,000
+ *  dipoles, 66 partners each: 84 us, against 144 with lanes over the home
+ *  particles of one r_cut cell and a queue of hits per block; 200,000 dipoles
+ *  with 105, 420 and 4300 partners (calls): 0.39, 0.91 and 6.9 ms against 0.71,
+ *  1.9 and 20. */
+template <bool DIP, bool EV, bool EXACT>
+__global__ __launch_bounds__(kColWaves * 64, DIP ? 3 : EV ? 4 : 5) void k_sr_columns(
     CellGrid g, int rx, int ry, int rz, int split, int sweeps, int const *__restrict__ offsets,
     int const *__restrict__ goff, int2 const *__restrict__ grp,
-    double4 const *__restrict__ spos, int const *__restrict__ sidx, double prefactor,
-    double alpha, double rc2, double *__restrict__ force, double *__restrict__ shares,
+    double4 const *__restrict__ spos, double4 const *__restrict__ sdip,
+    int const *__restrict__ sidx, double prefactor, double alpha, double rc2,
+    double *__restrict__ force, double *__restrict__ torque, double *__restrict__ shares,
     int *__restrict__ arrived, double *__restrict__ partials) {
   constexpr int W = kColWaves, U = 4, CAP = 24; // waves, candidates per batch, list length
-  static_assert(CAP >= 2 * U && CAP * 64 * sizeof(int) >= 3 * 64 * sizeof(double));
+  constexpr int NV = DIP ? 6 : 3, NE = DIP ? 1 : 7; // force (and torque); reduced terms
+  static_assert(CAP >= 2 * U && CAP * 64 * sizeof(int) >= NV * 64 * sizeof(double));
   __shared__ __align__(16) int list[W][CAP * 64];
   __shared__ double red[8 * 16];
   __shared__ int last;
   int const ngroups = goff[g.nc[0] * g.nc[1]];
   int const b = blockIdx.x, nblocks = ngroups * split;
   if (b >= nblocks) {
-    if (EV && threadIdx.x < 7) partials[static_cast<int64_t>(b) * 8 + threadIdx.x] = 0.;
+    if (EV && threadIdx.x < NE) partials[static_cast<int64_t>(b) * 8 + threadIdx.x] = 0.;
     return;
   }
   // contiguous groups per XCD (their candidates overlap)
@@ -401,6 +512,8 @@ __global__ __launch_bounds__(kColWaves * 64, EV ? 4 : 5) void k_sr_columns(
   bool const home = lane < nh;
   double4 hp = spos[h0 + min(lane, nh - 1)];
   double const qpi = prefactor * hp.w;
+  double4 hm{0., 0., 0., 0.};
+  if constexpr (DIP) hm = sdip[h0 + min(lane, nh - 1)];
   // z bins of the group (sorted by bin): first and last particle
   auto zbin = [&](double z) { return min(nz - 1, static_cast<int>(z * g.inv_cell[2])); };
   int const b0 = zbin(readlane_f64(hp.z, 0)), b1 = zbin(readlane_f64(hp.z, nh - 1));
@@ -408,8 +521,8 @@ __global__ __launch_bounds__(kColWaves * 64, EV ? 4 : 5) void k_sr_columns(
   bool const wrap = cx < rx || cx + rx >= g.nc[0] || cy < ry || cy + ry >= g.nc[1] ||
                     b0 < rz || b1 + rz >= nz;
   double const two_a = 2. * alpha * std::numbers::inv_sqrtpi;
-  double fx = 0., fy = 0., fz = 0.;
-  double ev[7] = {0., 0., 0., 0., 0., 0., 0.};
+  double f[DIP ? 7 : 3] = {}; // sums of pair_term or dip_pair
+  double ev[NE] = {};
   // byte offsets into `list` of the lane's first slot, of the slot the next
   // hit goes to, and of the last one a batch may start at
   char *const lists = reinterpret_cast<char *>(list);
@@ -423,14 +536,20 @@ __global__ __launch_bounds__(kColWaves * 64, EV ? 4 : 5) void k_sr_columns(
   auto listed = [&](int s) { return *reinterpret_cast<int const *>(lists + s); };
   auto drain = [&](bool rest) {
     int s = slot0;
-    double4 next = spos[(s < slot) ? listed(s) : h0];
+    int j = (s < slot) ? listed(s) : h0;
+    double4 next = spos[j], next_dip{0., 0., 0., 0.};
+    if constexpr (DIP) next_dip = sdip[j];
     for (int round = 0;; ++round) {
       uint64_t const busy = __ballot(s < slot);
       if (!busy || (!rest && round >= U && __popcll(busy) < 40)) break;
-      double4 const pj = next;
+      double4 const pj = next, mj = next_dip;
       bool const on = s < slot;
       s += 256;
-      if (s < slot) next = spos[listed(s)]; // in flight during this round
+      if (s < slot) { // in flight during this round
+        j = listed(s);
+        next = spos[j];
+        if constexpr (DIP) next_dip = sdip[j];
+      }
       if (on) {
         double dx = hp.x - pj.x, dy = hp.y - pj.y, dz = hp.z - pj.z;
         if (wrap) {
@@ -439,8 +558,13 @@ __global__ __launch_bounds__(kColWaves * 64, EV ? 4 : 5) void k_sr_columns(
           dz -= g.L[2] * rint(dz * iLz);
         }
         double const r2 = dx * dx + dy * dy + dz * dz;
-        if (r2 > 0.)
-          pair_term<EV>(dx, dy, dz, r2, qpi * pj.w, alpha, two_a, fx, fy, fz, ev);
+        if (r2 > 0.) {
+          if constexpr (DIP) {
+            dip_pair<EV, EXACT>(dx, dy, dz, r2, hm, mj, alpha, two_a, f, ev[0]);
+          } else {
+            pair_term<EV>(dx, dy, dz, r2, qpi * pj.w, alpha, two_a, f[0], f[1], f[2], ev);
+          }
+        }
       }
     }
     int d = slot0;
@@ -502,453 +626,128 @@ __global__ __launch_bounds__(kColWaves * 64, EV ? 4 : 5) void k_sr_columns(
     }
   }
   drain(true);
-  // the waves' forces, in wave order
+  if constexpr (DIP) {
+    double const h[3] = {f[3], f[4], f[5]};
+    f[0] = prefactor * (f[0] + hm.x * f[6]);
+    f[1] = prefactor * (f[1] + hm.y * f[6]);
+    f[2] = prefactor * (f[2] + hm.z * f[6]);
+    f[3] = prefactor * (hm.y * h[2] - hm.z * h[1]);
+    f[4] = prefactor * (hm.z * h[0] - hm.x * h[2]);
+    f[5] = prefactor * (hm.x * h[1] - hm.y * h[0]);
+    ev[0] *= prefactor;
+  }
+  // the waves' sums, in wave order
   double *const own = reinterpret_cast<double *>(list[wave]);
-  own[lane] = fx;
-  own[64 + lane] = fy;
-  own[128 + lane] = fz;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) own[64 * k + lane] = f[k];
   __syncthreads();
   if (wave == 0) {
 #pragma unroll
     for (int v = 1; v < W; ++v) {
       double const *o = reinterpret_cast<double const *>(list[v]);
-      fx += o[lane];
-      fy += o[64 + lane];
-      fz += o[128 + lane];
+#pragma unroll
+      for (int k = 0; k < NV; ++k) f[k] += o[64 * k + lane];
     }
   }
   bool add = wave == 0 && home;
   if (split > 1) {
     // the group's last block adds all shares, in share order
-    double *const mine = shares + static_cast<int64_t>(gi) * split * 192;
+    double *const mine = shares + static_cast<int64_t>(gi) * split * (64 * NV);
     if (wave == 0) {
-      double *const o = mine + share * 192;
-      __hip_atomic_store(o + lane, fx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(o + 64 + lane, fy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(o + 128 + lane, fz, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __threadfence();
+      double *const o = mine + share * (64 * NV);
+#pragma unroll
+      for (int k = 0; k < NV; ++k)
+        __hip_atomic_store(o + 64 * k + lane, f[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // the shares are written and read past the caches of the XCDs (agent
+      // scope), so the count only has to wait for the stores to complete
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       if (lane == 0)
-        last = __hip_atomic_fetch_add(arrived + gi, 1, __ATOMIC_ACQ_REL,
+        last = __hip_atomic_fetch_add(arrived + gi, 1, __ATOMIC_RELAXED,
                                       __HIP_MEMORY_SCOPE_AGENT) == split - 1;
     }
     __syncthreads();
     add = add && last;
     if (add) {
-      fx = fy = fz = 0.;
+#pragma unroll
+      for (int k = 0; k < NV; ++k) f[k] = 0.;
       for (int v = 0; v < split; ++v) {
-        double *const o = mine + v * 192;
-        fx += __hip_atomic_load(o + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        fy += __hip_atomic_load(o + 64 + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        fz += __hip_atomic_load(o + 128 + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        double *const o = mine + v * (64 * NV);
+#pragma unroll
+        for (int k = 0; k < NV; ++k)
+          f[k] += __hip_atomic_load(o + 64 * k + lane, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
       }
     }
   }
   if (add) {
-    double *f = force + 3 * static_cast<int64_t>(sidx[h0 + lane]);
-    f[0] += fx;
-    f[1] += fy;
-    f[2] += fz;
-  }
-  if constexpr (EV) {
-    block_sum<7>(ev, red);
-    if (threadIdx.x == 0)
-      for (int k = 0; k < 7; ++k) partials[static_cast<int64_t>(b) * 8 + k] = ev[k];
-  }
-}
-
-/** All charged pairs with the minimum-image displacement (boxes narrower
- *  than three cells of edge r_cut); one block per NT sorted particles. */
-template <int NT, bool EV>
-__global__ __launch_bounds__(NT) void k_sr_allpairs(int nq, CellGrid g,
-                                                    double4 const *__restrict__ spos,
-                                                    int const *__restrict__ sidx,
-                                                    double prefactor, double alpha, double rc2,
-                                                    double *__restrict__ force,
-                                                    double *partials, SrImages im) {
-  __shared__ double4 tile[NT];
-  __shared__ double red[8 * 16];
-  int const i = blockIdx.x * NT + static_cast<int>(threadIdx.x);
-  bool const has = i < nq;
-  double4 const pi = has ? spos[i] : double4{0., 0., 0., 0.};
-  double const qpi = prefactor * pi.w;
-  double const two_a = 2. * alpha * std::numbers::inv_sqrtpi;
-  double fx = 0., fy = 0., fz = 0.;
-  double ev[7] = {0., 0., 0., 0., 0., 0., 0.};
-  for (int tb = 0; tb < nq; tb += NT) {
-    __syncthreads();
-    int const j = tb + static_cast<int>(threadIdx.x);
-    if (j < nq) tile[threadIdx.x] = spos[j];
-    __syncthreads();
-    if (has)
-      tile_pairs<true, EV>(tile, min(NT, nq - tb), pi, qpi, g, rc2, alpha, two_a, fx, fy, fz,
-                           ev, im, 0.);
-  }
-  if (has) {
-    double *f = force + 3 * static_cast<int64_t>(sidx[i]);
-    f[0] += fx;
-    f[1] += fy;
-    f[2] += fz;
-  }
-  if constexpr (EV) {
-    block_sum<7>(ev, red);
-    if (threadIdx.x == 0)
-      for (int k = 0; k < 7; ++k) partials[blockIdx.x * 8 + k] = ev[k];
-  }
-}
-
-/** |mu|^2 of every particle (the dipolar binning key: zero dipoles take no
- *  part, dp3m.hpp:162). */
-__global__ __launch_bounds__(256) void k_sr_mu2(int64_t n, double const *__restrict__ dip,
-                                                double *__restrict__ mu2) {
-  int64_t const i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double const a = dip[3 * i], b = dip[3 * i + 1], c = dip[3 * i + 2];
-  mu2[i] = a * a + b * b + c * c;
-}
-
-/** Dipoles in cell order. */
-__global__ __launch_bounds__(256) void k_sr_sort_dip(int64_t n, int const *__restrict__ total,
-                                                     int const *__restrict__ sidx,
-                                                     double const *__restrict__ dip,
-                                                     double4 *__restrict__ sdip) {
-  int64_t const s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (s >= n || s >= *total) return;
-  int64_t const i = sidx[s];
-  sdip[s] = double4{dip[3 * i], dip[3 * i + 1], dip[3 * i + 2], 0.};
-}
-
-/** Dipolar pair term (DipolarP3M::pair_force / pair_energy,
- *  dp3m.hpp:160-235) of particle i with partner j at d = r_i - r_j, r2 =
- *  |d|^2 within the cutoff: force and torque on i, pair energy with EV. */
-template <bool EV>
-__device__ __forceinline__ void dip_pair(double dx, double dy, double dz, double r2,
-                                         double4 const &mi, double4 const &mj, double prefactor,
-                                         double alpha, int exact, double (&f)[3],
-                                         double (&t)[3], double &e) {
-  double const r = sqrt(r2);
-  double const ad = alpha * r;
-  double const ex = exp(-ad * ad);
-  double const r2i = 1. / r2;
-  double const coeff = 2. * alpha * std::numbers::inv_sqrtpi;
-  double B;
-  if (exact) {
-    B = (erfc(ad) / r + coeff * ex) * r2i;
-  } else {
-    double const tt = 1. / (1. + 0.3275911 * ad);
-    double const ep =
-        tt * (0.254829592 +
-              tt * (-0.284496736 + tt * (1.421413741 + tt * (-1.453152027 + tt * 1.061405429))));
-    B = (ep / r + coeff) * ex * r2i;
-  }
-  double const alpsq = alpha * alpha;
-  double const common = alpsq * coeff * ex;
-  double const Cr = r2i * (3. * B + 2. * common);
-  double const Dr = r2i * (5. * Cr + 4. * common * alpsq);
-  double const mimj = mi.x * mj.x + mi.y * mj.y + mi.z * mj.z;
-  double const mir = mi.x * dx + mi.y * dy + mi.z * dz;
-  double const mjr = mj.x * dx + mj.y * dy + mj.z * dz;
-  double const cd = mimj * Cr - mir * mjr * Dr;
-  f[0] += prefactor * (cd * dx + (mi.x * mjr + mj.x * mir) * Cr);
-  f[1] += prefactor * (cd * dy + (mi.y * mjr + mj.y * mir) * Cr);
-  f[2] += prefactor * (cd * dz + (mi.z * mjr + mj.z * mir) * Cr);
-  double const c1 = mjr * Cr;
-  t[0] += prefactor * (-(mi.y * mj.z - mi.z * mj.y) * B + (mi.y * dz - mi.z * dy) * c1);
-  t[1] += prefactor * (-(mi.z * mj.x - mi.x * mj.z) * B + (mi.z * dx - mi.x * dz) * c1);
-  t[2] += prefactor * (-(mi.x * mj.y - mi.y * mj.x) * B + (mi.x * dy - mi.y * dx) * c1);
-  if constexpr (EV) e += prefactor * (mimj * B - mir * mjr * Cr);
-}
-
-/** Dipolar pair terms over cells of edge r_cut/2 (NSUB = 2, dense systems),
- *  dense evaluation per block: one block of 256 threads per home cell.  The block enumerates the (home particle,
- *  candidate) pairs of the (2 NSUB + 1)^3 neighbour cells 256 at a time,
- *  appends the pairs inside r_cut to an LDS queue (wave ballots, one LDS
- *  atomic per wave) and drains the queue with every lane evaluating one
- *  pair, so the pair terms run without idle lanes however sparse the cells.
- *  Force and torque on each home particle accumulate in LDS (FP64 LDS
- *  atomics) and are added to the caller's arrays once. */
-template <int NSUB, bool EV>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_sr_dip_queue(CellGrid g, int const *__restrict__ offsets,
-                                                      double4 const *__restrict__ spos,
-                                                      double4 const *__restrict__ sdip,
-                                                      int const *__restrict__ sidx,
-                                                      double prefactor, double alpha, double rc2,
-                                                      int exact, double *__restrict__ force,
-                                                      double *__restrict__ torque,
-                                                      double *partials) {
-  constexpr int NT = 256, W = 2 * NSUB + 1, NN = W * W * W;
-  constexpr int TPT = 2;                  // candidate pairs tested per thread and chunk
-  constexpr int CH = NT * TPT;            // pairs per chunk
-  constexpr int QCAP = 1024, TCAP = 256;  // queue entries; candidates per table window
-  __shared__ double4 hp[NT], hm[NT];
-  __shared__ double acc[NT * 6];
-  __shared__ int2 queue[QCAP]; // (candidate index, home slot | neighbour << 16)
-  __shared__ int2 ctab[TCAP];  // (candidate index, neighbour)
-  __shared__ int nbeg[NN], npre[NN + 1];
-  __shared__ signed char nsc[NN * 3]; // periodic shift of each neighbour in box lengths
-  __shared__ int qn;
-  __shared__ double red[16];
-  int const cell = blockIdx.x;
-  int const cz = cell % g.nc[2], cy = (cell / g.nc[2]) % g.nc[1], cx = cell / (g.nc[2] * g.nc[1]);
-  int const beg = offsets[cell], end = offsets[cell + 1];
-  if (beg == end) {
-    if (EV && threadIdx.x == 0) partials[blockIdx.x * 8] = 0.;
-    return;
-  }
-  for (int o = threadIdx.x; o < NN; o += NT) {
-    int nx = cx + o / (W * W) - NSUB, ny = cy + (o / W) % W - NSUB, nz = cz + o % W - NSUB;
-    int sx = 0, sy = 0, sz = 0;
-    if (nx < 0) { nx += g.nc[0]; sx = -1; } else if (nx >= g.nc[0]) { nx -= g.nc[0]; sx = 1; }
-    if (ny < 0) { ny += g.nc[1]; sy = -1; } else if (ny >= g.nc[1]) { ny -= g.nc[1]; sy = 1; }
-    if (nz < 0) { nz += g.nc[2]; sz = -1; } else if (nz >= g.nc[2]) { nz -= g.nc[2]; sz = 1; }
-    int const nb = (nx * g.nc[1] + ny) * g.nc[2] + nz;
-    nbeg[o] = offsets[nb];
-    npre[o + 1] = offsets[nb + 1] - offsets[nb];
-    nsc[3 * o] = static_cast<signed char>(sx);
-    nsc[3 * o + 1] = static_cast<signed char>(sy);
-    nsc[3 * o + 2] = static_cast<signed char>(sz);
-  }
-  if (threadIdx.x == 0) qn = 0;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    npre[0] = 0;
-    for (int o = 0; o < NN; ++o) npre[o + 1] += npre[o];
-  }
-  __syncthreads();
-  int const ncand = npre[NN];
-  int const lane = static_cast<int>(threadIdx.x & 63);
-  double e = 0.;
-  for (int hb = beg; hb < end; hb += NT) {
-    int const ni = min(NT, end - hb);
-    if (static_cast<int>(threadIdx.x) < ni) {
-      hp[threadIdx.x] = spos[hb + threadIdx.x];
-      hm[threadIdx.x] = sdip[hb + threadIdx.x];
-    }
-    for (int x = threadIdx.x; x < ni * 6; x += NT) acc[x] = 0.;
-    for (int kw = 0; kw < ncand; kw += TCAP) {
-      int const nw = min(TCAP, ncand - kw);
-      __syncthreads(); // table readers of the previous window are done
-      for (int o = 0; o < NN; ++o) {
-        int const s0 = npre[o];
-        int const lo = max(s0, kw), hi = min(npre[o + 1], kw + nw);
-        for (int k = lo + static_cast<int>(threadIdx.x); k < hi; k += NT)
-          ctab[k - kw] = make_int2(nbeg[o] + (k - s0), o);
-      }
-      __syncthreads();
-      int const total = ni * nw;
-      bool const last_window = kw + TCAP >= ncand;
-      // pair c = k ni + il (candidate k, home slot il) of this thread:
-      // c = tid at the start, advanced by NT per test
-      int const dk = NT / ni, dil = NT - dk * ni;
-      int k = static_cast<int>(threadIdx.x) / ni;
-      int il = static_cast<int>(threadIdx.x) - k * ni;
-      for (int c0 = 0; c0 < total; c0 += CH) {
+    int64_t const i = 3 * static_cast<int64_t>(sidx[h0 + lane]);
+    if (!DIP || force) {
 #pragma unroll
-        for (int u = 0; u < TPT; ++u) {
-          bool hit = false;
-          int2 ent = make_int2(0, 0);
-          if (k < nw) { // c < total
-            int2 const cj = ctab[k];
-            double4 const pj = spos[cj.x];
-            double4 const pi = hp[il];
-            double const dx = pi.x - (pj.x + nsc[3 * cj.y] * g.L[0]);
-            double const dy = pi.y - (pj.y + nsc[3 * cj.y + 1] * g.L[1]);
-            double const dz = pi.z - (pj.z + nsc[3 * cj.y + 2] * g.L[2]);
-            double const r2 = dx * dx + dy * dy + dz * dz;
-            hit = r2 < rc2 && r2 > 0.;
-            ent = make_int2(cj.x, il | (cj.y << 16));
-          }
-          il += dil;
-          k += dk;
-          if (il >= ni) {
-            il -= ni;
-            ++k;
-          }
-          uint64_t const mask = __ballot(hit);
-          int base = 0;
-          if (lane == 0 && mask) base = atomicAdd(&qn, __popcll(mask));
-          base = __shfl(base, 0, 64);
-          if (hit) queue[base + __popcll(mask & ((1ull << lane) - 1ull))] = ent;
-        }
-        __syncthreads();
-        int const qcount = qn;
-        __syncthreads(); // every wave has read the count before it changes
-        // at most CH entries join per chunk: drain while they still fit
-        if (qcount > QCAP - CH || (last_window && c0 + CH >= total)) {
-          for (int q = threadIdx.x; q < qcount; q += NT) {
-            int2 const en = queue[q];
-            int const il = en.y & 0xffff, o = en.y >> 16;
-            double4 const pj = spos[en.x];
-            double4 const pi = hp[il];
-            double const dx = pi.x - (pj.x + nsc[3 * o] * g.L[0]);
-            double const dy = pi.y - (pj.y + nsc[3 * o + 1] * g.L[1]);
-            double const dz = pi.z - (pj.z + nsc[3 * o + 2] * g.L[2]);
-            double const r2 = dx * dx + dy * dy + dz * dz;
-            double f[3] = {0., 0., 0.}, t[3] = {0., 0., 0.};
-            dip_pair<EV>(dx, dy, dz, r2, hm[il], sdip[en.x], prefactor, alpha, exact, f, t, e);
-            atomicAdd(&acc[il * 6], f[0]);
-            atomicAdd(&acc[il * 6 + 1], f[1]);
-            atomicAdd(&acc[il * 6 + 2], f[2]);
-            atomicAdd(&acc[il * 6 + 3], t[0]);
-            atomicAdd(&acc[il * 6 + 4], t[1]);
-            atomicAdd(&acc[il * 6 + 5], t[2]);
-          }
-          __syncthreads();
-          if (threadIdx.x == 0) qn = 0;
-          __syncthreads();
-        }
-      }
+      for (int k = 0; k < 3; ++k) force[i + k] += f[k];
     }
-    if (static_cast<int>(threadIdx.x) < ni) {
-      int64_t const o = 3 * static_cast<int64_t>(sidx[hb + threadIdx.x]);
-      double const *a = acc + threadIdx.x * 6;
-      if (force) {
-        force[o] += a[0];
-        force[o + 1] += a[1];
-        force[o + 2] += a[2];
-      }
+    if constexpr (DIP) {
       if (torque) {
-        torque[o] += a[3];
-        torque[o + 1] += a[4];
-        torque[o + 2] += a[5];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) torque[i + k] += f[3 + k];
       }
     }
-    __syncthreads(); // before the next home chunk restages hp, hm and acc
   }
   if constexpr (EV) {
-    double v[1] = {e};
-    block_sum<1>(v, red);
-    if (threadIdx.x == 0) partials[blockIdx.x * 8] = v[0];
+    block_sum<NE>(ev, red);
+    if (threadIdx.x == 0)
+      for (int k = 0; k < NE; ++k) partials[static_cast<int64_t>(b) * 8 + k] = ev[k];
   }
 }
 
-/** Dipolar pair terms over cells of edge r_cut (NSUB = 1), dense evaluation
- *  per wave: one block of 256 threads per home cell.  Wave w takes the candidates w, w + 4, ... of
- *  each neighbour cell (one uniform load per candidate), its lanes the home
- *  particles; the pairs inside r_cut go to the wave's own LDS queue (ballot
- *  and a wave-uniform count, no atomics), which the wave drains itself with
- *  every lane evaluating one pair, so the pair terms run without idle
- *  lanes however sparse the cells and the loop needs no block barriers.
- *  Force and torque on each home particle accumulate in LDS (FP64 LDS
- *  atomics) and are added to the caller's arrays once. */
-template <int NSUB, bool EV>
-__global__ __launch_bounds__(256) void k_sr_dip_wave(
-    CellGrid g, int const *__restrict__ offsets, double4 const *__restrict__ spos,
-    double4 const *__restrict__ sdip, int const *__restrict__ sidx, double prefactor,
-    double alpha, double rc2, int exact, double *__restrict__ force, double *__restrict__ torque,
-    double *partials) {
-  constexpr int NT = 256, NW = NT / 64, W = 2 * NSUB + 1, NN = W * W * W;
-  constexpr int QW = 256;   // queue entries per wave
-  __shared__ double4 hp[NT], hm[NT];
-  __shared__ double acc[NT * 6];
-  __shared__ int2 queue[NW][QW]; // (candidate index, home slot | neighbour << 16)
-  __shared__ int nbeg[NN], ncnt[NN];
-  __shared__ signed char nsc[NN * 3]; // periodic shift of each neighbour in box lengths
-  __shared__ double red[16];
-  int const cell = blockIdx.x;
-  int const cz = cell % g.nc[2], cy = (cell / g.nc[2]) % g.nc[1], cx = cell / (g.nc[2] * g.nc[1]);
-  int const beg = offsets[cell], end = offsets[cell + 1];
-  if (beg == end) {
-    if (EV && threadIdx.x == 0) partials[blockIdx.x * 8] = 0.;
-    return;
+/** Columns of a box for k_sr_columns: edge >= r_cut (>= r_cut/2 along an axis
+ *  that does not hold three of those; wider columns make the 64-particle
+ *  groups compact), z bins of r_cut/4 while those hold about eight particles,
+ *  else r_cut/2. */
+struct Columns {
+  CellGrid g;
+  int reach[3];
+  int ncol, max_groups, split, sweeps;
+};
+Columns make_columns(ShortRangeParams const &p, int64_t n) {
+  Columns c;
+  double const per_cut = static_cast<double>(n) * p.r_cut * p.r_cut * p.r_cut /
+                         (p.box[0] * p.box[1] * p.box[2]);
+  for (int d = 0; d < 2; ++d) {
+    c.reach[d] = (std::floor(p.box[d] / p.r_cut) >= 3.) ? 1 : 2;
+    c.g.nc[d] =
+        std::min(kSRMaxCells, static_cast<int>(std::floor(p.box[d] * c.reach[d] / p.r_cut)));
   }
-  for (int o = threadIdx.x; o < NN; o += NT) {
-    int nx = cx + o / (W * W) - NSUB, ny = cy + (o / W) % W - NSUB, nz = cz + o % W - NSUB;
-    int sx = 0, sy = 0, sz = 0;
-    if (nx < 0) { nx += g.nc[0]; sx = -1; } else if (nx >= g.nc[0]) { nx -= g.nc[0]; sx = 1; }
-    if (ny < 0) { ny += g.nc[1]; sy = -1; } else if (ny >= g.nc[1]) { ny -= g.nc[1]; sy = 1; }
-    if (nz < 0) { nz += g.nc[2]; sz = -1; } else if (nz >= g.nc[2]) { nz -= g.nc[2]; sz = 1; }
-    int const nb = (nx * g.nc[1] + ny) * g.nc[2] + nz;
-    nbeg[o] = offsets[nb];
-    ncnt[o] = offsets[nb + 1] - offsets[nb];
-    nsc[3 * o] = static_cast<signed char>(sx);
-    nsc[3 * o + 1] = static_cast<signed char>(sy);
-    nsc[3 * o + 2] = static_cast<signed char>(sz);
+  c.reach[2] = (per_cut >= 32.) ? 4 : 2;
+  c.g.nc[2] = std::min(4 * kSRMaxCells,
+                       static_cast<int>(std::floor(p.box[2] * c.reach[2] / p.r_cut)));
+  for (int d = 0; d < 3; ++d) {
+    c.g.L[d] = p.box[d];
+    c.g.inv_cell[d] = c.g.nc[d] / p.box[d];
   }
-  int const lane = static_cast<int>(threadIdx.x & 63);
-  int const wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  int2 *const wq = queue[wave];
-  double e = 0.;
-  for (int hb = beg; hb < end; hb += NT) {
-    int const ni = min(NT, end - hb);
-    __syncthreads(); // neighbour table written; previous chunk's readers done
-    if (static_cast<int>(threadIdx.x) < ni) {
-      hp[threadIdx.x] = spos[hb + threadIdx.x];
-      hm[threadIdx.x] = sdip[hb + threadIdx.x];
-    }
-    for (int x = threadIdx.x; x < ni * 6; x += NT) acc[x] = 0.;
-    __syncthreads();
-    int const nr = (ni + 63) >> 6;
-    int count = 0; // wave-uniform
-    auto drain = [&]() {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      for (int q = lane; q < count; q += 64) {
-        int2 const en = wq[q];
-        int const il = en.y & 0xffff, o = en.y >> 16;
-        double4 const pj = spos[en.x];
-        double4 const pi = hp[il];
-        double const dx = pi.x - (pj.x + nsc[3 * o] * g.L[0]);
-        double const dy = pi.y - (pj.y + nsc[3 * o + 1] * g.L[1]);
-        double const dz = pi.z - (pj.z + nsc[3 * o + 2] * g.L[2]);
-        double const r2 = dx * dx + dy * dy + dz * dz;
-        double f[3] = {0., 0., 0.}, t[3] = {0., 0., 0.};
-        dip_pair<EV>(dx, dy, dz, r2, hm[il], sdip[en.x], prefactor, alpha, exact, f, t, e);
-        atomicAdd(&acc[il * 6], f[0]);
-        atomicAdd(&acc[il * 6 + 1], f[1]);
-        atomicAdd(&acc[il * 6 + 2], f[2]);
-        atomicAdd(&acc[il * 6 + 3], t[0]);
-        atomicAdd(&acc[il * 6 + 4], t[1]);
-        atomicAdd(&acc[il * 6 + 5], t[2]);
-      }
-      __builtin_amdgcn_wave_barrier();
-      count = 0;
-    };
-    for (int o = 0; o < NN; ++o) {
-      int const jb = __builtin_amdgcn_readfirstlane(nbeg[o]);
-      int const cnt = __builtin_amdgcn_readfirstlane(ncnt[o]);
-      double const shx = nsc[3 * o] * g.L[0], shy = nsc[3 * o + 1] * g.L[1],
-                   shz = nsc[3 * o + 2] * g.L[2];
-      for (int t = wave; t < cnt; t += NW) {
-        double4 const pj = spos[jb + t];
-        double const qx = pj.x + shx, qy = pj.y + shy, qz = pj.z + shz;
-        for (int r = 0; r < nr; ++r) {
-          int const il = lane + 64 * r;
-          double4 const pi = hp[min(il, NT - 1)];
-          double const dx = pi.x - qx, dy = pi.y - qy, dz = pi.z - qz;
-          double const r2 = dx * dx + dy * dy + dz * dz;
-          bool const hit = il < ni && r2 < rc2 && r2 > 0.;
-          uint64_t const mask = __ballot(hit);
-          if (hit)
-            wq[count + __popcll(mask & ((1ull << lane) - 1ull))] = make_int2(jb + t, il | (o << 16));
-          count += __popcll(mask);
-          // at most 64 entries join per test: drain while they still fit
-          if (count > QW - 64) drain();
-        }
-      }
-    }
-    drain();
-    __syncthreads(); // every wave's pairs are in acc
-    if (static_cast<int>(threadIdx.x) < ni) {
-      int64_t const o = 3 * static_cast<int64_t>(sidx[hb + threadIdx.x]);
-      double const *a = acc + threadIdx.x * 6;
-      if (force) {
-        force[o] += a[0];
-        force[o + 1] += a[1];
-        force[o + 2] += a[2];
-      }
-      if (torque) {
-        torque[o] += a[3];
-        torque[o + 1] += a[4];
-        torque[o + 2] += a[5];
-      }
-    }
-  }
-  if constexpr (EV) {
-    double v[1] = {e};
-    block_sum<1>(v, red);
-    if (threadIdx.x == 0) partials[blockIdx.x * 8] = v[0];
-  }
+  c.ncol = c.g.nc[0] * c.g.nc[1];
+  c.max_groups =
+      static_cast<int>(std::min<int64_t>(n, n / 64 + c.ncol)); // one partial group per column
+  // Few groups are shared by several blocks, each taking every split-th batch
+  // of candidates.  Up to 4096 blocks, four rounds of what the chip holds, as
+  // long as the lists of one wave still fill: its candidates must be a
+  // twentieth of the number of blocks.  Dipolar and Coulomb kernel, at that
+  // split against twice and half of it: 1006 groups of 980 candidates each
+  // 84 us in 2 blocks, 103 in 4, 111 in 1; 40 groups of 1900 32 us in 8, 36 in
+  // 16; 321 groups of 16,700 0.62 ms in 16, 0.71 in 8.
+  double const columns = (2. * c.reach[0] + 1.) * (2. * c.reach[1] + 1.);
+  double const in_reach = per_cut / (c.g.nc[0] * c.g.nc[1]) * p.box[0] * p.box[1] /
+                          (p.r_cut * p.r_cut); // candidates of one column per r_cut of z
+  double const tests = columns * (std::min(64., static_cast<double>(n) / c.ncol) +
+                                  2. * in_reach * (1. + 1. / c.reach[2]));
+  c.split = 1;
+  while (c.split < 16 && c.max_groups * c.split < 4096 &&
+         tests / (2 * c.split * kColWaves) >= std::max(32., 0.05 * c.max_groups * 2 * c.split))
+    c.split *= 2;
+  // one pass over the columns per 16 candidates (four batches) that a wave
+  // takes of each: with 4 against 16 passes, 200,000 dipoles of 4300 partners
+  // 9.3 against 6.9 ms; 2 against 4 passes at 105 partners 0.39 against 0.44 ms
+  c.sweeps = std::clamp(static_cast<int>(tests / (columns * 16. * c.split * kColWaves)), 1, 16);
+  return c;
 }
 
 template <typename T> void sr_grow(T *&p, size_t &cap, size_t need, char const *what) {
@@ -977,6 +776,16 @@ struct ShortRange::Impl {
   double4 *spos = nullptr;
   double *partials = nullptr;
   size_t cap_cells = 0, cap_off = 0, cap_pc = 0, cap_pr = 0, cap_si = 0, cap_sp = 0, cap_part = 0;
+
+  /** Buffers of the column search (nv sums per particle). */
+  void grow_columns(Columns const &c, int nv) {
+    sr_grow(goff, cap_goff, static_cast<size_t>(c.ncol) + 1, "hipMalloc group offsets");
+    sr_grow(grp, cap_grp, static_cast<size_t>(c.max_groups), "hipMalloc groups");
+    sr_grow(arrived, cap_arrived, static_cast<size_t>(c.max_groups), "hipMalloc groups");
+    if (c.split > 1)
+      sr_grow(shares, cap_shares, static_cast<size_t>(c.max_groups) * c.split * 64 * nv,
+              "hipMalloc group shares");
+  }
 };
 
 ShortRange::ShortRange(int device) : m(new Impl) { m->device = device; }
@@ -1042,46 +851,22 @@ void ShortRange::compute(hipStream_t st, ShortRangeParams const &p, int64_t n, d
     m->nc[d] = g.nc[d] = nc[d];
     g.L[d] = p.box[d];
   }
-  // without ELC images the pairs run over columns: edge >= r_cut (>= r_cut/2
-  // along an axis that does not hold three of those; wider columns make the
-  // 64-particle groups compact), z bins of r_cut/4 while those hold about
-  // eight particles, else r_cut/2
+  // without ELC images the pairs run over columns
   bool const columns = nsub != 0 && !p.elc_images;
-  int reach[3] = {1, 1, 1};
+  Columns cols{};
   if (columns) {
-    double const per_cut = static_cast<double>(n) * p.r_cut * p.r_cut * p.r_cut /
-                           (p.box[0] * p.box[1] * p.box[2]);
-    for (int d = 0; d < 2; ++d) {
-      reach[d] = (std::floor(p.box[d] / p.r_cut) >= 3.) ? 1 : 2;
-      g.nc[d] = std::min(kSRMaxCells, static_cast<int>(std::floor(p.box[d] * reach[d] / p.r_cut)));
-    }
-    reach[2] = (per_cut >= 32.) ? 4 : 2;
-    g.nc[2] = std::min(4 * kSRMaxCells,
-                       static_cast<int>(std::floor(p.box[2] * reach[2] / p.r_cut)));
+    cols = make_columns(p, n);
+    g = cols.g;
   }
   for (int d = 0; d < 3; ++d) g.inv_cell[d] = g.nc[d] / p.box[d];
-  int const ncells = g.nc[0] * g.nc[1] * g.nc[2], ncol = g.nc[0] * g.nc[1];
-  int const max_groups =
-      static_cast<int>(std::min<int64_t>(n, n / 64 + ncol)); // at most one partial per column
-  int split = 1;
+  int const ncells = g.nc[0] * g.nc[1] * g.nc[2];
   sr_grow(m->counts, m->cap_cells, static_cast<size_t>(ncells), "hipMalloc cell counts");
   sr_grow(m->offsets, m->cap_off, static_cast<size_t>(ncells) + 1, "hipMalloc cell offsets");
   sr_grow(m->p_cell, m->cap_pc, static_cast<size_t>(n), "hipMalloc cell ids");
   sr_grow(m->p_rank, m->cap_pr, static_cast<size_t>(n), "hipMalloc cell ranks");
   sr_grow(m->sidx, m->cap_si, static_cast<size_t>(n), "hipMalloc cell order");
   sr_grow(m->spos, m->cap_sp, static_cast<size_t>(n) + kSortedSlack, "hipMalloc cell positions");
-  if (columns) {
-    sr_grow(m->goff, m->cap_goff, static_cast<size_t>(ncol) + 1, "hipMalloc group offsets");
-    sr_grow(m->grp, m->cap_grp, static_cast<size_t>(max_groups), "hipMalloc groups");
-    sr_grow(m->arrived, m->cap_arrived, static_cast<size_t>(max_groups), "hipMalloc groups");
-    // about 8192 waves, two rounds of the chip's 1024 SIMDs at four to five
-    // each: few groups are shared by several blocks (18 groups: 41 us in 16
-    // shares, 57 us in one block of 16 waves each)
-    while (split < 16 && max_groups * split < 2048) split *= 2;
-    if (split > 1)
-      sr_grow(m->shares, m->cap_shares, static_cast<size_t>(max_groups) * split * 192,
-              "hipMalloc group shares");
-  }
+  if (columns) m->grow_columns(cols, 3);
   int const nb = static_cast<int>((n + 255) / 256);
   k_sr_fill<<<std::min((ncells + 255) / 256, 1024), 256, 0, st>>>(m->counts, ncells);
   k_sr_bin<<<nb, 256, 0, st>>>(n, pos, q, g, m->counts, m->p_cell, m->p_rank);
@@ -1090,7 +875,7 @@ void ShortRange::compute(hipStream_t st, ShortRangeParams const &p, int64_t n, d
   k_sr_scatter<<<nb, 256, 0, st>>>(n, pos, q, g, m->p_cell, m->p_rank, m->offsets, m->spos,
                                    m->sidx, g.nc[2], m->goff, columns ? m->grp : nullptr);
   double const rc2 = p.r_cut * p.r_cut;
-  int blocks = columns ? max_groups * split : ncells;
+  int blocks = columns ? cols.max_groups * cols.split : ncells;
   int nq = 0;
   if (nsub == 0) {
     // all-pairs: the number of charged particles decides the grid
@@ -1104,9 +889,11 @@ void ShortRange::compute(hipStream_t st, ShortRangeParams const &p, int64_t n, d
   auto launch = [&](auto EVc) {
     constexpr bool EV = decltype(EVc)::value;
     if (columns) {
-      k_sr_columns<EV><<<blocks, kColWaves * 64, 0, st>>>(
-          g, reach[0], reach[1], reach[2], split, split > 1 ? 1 : 4, m->offsets, m->goff, m->grp,
-          m->spos, m->sidx, p.prefactor, p.alpha, rc2, force, m->shares, m->arrived, m->partials);
+      k_sr_columns<false, EV, false><<<blocks, kColWaves * 64, 0, st>>>(
+          g, cols.reach[0], cols.reach[1], cols.reach[2], cols.split, cols.sweeps,
+          m->offsets, m->goff, m->grp,
+          m->spos, nullptr, m->sidx, p.prefactor, p.alpha, rc2, force, nullptr, m->shares,
+          m->arrived, m->partials);
     } else if (nsub == 2) {
       k_sr_cells<2, 64, EV><<<blocks, 64, 0, st>>>(g, m->offsets, m->spos, m->sidx, p.prefactor,
                                                    p.alpha, rc2, force, m->partials, im);
@@ -1146,78 +933,60 @@ bool ShortRange::compute_dipolar(hipStream_t st, ShortRangeParams const &p, bool
   if (energy) *energy = 0.;
   if (!(p.r_cut > 0.)) throw std::invalid_argument("P3M: short range needs r_cut > 0");
   if (n > INT32_MAX) throw std::invalid_argument("P3M: too many particles for the short range");
-  int nsub = (p.subdivision == 1) ? 1 : 2;
-  int nc[3];
-  auto fit = [&](int s) {
-    bool ok = true;
-    for (int d = 0; d < 3; ++d) {
-      nc[d] = std::min(kSRMaxCells, static_cast<int>(std::floor(p.box[d] * s / p.r_cut)));
-      if (nc[d] < 2 * s + 1) ok = false;
-    }
-    return ok;
-  };
-  if (!fit(nsub)) {
-    nsub = 1;
-    if (!fit(1)) return false;
-  }
+  // three cells of r_cut along every axis, or five of r_cut/2 if allowed
+  for (int d = 0; d < 3; ++d)
+    if (std::floor(p.box[d] / p.r_cut) < 3. &&
+        (p.subdivision == 1 || std::floor(2. * p.box[d] / p.r_cut) < 5.))
+      return false;
   if (n == 0) return true;
   hip_check(hipSetDevice(m->device), "hipSetDevice");
-  CellGrid g;
-  for (int d = 0; d < 3; ++d) {
-    m->nc[d] = g.nc[d] = nc[d];
-    g.L[d] = p.box[d];
-    g.inv_cell[d] = nc[d] / p.box[d];
-  }
-  int const ncells = nc[0] * nc[1] * nc[2];
+  Columns const cols = make_columns(p, n);
+  CellGrid const &g = cols.g;
+  int const ncells = cols.ncol * g.nc[2];
   sr_grow(m->counts, m->cap_cells, static_cast<size_t>(ncells), "hipMalloc cell counts");
   sr_grow(m->offsets, m->cap_off, static_cast<size_t>(ncells) + 1, "hipMalloc cell offsets");
   sr_grow(m->p_cell, m->cap_pc, static_cast<size_t>(n), "hipMalloc cell ids");
   sr_grow(m->p_rank, m->cap_pr, static_cast<size_t>(n), "hipMalloc cell ranks");
   sr_grow(m->sidx, m->cap_si, static_cast<size_t>(n), "hipMalloc cell order");
-  sr_grow(m->spos, m->cap_sp, static_cast<size_t>(n), "hipMalloc cell positions");
+  sr_grow(m->spos, m->cap_sp, static_cast<size_t>(n) + kSortedSlack, "hipMalloc cell positions");
   sr_grow(m->mu2, m->cap_mu2, static_cast<size_t>(n), "hipMalloc dipole norms");
   sr_grow(m->sdip, m->cap_sdip, static_cast<size_t>(n), "hipMalloc cell dipoles");
-  if (energy) sr_grow(m->partials, m->cap_part, static_cast<size_t>(ncells) * 8, "hipMalloc partials");
+  m->grow_columns(cols, 6);
+  int const blocks = cols.max_groups * cols.split;
+  if (energy) sr_grow(m->partials, m->cap_part, static_cast<size_t>(blocks) * 8, "hipMalloc partials");
   int const nb = static_cast<int>((n + 255) / 256);
-  k_sr_mu2<<<nb, 256, 0, st>>>(n, dip, m->mu2);
-  k_sr_fill<<<std::min((ncells + 255) / 256, 1024), 256, 0, st>>>(m->counts, ncells);
+  k_sr_mu2<<<nb, 256, 0, st>>>(n, dip, m->mu2, m->counts, ncells);
   k_sr_bin<<<nb, 256, 0, st>>>(n, pos, m->mu2, g, m->counts, m->p_cell, m->p_rank);
-  k_sr_scan<<<1, 1024, 0, st>>>(m->counts, ncells, m->offsets, 1, nullptr, nullptr);
+  k_sr_scan<<<1, 1024, 0, st>>>(m->counts, ncells, m->offsets, g.nc[2], m->goff, m->arrived);
   k_sr_scatter<<<nb, 256, 0, st>>>(n, pos, m->mu2, g, m->p_cell, m->p_rank, m->offsets, m->spos,
-                                   m->sidx, 1, nullptr, nullptr);
+                                   m->sidx, g.nc[2], m->goff, m->grp);
   k_sr_sort_dip<<<nb, 256, 0, st>>>(n, m->offsets + ncells, m->sidx, dip, m->sdip);
   double const rc2 = p.r_cut * p.r_cut;
-  int const ex = exact_erfc ? 1 : 0;
-  auto launch = [&](auto EVc) {
-    constexpr bool EV = decltype(EVc)::value;
-    if (nsub == 2)
-      k_sr_dip_queue<2, EV><<<ncells, 256, 0, st>>>(g, m->offsets, m->spos, m->sdip, m->sidx,
-                                                    p.prefactor, p.alpha, rc2, ex, force, torque,
-                                                    m->partials);
-    // cells of r_cut: the per-wave kernel needs about half a wave of home
-    // particles per cell; sparser cells run faster on the block queue
-    else if (static_cast<double>(n) >= 32. * static_cast<double>(ncells))
-      k_sr_dip_wave<1, EV><<<ncells, 256, 0, st>>>(g, m->offsets, m->spos, m->sdip, m->sidx,
-                                                   p.prefactor, p.alpha, rc2, ex, force, torque,
-                                                   m->partials);
-    else
-      k_sr_dip_queue<1, EV><<<ncells, 256, 0, st>>>(g, m->offsets, m->spos, m->sdip, m->sidx,
-                                                    p.prefactor, p.alpha, rc2, ex, force, torque,
-                                                    m->partials);
+  auto launch = [&](auto EVc, auto EXc) {
+    k_sr_columns<true, decltype(EVc)::value, decltype(EXc)::value>
+        <<<blocks, kColWaves * 64, 0, st>>>(g, cols.reach[0], cols.reach[1], cols.reach[2],
+                                            cols.split, cols.sweeps, m->offsets,
+                                            m->goff, m->grp, m->spos, m->sdip, m->sidx,
+                                            p.prefactor, p.alpha, rc2, force, torque, m->shares,
+                                            m->arrived, m->partials);
   };
-  if (energy)
-    launch(std::true_type{});
+  if (energy && exact_erfc)
+    launch(std::true_type{}, std::true_type{});
+  else if (energy)
+    launch(std::true_type{}, std::false_type{});
+  else if (exact_erfc)
+    launch(std::false_type{}, std::true_type{});
   else
-    launch(std::false_type{});
+    launch(std::false_type{}, std::false_type{});
   hip_check(hipGetLastError(), "dipolar short-range kernels");
   if (!energy) return true;
-  std::vector<double> part(static_cast<size_t>(ncells) * 8);
+  std::vector<double> part(static_cast<size_t>(blocks) * 8);
   hip_check(hipMemcpyAsync(part.data(), m->partials, sizeof(double) * part.size(),
                            hipMemcpyDeviceToHost, st),
             "copy partials");
   hip_check(hipStreamSynchronize(st), "sync dipolar short range");
   double s = 0.;
-  for (int c = 0; c < ncells; ++c) s += part[static_cast<size_t>(c) * 8];
+  for (int b = 0; b < blocks; ++b) s += part[static_cast<size_t>(b) * 8];
   *energy = 0.5 * s;
   return true;
 }

@@ -344,8 +344,9 @@ int p3m_dipolar_solve(p3m_dipolar *ctx, int64_t n, const double *pos, const doub
  * below half the box): forces and torques added, energy with P3M_ENERGY. */
 int p3m_dipolar_short_range(p3m_dipolar *ctx, int64_t n, const double *pos, const double *dip,
                             double *force, double *torque, unsigned flags, double *energy);
-/* Cells per r_cut of p3m_dipolar_short_range: 0 = by occupancy (r_cut/2
- * cells when they hold about 40 dipoles or more), 1 or 2. */
+/* Cells per r_cut of p3m_dipolar_short_range: 0 = automatic, 1 or 2; as for
+ * p3m_set_short_range_subdivision, all pairs are taken in boxes narrower than
+ * 3 r_cut with 1, else 2.5 r_cut. */
 int p3m_dipolar_set_short_range_subdivision(p3m_dipolar *ctx, int cells_per_cutoff);
 int p3m_dipolar_get_stream(const p3m_dipolar *ctx, void **stream);
 int p3m_dipolar_wait_stream(p3m_dipolar *ctx, void *producer); /* as p3m_wait_stream */

@@ -147,6 +147,40 @@ def test_short_range_dense_cluster_matches_oracle(subdiv, r_cut):
 
 
 @pytest.mark.parametrize("accuracy", [1e-4, 1e-7])
+@pytest.mark.parametrize("L,r_cut,n,spread", [
+    (9., 2.2, 1, 1.),            # no pair at all
+    (9., 2.2, 2, 0.1),
+    (9., 2.2, 700, 0.25),        # crowded columns: full groups of 64 and a remainder
+    (5.8, 2.2, 64 * 14 + 1, 1.), # five columns of r_cut/2 along x and y
+    (130., 2., 4000, 0.05),      # 65 columns along x, one block per group
+])
+def test_dipolar_column_pairs_match_oracle(L, r_cut, n, spread, accuracy):
+    """Forces, torques and energy of the column kernel at the edges of its
+    home groups, reaches and block shares, some dipoles zero; then torques and
+    forces alone.  Tolerance as in the other real-space tests: FP64 sums of
+    the same terms."""
+    import torch
+    from espresso_amd.magnetostatics import DipolarP3M
+    from oracle import dp3m as D
+    rng = np.random.default_rng(n)
+    pos = (rng.uniform(-0.5, 0.5, (n, 3)) * spread * L) % L
+    dip = rng.normal(size=(n, 3)) * (np.arange(n) % 7 != 3)[:, None]
+    dp = DipolarP3M(prefactor=1.3, accuracy=accuracy, mesh=16, cao=4, alpha=1.1, r_cut=r_cut,
+                    tune=False)
+    dp.activate(pos, dip, box_l=L)
+    tp, td = torch.tensor(pos, device="cuda"), torch.tensor(dip, device="cuda")
+    tf, tt, f1, t1 = (torch.zeros_like(tp) for _ in range(4))
+    e = dp.add_short_range_forces(tp, td, tf, tt, energy=True)
+    dp.add_short_range_forces(tp, td, None, t1)
+    dp.add_short_range_forces(tp, td, f1, None)
+    fr, tr, er = D.pair_terms(pos, dip, L, 1.3, 1.1, r_cut, accuracy)
+    for got, ref in ((tf, fr), (tt, tr), (f1, fr), (t1, tr)):
+        scale = max(np.sqrt(np.mean(ref ** 2)), 1e-300)
+        assert np.sqrt(np.mean((got.cpu().numpy() - ref) ** 2)) <= 1e-12 * scale
+    assert abs(e - er) <= 1e-12 * abs(er)
+
+
+@pytest.mark.parametrize("accuracy", [1e-4, 1e-7])
 def test_short_range_matches_oracle(accuracy):
     """A&S erfc for accuracy > 5e-6, libm erfc below (dp3m.hpp:176-178)."""
     import torch
