@@ -20,7 +20,9 @@ using C2 = double2;
 constexpr int kDpBlock = 256;
 constexpr int kDpLines = 8; // FFT lines per block
 constexpr int kDpGatherBlock = 512;
-constexpr int kDpPlaneBlock = 1024; // threads of the z/y plane transform
+// most threads of the z/y plane transform: 512 when two blocks share the LDS
+// of a CU, else all
+constexpr int kDpPlaneBlock = 1024;
 // bucket counters per bucket: block b counts into copy b % kDpCopies, which
 // spreads the returning atomics on one bucket over several addresses
 constexpr int kDpCopies = 8;
@@ -30,13 +32,14 @@ constexpr int kDpGatherLds = 160 * 1024 - 256;
 
 
 
-/** Start of a solve: the three dipole meshes (blockIdx.y), the bucket
- *  counters and the error flag set to zero in one launch. */
-__global__ __launch_bounds__(kDpBlock) void k_dp_prep(C2 *a0, C2 *a1, C2 *a2, int64_t m3,
-                                                      int *counts, int nk, int *err) {
+/** Start of a solve: the three dipole meshes (blockIdx.y, two points per
+ *  thread), the bucket counters and the error flag set to zero in one launch. */
+__global__ __launch_bounds__(kDpBlock) void k_dp_prep(double *a0, double *a1, double *a2,
+                                                      int64_t pairs, int *counts, int nk,
+                                                      int *err) {
   int64_t const i = (int64_t)blockIdx.x * kDpBlock + threadIdx.x;
-  C2 *a = blockIdx.y == 0 ? a0 : blockIdx.y == 1 ? a1 : a2;
-  if (i < m3) a[i] = C2{0., 0.};
+  double *a = blockIdx.y == 0 ? a0 : blockIdx.y == 1 ? a1 : a2;
+  if (i < pairs) reinterpret_cast<C2 *>(a)[i] = C2{0., 0.};
   if (blockIdx.y == 0 && i < (int64_t)nk * kDpCopies) counts[i] = 0;
   if (blockIdx.y == 0 && i == 0) *err = 0;
 }
@@ -65,8 +68,8 @@ __device__ __forceinline__ bool dp_weights(DevGeo const &g, double const x[3], i
 template <int P>
 __global__ __launch_bounds__(kDpBlock) void k_dp_spread_tile(
     int const *__restrict__ offsets, int const *__restrict__ counts,
-    double const *__restrict__ pos, double const *__restrict__ dip, DevGeo g, int E, C2 *A0,
-    C2 *A1, C2 *A2, int *err) {
+    double const *__restrict__ pos, double const *__restrict__ dip, DevGeo g, int E,
+    double *A0, double *A1, double *A2, int *err) {
   extern __shared__ double tile[]; // [3][E][E][E]
   __shared__ int org[3];
   int const beg = offsets[blockIdx.x], cnt = counts[blockIdx.x];
@@ -134,9 +137,9 @@ __global__ __launch_bounds__(kDpBlock) void k_dp_spread_tile(
         for (int b = 0; b < P; ++b) {
           int64_t const idx = ((int64_t)ix * M + wrap_once(gi[1] + b, M)) * M + iz;
           double const wt = w[0][rr] * w[1][b] * wz;
-          atomicAdd(&A0[idx].x, wt * mu[0]);
-          atomicAdd(&A1[idx].x, wt * mu[1]);
-          atomicAdd(&A2[idx].x, wt * mu[2]);
+          atomicAdd(&A0[idx], wt * mu[0]);
+          atomicAdd(&A1[idx], wt * mu[1]);
+          atomicAdd(&A2[idx], wt * mu[2]);
         }
       }
     }
@@ -150,93 +153,175 @@ __global__ __launch_bounds__(kDpBlock) void k_dp_spread_tile(
     int const tz = e % E, ty = (e / E) % E, tx = e / (E * E);
     int64_t const idx =
         ((int64_t)((b0 + tx) % M) * M + (b1 + ty) % M) * M + (b2 + tz) % M;
-    if (v0 != 0.) atomicAdd(&A0[idx].x, v0);
-    if (v1 != 0.) atomicAdd(&A1[idx].x, v1);
-    if (v2 != 0.) atomicAdd(&A2[idx].x, v2);
+    if (v0 != 0.) atomicAdd(&A0[idx], v0);
+    if (v1 != 0.) atomicAdd(&A1[idx], v1);
+    if (v2 != 0.) atomicAdd(&A2[idx], v2);
   }
 }
 
-/** In-place complex FFT of the lines along `axis` of nmesh cubic meshes
- *  (blockIdx.y: mesh), kDpLines lines per block, unnormalised, forward
- *  sign -1 (inv: +1).  With rout, the real parts go to the real meshes
- *  rout[mesh] instead (the last pass of a back transform). */
+// The meshes are real, so the transforms keep the half spectrum [x][y][kz],
+// kz <= M / 2: z lines a and b go through one complex transform as a + i b.
+
+/** Spectra A, B (kz <= M / 2) of the real lines a, b from the transform c of
+ *  a + i b: A = (c(kz) + conj c(-kz)) / 2, B = (c(kz) - conj c(-kz)) / 2i. */
+__device__ __forceinline__ void split_pair(C2 const *c, int M, int kz, C2 &A, C2 &B) {
+  C2 const u = c[kz], v = c[kz ? M - kz : 0];
+  A = C2{0.5 * (u.x + v.x), 0.5 * (u.y - v.y)};
+  B = C2{0.5 * (u.y + v.y), 0.5 * (v.x - u.x)};
+}
+
+/** Spectrum of a + i b from the half spectra of the real lines a, b: elements
+ *  kz and -kz (the imaginary parts of kz = 0 and M / 2 are zero). */
+__device__ __forceinline__ void join_pair(C2 const &A, C2 const &B, int M, int kz, C2 *c) {
+  if (kz == 0 || 2 * kz == M) {
+    c[kz] = C2{A.x, B.x};
+  } else {
+    c[kz] = C2{A.x - B.y, A.y + B.x};
+    c[M - kz] = C2{A.x + B.y, B.x - A.y};
+  }
+}
+
+/** In-place complex FFT of the lines along x (axis 0) or y (axis 1) of nmesh
+ *  half spectra (blockIdx.y: mesh), kDpLines lines per block, unnormalised,
+ *  forward sign -1 (inv: +1).  Neighbouring lanes take neighbouring lines
+ *  (consecutive kz): 128 contiguous bytes per element of the lines. */
 __global__ __launch_bounds__(kDpBlock) void k_dp_fft(C2 *const *meshes, int M, int axis,
                                                      FftPlanDev plan, C2 const *__restrict__ tw,
-                                                     bool inv, double *const *rout) {
+                                                     bool inv) {
   extern __shared__ double smem_d[];
   C2 *twl = reinterpret_cast<C2 *>(smem_d);
-  int const ls = M + 1;
+  int const ls = M + 1, Kz = M / 2 + 1;
   C2 *X = twl + M;
   C2 *Y = X + kDpLines * ls;
   for (int m = threadIdx.x; m < M; m += blockDim.x) twl[m] = tw[m];
   C2 *data = meshes[blockIdx.y];
-  int64_t const M2 = (int64_t)M * M;
+  int const plane = M * Kz;
   int const l0 = blockIdx.x * kDpLines;
-  int const nl = min(kDpLines, static_cast<int>(M2 - l0));
-  int64_t const stride = axis == 2 ? 1 : axis == 1 ? M : M2;
-  auto base = [&](int l) -> int64_t {
-    if (axis == 2) return (int64_t)l * M;
-    int const hi = l / M, lo = l - hi * M;
-    return axis == 1 ? (int64_t)hi * M2 + lo : (int64_t)hi * M + lo;
+  int const nl = min(kDpLines, plane - l0);
+  int64_t const stride = axis == 1 ? Kz : plane;
+  auto base = [&](int l) -> int64_t { // of line l: (y, kz) along x, (x, kz) along y
+    if (axis == 0) return l;
+    int const x = l / Kz;
+    return (int64_t)x * plane + (l - x * Kz);
   };
   for (int e = threadIdx.x; e < kDpLines * M; e += blockDim.x) {
-    int const l = e / M, j = e - l * M;
+    int const j = e / kDpLines, l = e % kDpLines;
     X[l * ls + j] = (l < nl) ? data[base(l0 + l) + j * stride] : C2{0., 0.};
   }
   __syncthreads();
-  C2 *res = lds_fft(X, Y, kDpLines, ls, plan, twl, inv);
-  if (rout) { // last pass of a back transform: real parts only, compact
-    double *r = rout[blockIdx.y];
-    for (int e = threadIdx.x; e < nl * M; e += blockDim.x) {
-      int const l = e / M, j = e - l * M;
-      r[base(l0 + l) + j * stride] = res[l * ls + j].x;
-    }
-    return;
-  }
-  for (int e = threadIdx.x; e < nl * M; e += blockDim.x) {
-    int const l = e / M, j = e - l * M;
-    data[base(l0 + l) + j * stride] = res[l * ls + j];
+  C2 const *res = lds_fft(X, Y, kDpLines, ls, plan, twl, inv);
+  for (int e = threadIdx.x; e < kDpLines * M; e += blockDim.x) {
+    int const j = e / kDpLines, l = e % kDpLines;
+    if (l < nl) data[base(l0 + l) + j * stride] = res[l * ls + j];
   }
 }
 
-/** z and y transforms of one x plane (blockIdx.x) of nmesh cubic meshes
- *  (blockIdx.y) in LDS: z lines, a transpose, then y lines, for meshes whose
- *  plane fits twice in a workgroup's LDS.  Unnormalised, sign as k_dp_fft. */
-__global__ __launch_bounds__(kDpPlaneBlock) void k_dp_fft_zy(C2 *const *meshes, int M,
-                                                             FftPlanDev plan,
-                                                             C2 const *__restrict__ tw, bool inv) {
+/** z transforms between nmesh real meshes (blockIdx.y) and their half
+ *  spectra, kDpLines pairs of lines per block: real to complex, or (inv)
+ *  complex to real.  For meshes whose plane does not fit k_dp_fft_plane. */
+__global__ __launch_bounds__(kDpBlock) void k_dp_fft_z(double *const *real, C2 *const *meshes,
+                                                       int M, FftPlanDev plan,
+                                                       C2 const *__restrict__ tw, bool inv) {
   extern __shared__ double smem_d[];
   C2 *twl = reinterpret_cast<C2 *>(smem_d);
-  int const ls = M + 1;
-  int const MM = M * M;
+  int const ls = M + 1, Kz = M / 2 + 1;
   C2 *X = twl + M;
-  C2 *Y = X + M * ls;
+  C2 *Y = X + kDpLines * ls;
   for (int m = threadIdx.x; m < M; m += blockDim.x) twl[m] = tw[m];
-  C2 *data = meshes[blockIdx.y] + (int64_t)blockIdx.x * MM;
-  for (int e = threadIdx.x; e < MM; e += blockDim.x) {
-    int const y = e / M, z = e - y * M;
-    X[y * ls + z] = data[e];
-  }
+  int64_t const p0 = (int64_t)blockIdx.x * kDpLines; // pairs of lines (x, y), y even
+  int const np = static_cast<int>(min((int64_t)kDpLines, (int64_t)M * M / 2 - p0));
+  double *r = real[blockIdx.y] + 2 * p0 * M;
+  C2 *h = meshes[blockIdx.y] + 2 * p0 * Kz;
+  if (inv)
+    for (int e = threadIdx.x; e < np * Kz; e += blockDim.x) {
+      int const p = e / Kz, kz = e - p * Kz;
+      join_pair(h[2 * p * Kz + kz], h[(2 * p + 1) * Kz + kz], M, kz, X + p * ls);
+    }
+  else
+    for (int e = threadIdx.x; e < np * M; e += blockDim.x) {
+      int const p = e / M, z = e - p * M;
+      X[p * ls + z] = C2{r[2 * p * M + z], r[(2 * p + 1) * M + z]};
+    }
   __syncthreads();
-  C2 *r1 = lds_fft(X, Y, M, ls, plan, twl, inv); // along z, line y
-  C2 *o = (r1 == X) ? Y : X;
-  for (int e = threadIdx.x; e < MM; e += blockDim.x) {
-    int const y = e / M, z = e - y * M;
-    o[z * ls + y] = r1[y * ls + z];
-  }
-  __syncthreads();
-  C2 *r2 = lds_fft(o, r1, M, ls, plan, twl, inv); // along y, line z
-  for (int e = threadIdx.x; e < MM; e += blockDim.x) {
-    int const y = e / M, z = e - y * M;
-    data[e] = r2[z * ls + y];
+  C2 const *res = lds_fft(X, Y, np, ls, plan, twl, inv);
+  if (inv)
+    for (int e = threadIdx.x; e < np * M; e += blockDim.x) {
+      int const p = e / M, z = e - p * M;
+      C2 const v = res[p * ls + z];
+      r[2 * p * M + z] = v.x;
+      r[(2 * p + 1) * M + z] = v.y;
+    }
+  else
+    for (int e = threadIdx.x; e < np * Kz; e += blockDim.x) {
+      int const p = e / Kz, kz = e - p * Kz;
+      split_pair(res + p * ls, M, kz, h[2 * p * Kz + kz], h[(2 * p + 1) * Kz + kz]);
+    }
+}
+
+/** z and y transforms of one x plane (blockIdx.x) of nmesh meshes
+ *  (blockIdx.y) in LDS: pairs of real z lines, then the M / 2 + 1 y lines of
+ *  the half spectrum; inv the other way round.  For meshes whose half plane
+ *  fits twice in a workgroup's LDS.  Unnormalised, sign as k_dp_fft.
+ *  Bound by latency: a plane passes LDS four to six times, one barrier each. */
+__global__ __launch_bounds__(kDpPlaneBlock) void k_dp_fft_plane(double *const *real,
+                                                                C2 *const *meshes, int M,
+                                                                FftPlanDev plan,
+                                                                C2 const *__restrict__ tw,
+                                                                bool inv) {
+  extern __shared__ double smem_d[];
+  C2 *twl = reinterpret_cast<C2 *>(smem_d);
+  int const ls = M + 1, Kz = M / 2 + 1;
+  C2 *X = twl + M;
+  C2 *Y = X + Kz * ls;
+  for (int m = threadIdx.x; m < M; m += blockDim.x) twl[m] = tw[m];
+  double *r = real[blockIdx.y] + (int64_t)blockIdx.x * M * M;
+  C2 *h = meshes[blockIdx.y] + (int64_t)blockIdx.x * M * Kz;
+  if (!inv) {
+    for (int e = threadIdx.x; e < M * M / 2; e += blockDim.x) {
+      int const p = e / M, z = e - p * M;
+      X[p * ls + z] = C2{r[2 * p * M + z], r[(2 * p + 1) * M + z]};
+    }
+    __syncthreads();
+    C2 *c = lds_fft(X, Y, M / 2, ls, plan, twl, false); // along z, pairs of lines y
+    C2 *o = (c == X) ? Y : X;
+    for (int e = threadIdx.x; e < M / 2 * Kz; e += blockDim.x) {
+      int const p = e / Kz, kz = e - p * Kz;
+      split_pair(c + p * ls, M, kz, o[kz * ls + 2 * p], o[kz * ls + 2 * p + 1]);
+    }
+    __syncthreads();
+    C2 const *res = lds_fft(o, c, Kz, ls, plan, twl, false); // along y, line kz
+    for (int e = threadIdx.x; e < M * Kz; e += blockDim.x) {
+      int const y = e / Kz, kz = e - y * Kz;
+      h[e] = res[kz * ls + y];
+    }
+  } else {
+    for (int e = threadIdx.x; e < M * Kz; e += blockDim.x) {
+      int const y = e / Kz, kz = e - y * Kz;
+      X[kz * ls + y] = h[e];
+    }
+    __syncthreads();
+    C2 *c = lds_fft(X, Y, Kz, ls, plan, twl, true);
+    C2 *o = (c == X) ? Y : X;
+    for (int e = threadIdx.x; e < M / 2 * Kz; e += blockDim.x) {
+      int const p = e / Kz, kz = e - p * Kz;
+      join_pair(c[kz * ls + 2 * p], c[kz * ls + 2 * p + 1], M, kz, o + p * ls);
+    }
+    __syncthreads();
+    C2 const *res = lds_fft(o, c, M / 2, ls, plan, twl, true);
+    for (int e = threadIdx.x; e < M * M / 2; e += blockDim.x) {
+      int const p = e / M, z = e - p * M;
+      C2 const v = res[p * ls + z];
+      r[2 * p * M + z] = v.x;
+      r[(2 * p + 1) * M + z] = v.y;
+    }
   }
 }
 
 /** k-space step (dp3m.cpp:270-311, 322-343, 369-389) and back-transform
- *  meshes in one pass over the mesh (Nyquist wave number 0): with
+ *  meshes in one pass over the half spectrum (Nyquist wave number 0): with
  *  the transformed dipole components A_d (table entries 0..2) and the
  *  integer wave numbers D, z = sum_d D_d A_d gives the energy partials
- *  G_e |z|^2.  With back != 0 the field meshes T_d = D_d G_e z overwrite
+ *  G_e |z|^2, twice where -k lies in the other half.  With back != 0 the field meshes T_d = D_d G_e z overwrite
  *  A_d, and with forces != 0 the six force meshes F_ab = D_a D_b (-i G_f z)
  *  (xx xy xz yy yz zz, table entries 3..8) are written. */
 __global__ __launch_bounds__(kDpBlock) void k_dp_kspace(C2 *const *T, C2 *const *F,
@@ -245,13 +330,13 @@ __global__ __launch_bounds__(kDpBlock) void k_dp_kspace(C2 *const *T, C2 *const 
                                                         int back, int forces,
                                                         double *partials) {
   __shared__ double red[16];
-  int64_t const M3 = (int64_t)M * M * M;
+  int const Kz = M / 2 + 1;
   int64_t const k = (int64_t)blockIdx.x * kDpBlock + threadIdx.x;
   double e = 0.;
-  if (k < M3) {
-    int const iz = static_cast<int>(k % M);
-    int const iy = static_cast<int>((k / M) % M);
-    int const ix = static_cast<int>(k / ((int64_t)M * M));
+  if (k < (int64_t)M * M * Kz) {
+    int const iz = static_cast<int>(k % Kz);
+    int const iy = static_cast<int>((k / Kz) % M);
+    int const ix = static_cast<int>(k / ((int64_t)M * Kz));
     double const D[3] = {static_cast<double>(dop_shift(ix, M)),
                          static_cast<double>(dop_shift(iy, M)),
                          static_cast<double>(dop_shift(iz, M))};
@@ -259,7 +344,7 @@ __global__ __launch_bounds__(kDpBlock) void k_dp_kspace(C2 *const *T, C2 *const 
     double const re = D[0] * a0.x + D[1] * a1.x + D[2] * a2.x;
     double const im = D[0] * a0.y + D[1] * a1.y + D[2] * a2.y;
     double const ge = Ge[k];
-    e = ge * (re * re + im * im);
+    e = ge * (re * re + im * im) * ((iz == 0 || 2 * iz == M) ? 1. : 2.);
     if (back) {
       C2 const kt = C2{ge * re, ge * im};
 #pragma unroll
@@ -284,8 +369,8 @@ __global__ __launch_bounds__(kDpBlock) void k_dp_kspace(C2 *const *T, C2 *const 
 }
 
 /** AssignTorques / AssignForces (dp3m.cpp:195-244): torque -= mu x (pt E),
- *  force_a += pf sum_b mu_b H_ab with E and H interpolated from the real
- *  parts of the back-transformed meshes, over particles sorted into buckets
+ *  force_a += pf sum_b mu_b H_ab with E and H interpolated from the
+ *  back-transformed meshes, over particles sorted into buckets
  *  of mesh cells.  One block per bucket stages the bucket's E^3 tile of the
  *  three field meshes (and the six force meshes when forces are wanted) in
  *  LDS, tile origin as in the spread; eight lanes per particle (lane a < P
@@ -739,6 +824,14 @@ void dp3m_calculate_accuracy(double box, int mesh, int cao, double r_cut_iL, int
 // ---------------------------------------------------------------------------
 // solver
 // ---------------------------------------------------------------------------
+namespace {
+/** LDS of the line and plane transforms: twiddles and two buffers. */
+size_t line_lds(int M) { return sizeof(C2) * (M + 2 * kDpLines * (static_cast<size_t>(M) + 1)); }
+size_t plane_lds(int M) {
+  return sizeof(C2) * (M + 2 * static_cast<size_t>(M / 2 + 1) * (M + 1));
+}
+} // namespace
+
 struct DipolarSolver::Impl {
   int device = 0;
   hipStream_t st = nullptr;
@@ -748,9 +841,9 @@ struct DipolarSolver::Impl {
   FftPlanDev plan{};
   int M = 0;
   C2 *tw = nullptr, *twi = nullptr;
-  C2 *mesh[9] = {};       // A0..A2 (T0..T2), F0..F5
+  C2 *mesh[9] = {};       // half spectra A0..A2 (T0..T2), F0..F5
   C2 **d_ptrs = nullptr;  // device pointer table: A[3], F[6]
-  double *rmesh[9] = {};  // real parts of the back-transformed meshes
+  double *rmesh[9] = {};  // dipole meshes (0..2), then the back-transformed meshes
   double **d_rptrs = nullptr; // device pointer table of rmesh
   double *Ge = nullptr, *Gf = nullptr;
   double *part = nullptr;
@@ -854,13 +947,14 @@ void DipolarSolver::configure(DipolarParams const &p) {
     dp_free(m->Ge);
     dp_free(m->Gf);
     size_t const M3 = static_cast<size_t>(M) * M * M;
-    for (auto *&x : m->mesh) hip_check(hipMalloc(&x, sizeof(C2) * M3), "hipMalloc dp3m mesh");
+    size_t const H3 = static_cast<size_t>(M) * M * (M / 2 + 1);
+    for (auto *&x : m->mesh) hip_check(hipMalloc(&x, sizeof(C2) * H3), "hipMalloc dp3m mesh");
     for (auto *&x : m->rmesh)
       hip_check(hipMalloc(&x, sizeof(double) * M3), "hipMalloc dp3m real mesh");
     hip_check(hipMemcpy(m->d_rptrs, m->rmesh, sizeof(m->rmesh), hipMemcpyHostToDevice),
               "copy table");
-    hip_check(hipMalloc(&m->Ge, sizeof(double) * M3), "hipMalloc dp3m G");
-    hip_check(hipMalloc(&m->Gf, sizeof(double) * M3), "hipMalloc dp3m G");
+    hip_check(hipMalloc(&m->Ge, sizeof(double) * H3), "hipMalloc dp3m G");
+    hip_check(hipMalloc(&m->Gf, sizeof(double) * H3), "hipMalloc dp3m G");
     hip_check(hipMalloc(&m->tw, sizeof(C2) * M), "hipMalloc dp3m twiddles");
     std::vector<C2> tw(static_cast<size_t>(M));
     for (int k = 0; k < M; ++k) {
@@ -915,8 +1009,16 @@ void DipolarSolver::configure(DipolarParams const &p) {
           if (!std::isfinite(ge[idx])) ge[idx] = 0.;
           if (!std::isfinite(gf[idx])) gf[idx] = 0.;
         }
-    hip_check(hipMemcpy(m->Ge, ge.data(), sizeof(double) * M3, hipMemcpyHostToDevice), "copy G");
-    hip_check(hipMemcpy(m->Gf, gf.data(), sizeof(double) * M3, hipMemcpyHostToDevice), "copy G");
+    // the device keeps kz <= M / 2
+    std::vector<double> he, hf;
+    for (size_t l = 0; l < M3; l += static_cast<size_t>(M)) {
+      he.insert(he.end(), ge.begin() + l, ge.begin() + l + half + 1);
+      hf.insert(hf.end(), gf.begin() + l, gf.begin() + l + half + 1);
+    }
+    hip_check(hipMemcpy(m->Ge, he.data(), sizeof(double) * he.size(), hipMemcpyHostToDevice),
+              "copy G");
+    hip_check(hipMemcpy(m->Gf, hf.data(), sizeof(double) * hf.size(), hipMemcpyHostToDevice),
+              "copy G");
     // self-energy sum of the energy correction (influence_function_dipolar.hpp:160-218)
     double se = 0.;
     idx = 0;
@@ -941,16 +1043,18 @@ void DipolarSolver::configure(DipolarParams const &p) {
         }
     m->self_sum = se;
   }
-  int const lds = static_cast<int>(sizeof(C2) * (M + 2 * kDpLines * (M + 1)));
-  if (lds > 64 * 1024)
-    hip_check(hipFuncSetAttribute(reinterpret_cast<void const *>(k_dp_fft),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds),
-              "hipFuncSetAttribute");
-  size_t const lds_plane = sizeof(C2) * (M + 2 * static_cast<size_t>(M) * (M + 1));
+  // the limit of the kernel holds for every solver of the process: raised to
+  // what any of them takes
+  int const lds = std::max(static_cast<int>(line_lds(M)), kDpGatherLds);
+  if (line_lds(M) > 64 * 1024)
+    for (void const *k : {reinterpret_cast<void const *>(k_dp_fft),
+                          reinterpret_cast<void const *>(k_dp_fft_z)})
+      hip_check(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds),
+                "hipFuncSetAttribute");
+  size_t const lds_plane = plane_lds(M);
   if (lds_plane > 64 * 1024 && lds_plane <= static_cast<size_t>(kDpGatherLds))
-    hip_check(hipFuncSetAttribute(reinterpret_cast<void const *>(k_dp_fft_zy),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  static_cast<int>(lds_plane)),
+    hip_check(hipFuncSetAttribute(reinterpret_cast<void const *>(k_dp_fft_plane),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, kDpGatherLds),
               "hipFuncSetAttribute");
   m->p = p;
   m->configured = true;
@@ -960,7 +1064,7 @@ namespace {
 
 template <int P> void launch_spread(hipStream_t st, int nk, int E, int const *offsets,
                                     int const *counts, double const *pos, double const *dip,
-                                    DevGeo const &g, C2 *const *mesh, int *err) {
+                                    DevGeo const &g, double *const *mesh, int *err) {
   size_t const lds = sizeof(double) * 3 * static_cast<size_t>(E) * E * E;
   k_dp_spread_tile<P><<<nk, kDpBlock, lds, st>>>(offsets, counts, pos, dip, g, E, mesh[0],
                                                  mesh[1], mesh[2], err);
@@ -995,7 +1099,8 @@ void DipolarSolver::solve(int64_t n, double const *pos, double const *dip, doubl
   int const M = m->M;
   int64_t const M3 = static_cast<int64_t>(M) * M * M;
   int const nb = static_cast<int>((n + kDpBlock - 1) / kDpBlock);
-  int const kb = static_cast<int>((M3 + kDpBlock - 1) / kDpBlock);
+  int const kb = static_cast<int>(
+      (static_cast<int64_t>(M) * M * (M / 2 + 1) + kDpBlock - 1) / kDpBlock);
   size_t const need = std::max(static_cast<size_t>(kb), static_cast<size_t>(nb) * 4);
   if (need > m->cap_part) {
     hip_check(hipStreamSynchronize(st), "sync");
@@ -1040,7 +1145,8 @@ void DipolarSolver::solve(int64_t n, double const *pos, double const *dip, doubl
   k_dp_prep<<<dim3(static_cast<unsigned>(std::max<int64_t>(
                        kb, (static_cast<int64_t>(nk) * kDpCopies + kDpBlock - 1) / kDpBlock)),
                    3),
-              kDpBlock, 0, st>>>(m->mesh[0], m->mesh[1], m->mesh[2], M3, m->counts, nk, m->err);
+              kDpBlock, 0, st>>>(m->rmesh[0], m->rmesh[1], m->rmesh[2], M3 / 2, m->counts, nk,
+                                 m->err);
   // bucket keys, and the moments (sum |mu|^2, total dipole) on the device
   k_dp_key<<<nb, kDpBlock, 0, st>>>(n, pos, dip, p.box, nbk, m->counts, m->key, m->rank,
                                     m->part);
@@ -1055,33 +1161,40 @@ void DipolarSolver::solve(int64_t n, double const *pos, double const *dip, doubl
   double const dipole_prefac = p.prefactor / static_cast<double>(M3);
   {
     switch (p.cao) {
-    case 1: launch_spread<1>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->mesh, m->err); break;
-    case 2: launch_spread<2>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->mesh, m->err); break;
-    case 3: launch_spread<3>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->mesh, m->err); break;
-    case 4: launch_spread<4>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->mesh, m->err); break;
-    case 5: launch_spread<5>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->mesh, m->err); break;
-    case 6: launch_spread<6>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->mesh, m->err); break;
-    default: launch_spread<7>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->mesh, m->err); break;
+    case 1: launch_spread<1>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->rmesh, m->err); break;
+    case 2: launch_spread<2>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->rmesh, m->err); break;
+    case 3: launch_spread<3>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->rmesh, m->err); break;
+    case 4: launch_spread<4>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->rmesh, m->err); break;
+    case 5: launch_spread<5>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->rmesh, m->err); break;
+    case 6: launch_spread<6>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->rmesh, m->err); break;
+    default: launch_spread<7>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->rmesh, m->err); break;
     }
-    size_t const lds = sizeof(C2) * (M + 2 * kDpLines * (M + 1));
-    int const lines = static_cast<int>((static_cast<int64_t>(M) * M + kDpLines - 1) / kDpLines);
-    size_t const lds_plane = sizeof(C2) * (M + 2 * static_cast<size_t>(M) * (M + 1));
+    auto const blocks = [](int64_t lines) {
+      return static_cast<unsigned>((lines + kDpLines - 1) / kDpLines);
+    };
+    size_t const lds = line_lds(M), lds_plane = plane_lds(M);
+    unsigned const lines = blocks(static_cast<int64_t>(M) * (M / 2 + 1));
     bool const plane = lds_plane <= static_cast<size_t>(kDpGatherLds);
-    // rout: real meshes for the real parts of the last (x) pass, or null
-    auto fft = [&](C2 *const *table, int nmesh, bool inv, double *const *rout) {
+    // real meshes <-> half spectra of nmesh meshes
+    auto fft = [&](int nmesh, bool inv) {
+      auto along = [&](int axis) {
+        k_dp_fft<<<dim3(lines, nmesh), kDpBlock, lds, st>>>(m->d_ptrs, M, axis, m->plan, m->tw,
+                                                            inv);
+      };
+      if (inv) along(0);
       if (plane) {
-        k_dp_fft_zy<<<dim3(M, nmesh), kDpPlaneBlock, lds_plane, st>>>(table, M, m->plan, m->tw,
-                                                                       inv);
-        k_dp_fft<<<dim3(lines, nmesh), kDpBlock, lds, st>>>(table, M, 0, m->plan, m->tw, inv,
-                                                            rout);
+        k_dp_fft_plane<<<dim3(M, nmesh), lds_plane <= 80 * 1024 ? 512 : kDpPlaneBlock, lds_plane,
+                         st>>>(m->d_rptrs, m->d_ptrs, M, m->plan, m->tw, inv);
       } else {
-        for (int axis = 2; axis >= 0; --axis)
-          k_dp_fft<<<dim3(lines, nmesh), kDpBlock, lds, st>>>(table, M, axis, m->plan, m->tw,
-                                                              inv, axis == 0 ? rout : nullptr);
+        if (inv) along(1);
+        k_dp_fft_z<<<dim3(blocks(static_cast<int64_t>(M) * M / 2), nmesh), kDpBlock, lds, st>>>(
+            m->d_rptrs, m->d_ptrs, M, m->plan, m->tw, inv);
+        if (!inv) along(1);
       }
+      if (!inv) along(0);
     };
     // device table: [0..2] A (field meshes after the k-space step), [3..8] F
-    fft(m->d_ptrs, 3, false, nullptr);
+    fft(3, false);
     bool const wf = force != nullptr, wt = torque != nullptr;
     k_dp_kspace<<<kb, kDpBlock, 0, st>>>(m->d_ptrs, m->d_ptrs + 3, m->Ge, m->Gf, M,
                                          (wf || wt) ? 1 : 0, wf ? 1 : 0, m->part);
@@ -1097,7 +1210,7 @@ void DipolarSolver::solve(int64_t n, double const *pos, double const *dip, doubl
     if (wf || wt) {
       // the field meshes [0..2] and force meshes [3..8] are consecutive in
       // the table: one launch per axis transforms all of them
-      fft(m->d_ptrs, wf ? 9 : 3, true, m->d_rptrs);
+      fft(wf ? 9 : 3, true);
       double const pt = dipole_prefac * wn, pf = dipole_prefac * wn * wn;
       switch (p.cao) {
       case 1: launch_gather<1>(st, nk, E, m->offsets, m->total, sp, sd, m->g, m->d_rptrs, pt, pf, perm, force, torque); break;
