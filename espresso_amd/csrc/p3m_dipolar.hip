@@ -376,8 +376,13 @@ __global__ __launch_bounds__(kDpBlock) void k_dp_kspace(C2 *const *T, C2 *const 
  *  LDS, tile origin as in the spread; eight lanes per particle (lane a < P
  *  sums the stencil points with z offset a), combined by lane shuffles.  A
  *  particle whose stencil leaves the tile reads the meshes directly.
- *  Results go to the caller's row perm[i]. */
-template <int P>
+ *  Results go to the caller's row perm[i].
+ *  One block fills the LDS of a CU, two waves per SIMD, so loads must be in
+ *  flight together.  Staging takes 16 lanes per row without divisions, four
+ *  rows at a time; the stencil loops are unrolled up to cao 5 (10^5 dipoles,
+ *  mesh 64, cao 5: 103 us, with a loop over x planes 133 us, before both 122),
+ *  above that unrolled planes in a loop, as all of it would spill. */
+template <int P, bool WF>
 __global__ __launch_bounds__(kDpGatherBlock) void k_dp_gather_tile(
     int const *__restrict__ offsets, int const *__restrict__ counts,
     double const *__restrict__ pos, double const *__restrict__ dip, DevGeo g, int E,
@@ -387,8 +392,7 @@ __global__ __launch_bounds__(kDpGatherBlock) void k_dp_gather_tile(
   __shared__ int org[3];
   int const beg = offsets[blockIdx.x], cnt = counts[blockIdx.x];
   if (cnt == 0) return;
-  bool const wf = force != nullptr;
-  int const nm = wf ? 9 : 3;
+  constexpr int NM = WF ? 9 : 3;
   int const M = g.M[0];
   int const E3 = E * E * E;
   if (threadIdx.x < 3) org[threadIdx.x] = INT_MAX;
@@ -420,19 +424,31 @@ __global__ __launch_bounds__(kDpGatherBlock) void k_dp_gather_tile(
                     org[2] == INT_MAX ? 0 : org[2]};
   int const b0 = ((gref[0] + o[0]) % M + M) % M, b1 = ((gref[1] + o[1]) % M + M) % M,
             b2 = ((gref[2] + o[2]) % M + M) % M;
-  for (int e = threadIdx.x; e < nm * E3; e += kDpGatherBlock) {
-    int const c = e / E3, q = e - c * E3;
-    int const tz = q % E, ty = (q / E) % E, tx = q / (E * E);
-    int64_t const idx =
-        ((int64_t)((b0 + tx) % M) * M + (b1 + ty) % M) * M + (b2 + tz) % M;
-    tile[e] = R[c][idx];
-  }
+  // 16 lanes per row along z (E <= 16), four rows in flight
+  FastDiv const fE = make_fastdiv(E);
+  int const tz = threadIdx.x & 15, rows = NM * E * E;
+  int const iz = periodic_index(b2 + tz, M);
+  auto row = [&](int r) { // first mesh element
+    int const q = fdiv(r, fE), c = fdiv(q, fE);
+    return R[c] + ((int64_t)periodic_index(b0 + q - c * E, M) * M +
+                   periodic_index(b1 + r - q * E, M)) * M;
+  };
+  if (tz < E)
+    for (int r0 = threadIdx.x >> 4; r0 < rows; r0 += 4 * (kDpGatherBlock / 16)) {
+      double v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = row(min(r0 + u * (kDpGatherBlock / 16), rows - 1))[iz];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (r0 + u * (kDpGatherBlock / 16) < rows)
+          tile[(r0 + u * (kDpGatherBlock / 16)) * E + tz] = v[u];
+    }
   __syncthreads();
   int const a = static_cast<int>(threadIdx.x & 7);
   // the eight lanes of a particle share j and run the loop together
   for (int j = threadIdx.x >> 3; j < cnt; j += kDpGatherBlock / 8) {
     int64_t const i = beg + j;
-    double v[9] = {0., 0., 0., 0., 0., 0., 0., 0., 0.}; // E[3], H[6]
+    double v[NM] = {}; // E[3], H[6]
     double const mu[3] = {dip[3 * i], dip[3 * i + 1], dip[3 * i + 2]};
     bool const act = (mu[0] != 0. || mu[1] != 0. || mu[2] != 0.);
     if (act && a < P) {
@@ -443,37 +459,53 @@ __global__ __launch_bounds__(kDpGatherBlock) void k_dp_gather_tile(
         int r[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) r[d] = rel(gi[d], gref[d]) - o[d];
-        double const wz = w[2][a];
+        double wx = w[0][0], wz = w[2][0]; // of stencil plane and column a
+#pragma unroll
+        for (int k = 1; k < P; ++k) {
+          wx = (a == k) ? w[0][k] : wx;
+          wz = (a == k) ? w[2][k] : wz;
+        }
         if (r[0] + P <= E && r[1] + P <= E && r[2] + P <= E) {
-          for (int rr = 0; rr < P; ++rr)
-            for (int b = 0; b < P; ++b) {
-              int const t = ((r[0] + rr) * E + r[1] + b) * E + r[2] + a;
-              double const wt = w[0][rr] * w[1][b] * wz;
+          double const *tp = tile + (r[0] * E + r[1]) * E + r[2] + a;
+          if constexpr (P <= 5) {
 #pragma unroll
-              for (int d = 0; d < 3; ++d) v[d] += wt * tile[d * E3 + t];
-              if (wf)
+            for (int rr = 0; rr < P; ++rr) {
 #pragma unroll
-                for (int d = 0; d < 6; ++d) v[3 + d] += wt * tile[(3 + d) * E3 + t];
+              for (int b = 0; b < P; ++b) {
+                double const wt = w[0][rr] * w[1][b] * wz;
+#pragma unroll
+                for (int d = 0; d < NM; ++d) v[d] += wt * tp[d * E3 + (rr * E + b) * E];
+              }
             }
+          } else {
+#pragma unroll 1
+            for (int rr = 0; rr < P; ++rr, tp += E * E) {
+              double const wr = __shfl(wx, rr, 8);
+#pragma unroll
+              for (int b = 0; b < P; ++b) {
+                double const wt = wr * w[1][b] * wz;
+#pragma unroll
+                for (int d = 0; d < NM; ++d) v[d] += wt * tp[d * E3 + b * E];
+              }
+            }
+          }
         } else {
           int const iz = wrap_once(gi[2] + a, M);
           for (int rr = 0; rr < P; ++rr) {
+            double const wr = __shfl(wx, rr, 8);
             int const ix = wrap_once(gi[0] + rr, M);
             for (int b = 0; b < P; ++b) {
               int64_t const idx = ((int64_t)ix * M + wrap_once(gi[1] + b, M)) * M + iz;
-              double const wt = w[0][rr] * w[1][b] * wz;
+              double const wt = wr * w[1][b] * wz;
 #pragma unroll
-              for (int d = 0; d < 3; ++d) v[d] += wt * R[d][idx];
-              if (wf)
-#pragma unroll
-                for (int d = 0; d < 6; ++d) v[3 + d] += wt * R[3 + d][idx];
+              for (int d = 0; d < NM; ++d) v[d] += wt * R[d][idx];
             }
           }
         }
       }
     }
 #pragma unroll
-    for (int k = 0; k < 9; ++k) {
+    for (int k = 0; k < NM; ++k) {
       v[k] += __shfl_xor(v[k], 1, 64);
       v[k] += __shfl_xor(v[k], 2, 64);
       v[k] += __shfl_xor(v[k], 4, 64);
@@ -486,7 +518,7 @@ __global__ __launch_bounds__(kDpGatherBlock) void k_dp_gather_tile(
       torque[ro + 1] -= mu[2] * e0 - mu[0] * e2;
       torque[ro + 2] -= mu[0] * e1 - mu[1] * e0;
     }
-    if (wf) {
+    if constexpr (WF) {
       double const *H = v + 3; // xx xy xz yy yz zz
       force[ro] += pf * (mu[0] * H[0] + mu[1] * H[1] + mu[2] * H[2]);
       force[ro + 1] += pf * (mu[0] * H[1] + mu[1] * H[3] + mu[2] * H[4]);
@@ -1069,22 +1101,30 @@ template <int P> void launch_spread(hipStream_t st, int nk, int E, int const *of
   k_dp_spread_tile<P><<<nk, kDpBlock, lds, st>>>(offsets, counts, pos, dip, g, E, mesh[0],
                                                  mesh[1], mesh[2], err);
 }
-template <int P> void launch_gather(hipStream_t st, int nk, int E, int const *offsets,
-                                    int const *counts, double const *pos, double const *dip,
-                                    DevGeo const &g, double const *const *R, double pt,
-                                    double pf, int const *perm, double *force, double *torque) {
+template <int P, bool WF>
+void launch_gather_of(hipStream_t st, int nk, int E, int const *offsets, int const *counts,
+                      double const *pos, double const *dip, DevGeo const &g,
+                      double const *const *R, double pt, double pf, int const *perm,
+                      double *force, double *torque) {
   static bool const raised = [] {
-    hip_check(hipFuncSetAttribute(reinterpret_cast<void const *>(k_dp_gather_tile<P>),
+    hip_check(hipFuncSetAttribute(reinterpret_cast<void const *>(k_dp_gather_tile<P, WF>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, kDpGatherLds),
               "hipFuncSetAttribute");
     return true;
   }();
   (void)raised;
-  size_t const lds = sizeof(double) * (force ? 9 : 3) * static_cast<size_t>(E) * E * E;
+  size_t const lds = sizeof(double) * (WF ? 9 : 3) * static_cast<size_t>(E) * E * E;
   if (lds > static_cast<size_t>(kDpGatherLds))
     throw std::runtime_error("DipolarP3M: gather tile exceeds the LDS of a workgroup");
-  k_dp_gather_tile<P><<<nk, kDpGatherBlock, lds, st>>>(offsets, counts, pos, dip, g, E, R,
-                                                       pt, pf, perm, force, torque);
+  k_dp_gather_tile<P, WF><<<nk, kDpGatherBlock, lds, st>>>(offsets, counts, pos, dip, g, E, R,
+                                                           pt, pf, perm, force, torque);
+}
+template <int P> void launch_gather(hipStream_t st, int nk, int E, int const *offsets,
+                                    int const *counts, double const *pos, double const *dip,
+                                    DevGeo const &g, double const *const *R, double pt,
+                                    double pf, int const *perm, double *force, double *torque) {
+  auto const f = force ? launch_gather_of<P, true> : launch_gather_of<P, false>;
+  f(st, nk, E, offsets, counts, pos, dip, g, R, pt, pf, perm, force, torque);
 }
 } // namespace
 
