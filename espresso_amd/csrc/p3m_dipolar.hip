@@ -20,6 +20,7 @@ using C2 = double2;
 constexpr int kDpBlock = 256;
 constexpr int kDpLines = 8; // FFT lines per block
 constexpr int kDpGatherBlock = 512;
+constexpr int kDpTile = 13; // most points per edge of a tile: nine fill the LDS of a CU
 // most threads of the z/y plane transform: 512 when two blocks share the LDS
 // of a CU, else all
 constexpr int kDpPlaneBlock = 1024;
@@ -1148,15 +1149,20 @@ void DipolarSolver::solve(int64_t n, double const *pos, double const *dip, doubl
     hip_check(hipMalloc(&m->part, sizeof(double) * need), "hipMalloc dp3m partials");
     m->cap_part = need;
   }
-  // particles sorted into buckets of S^3 mesh cells for the spread and
-  // gather; the spread's LDS tile of E = ceil(M / nbk) + cao points per edge
-  // and component stays within 64 KiB
-  int nbk = 1, E = 0;
-  for (int S : {8, 4, 2, 1}) {
-    nbk = std::max(1, M / S);
-    E = (M + nbk - 1) / nbk + p.cao;
-    if (3 * E * E * E * static_cast<int>(sizeof(double)) <= 65536) break;
+  // particles sorted into nbk^3 buckets for the spread and gather, whose LDS
+  // tiles have E points per edge: as wide as they fit (a narrow bucket stages
+  // and flushes mostly stencil margin), up to 8 cells, but narrower until there
+  // are 500 of them, two blocks per CU, or ten particles in each.  10^5 dipoles
+  // at mesh 64, cao 6: 0.47 ms in 1000 buckets of up to 7 cells, 0.74 in 4096
+  // of 4; 10^4 at mesh 24, cao 5: 160 us in 512 buckets of 3 cells, 242 in 27
+  // of 8; 2000 at mesh 24, cao 7: 165 us in 216, 188 in 512
+  int64_t const enough = std::min<int64_t>(500, n / 10);
+  int width = std::min(8, kDpTile - p.cao), nbk = 1;
+  for (;; --width) {
+    nbk = (M + width - 1) / width;
+    if (width == 2 || static_cast<int64_t>(nbk) * nbk * nbk >= enough) break;
   }
+  int const E = (M + nbk - 1) / nbk + p.cao;
   int const nk = nbk * nbk * nbk;
   if (n > m->cap_sort || nk > m->cap_keys) {
     hip_check(hipStreamSynchronize(st), "sync");

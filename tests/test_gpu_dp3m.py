@@ -146,6 +146,35 @@ def test_short_range_dense_cluster_matches_oracle(subdiv, r_cut):
     assert abs(e - er) <= 1e-12 * abs(er)
 
 
+@pytest.mark.parametrize("mesh,cao,n", [
+    (2, 1, 3), (8, 7, 40), (14, 6, 900),  # tiles that wrap around the mesh
+    (24, 5, 1), (24, 5, 6000),            # buckets of 8 and of 3 cells
+    (50, 6, 6000),                        # buckets that do not divide the mesh
+    (96, 3, 500), (98, 3, 500),           # last mesh transformed by planes, first by lines
+])
+def test_kspace_transform_and_bucket_edges_match_oracle(mesh, cao, n):
+    """Half-spectrum transforms and particle buckets at the edges of their
+    rules; forces and torques, then each alone, and the energy.  Tolerance of
+    the k-space tests (FP64 rounding of the FFTs and sums)."""
+    from espresso_amd.magnetostatics import DipolarP3M
+    from oracle import dp3m as D
+    L = 10.
+    pos, dip = _system(n, L, n + mesh)
+    dp = DipolarP3M(prefactor=1.3, accuracy=1e-4, mesh=mesh, cao=cao, alpha=0.6, r_cut=3.,
+                    tune=False)
+    dp.activate(pos, dip, box_l=L)
+    f, t, f1, t1 = (np.zeros((n, 3)) for _ in range(4))
+    dp.add_long_range_forces(pos, dip, f, t)
+    e = dp.long_range_energy(pos, dip)
+    dp.add_long_range_forces(pos, dip, None, t1)
+    dp.add_long_range_forces(pos, dip, f1, None)
+    fr, tr, er = D.OracleDP3M(L, mesh, cao, 0.6, 3., 1.3).solve(pos - L * np.floor(pos / L), dip)
+    for got, ref in ((f, fr), (t, tr), (f1, fr), (t1, tr)):
+        scale = max(np.sqrt(np.mean(ref ** 2)), 1e-6)
+        assert np.sqrt(np.mean((got - ref) ** 2)) <= 1e-10 * scale
+    assert abs(e - er) <= 1e-10 * max(abs(er), 1e-6)
+
+
 @pytest.mark.parametrize("accuracy", [1e-4, 1e-7])
 @pytest.mark.parametrize("L,r_cut,n,spread", [
     (9., 2.2, 1, 1.),            # no pair at all
