@@ -768,23 +768,22 @@ struct ShortRange::Impl {
   size_t cap_mu2 = 0, cap_sdip = 0;
   int *counts = nullptr, *offsets = nullptr, *p_cell = nullptr, *p_rank = nullptr,
       *sidx = nullptr;
-  int *goff = nullptr;
+  double *shares = nullptr; // and, in the same allocation:
   int2 *grp = nullptr;
-  int *arrived = nullptr;
-  double *shares = nullptr;
-  size_t cap_goff = 0, cap_grp = 0, cap_arrived = 0, cap_shares = 0;
+  int *goff = nullptr, *arrived = nullptr;
+  size_t cap_shares = 0;
   double4 *spos = nullptr;
   double *partials = nullptr;
   size_t cap_cells = 0, cap_off = 0, cap_pc = 0, cap_pr = 0, cap_si = 0, cap_sp = 0, cap_part = 0;
 
-  /** Buffers of the column search (nv sums per particle). */
+  /** Buffers of the column search (nv sums per particle), one allocation. */
   void grow_columns(Columns const &c, int nv) {
-    sr_grow(goff, cap_goff, static_cast<size_t>(c.ncol) + 1, "hipMalloc group offsets");
-    sr_grow(grp, cap_grp, static_cast<size_t>(c.max_groups), "hipMalloc groups");
-    sr_grow(arrived, cap_arrived, static_cast<size_t>(c.max_groups), "hipMalloc groups");
-    if (c.split > 1)
-      sr_grow(shares, cap_shares, static_cast<size_t>(c.max_groups) * c.split * 64 * nv,
-              "hipMalloc group shares");
+    size_t const groups = static_cast<size_t>(c.max_groups), ints = c.ncol + 1 + groups;
+    size_t const sums = (c.split > 1) ? groups * c.split * 64 * nv : 0;
+    sr_grow(shares, cap_shares, sums + groups + (ints + 1) / 2, "hipMalloc home groups");
+    grp = reinterpret_cast<int2 *>(shares + sums);
+    goff = reinterpret_cast<int *>(grp + groups);
+    arrived = goff + c.ncol + 1;
   }
 };
 
@@ -796,9 +795,7 @@ ShortRange::~ShortRange() {
                   static_cast<void *>(m->p_cell), static_cast<void *>(m->p_rank),
                   static_cast<void *>(m->sidx), static_cast<void *>(m->spos),
                   static_cast<void *>(m->partials), static_cast<void *>(m->mu2),
-                  static_cast<void *>(m->sdip), static_cast<void *>(m->goff),
-                  static_cast<void *>(m->grp), static_cast<void *>(m->arrived),
-                  static_cast<void *>(m->shares)})
+                  static_cast<void *>(m->sdip), static_cast<void *>(m->shares)})
     if (p) (void)hipFree(p);
   delete m;
 }
