@@ -2408,7 +2408,7 @@ struct Plan {
   int blocks_part = 0;
   int *d_small = nullptr; // systems binned by bin_system
   int nsmall = 0;
-  bool wide = false; // fused pass with a block per column and component
+  size_t field_bytes = 0; // y field of the wide fused pass, 0: not for this selection
   int blocks_bin = 0, blocks_fill = 0, blocks_z = 0, blocks_zc = 0, blocks_y = 0, blocks_x = 0,
       blocks_yi = 0, blocks_f = 0;
   int *soff = nullptr; // per system id: first particle of the system in the lane scratch
@@ -2447,8 +2447,10 @@ struct Lane {
   double4 *spos = nullptr;
   void *own = nullptr;
   size_t own_bytes = 0;
-  void *ybuf = nullptr; // y field of the wide fused pass
-  size_t ybuf_bytes = 0;
+  // y field of the wide fused pass of the current solve: null (one block per
+  // column), the lane's own, or after the particle scratch passed in
+  void *ybuf = nullptr, *own_ybuf = nullptr;
+  size_t own_ybuf_bytes = 0;
   double *bin_part = nullptr, *conv_part = nullptr;
   int bin_cap = 0, conv_cap = 0;
   double *sums = nullptr;
@@ -2517,8 +2519,8 @@ void destroy_lane(Lane &ln) {
   dfree(ln.offsets);
   if (ln.own) (void)hipFree(ln.own);
   ln.own = nullptr;
-  if (ln.ybuf) (void)hipFree(ln.ybuf);
-  ln.ybuf = nullptr;
+  if (ln.own_ybuf) (void)hipFree(ln.own_ybuf);
+  ln.own_ybuf = nullptr;
   dfree(ln.bin_part);
   dfree(ln.conv_part);
   dfree(ln.sums);
@@ -2605,6 +2607,21 @@ size_t scratch_bytes(int64_t n) {
   size_t const u = static_cast<size_t>(std::max<int64_t>(n, 1));
   return align256(u * sizeof(double4)) + 3 * align256(u * sizeof(int));
 }
+size_t mesh_complex_bytes(MeshPrecision prec) { return prec == MeshPrecision::FP64 ? 16 : 8; }
+/** Elements of the y field of k_fft_yx_conv_wide over the kz columns of `sel`,
+ *  0 where it has none or too many of them for that kernel. */
+size_t wide_elements(BatchSolver::Impl const *m, std::vector<int> const &sel) {
+  int columns = 0;
+  size_t elements = 0;
+  for (int s : sel) {
+    SysDesc const &d = m->sys.at(s).desc;
+    if (!d.kzmajor) continue;
+    columns += d.g.Kz;
+    if (columns > kWideColumns) return 0;
+    elements += static_cast<size_t>(d.g.Kz) * d.g.M[0] * d.g.M[1];
+  }
+  return elements;
+}
 void carve(Lane &ln, void *base, int64_t n) {
   size_t const u = static_cast<size_t>(std::max<int64_t>(n, 1));
   char *p = static_cast<char *>(base);
@@ -2622,6 +2639,10 @@ size_t BatchSolver::working_bytes(std::vector<int> const &sel) const {
   int64_t n = 0;
   for (int s : sel) n += m->sys.at(s).n;
   return scratch_bytes(n);
+}
+
+size_t BatchSolver::field_bytes(std::vector<int> const &sel) const {
+  return align256(wide_elements(m, sel) * mesh_complex_bytes(m_prec));
 }
 
 namespace {
@@ -3067,21 +3088,29 @@ void upload_descs(BatchSolver::Impl *m, hipStream_t st) {
   m->descs_dirty = false;
 }
 
-/** Particle scratch for `npart` particles of a selection, brick counters of
- *  all systems, per-system sums; grows only, after draining the lane. */
+/** Particle scratch for `npart` particles of a selection, the y field of the
+ *  wide fused pass, brick counters of all systems, per-system sums; grows
+ *  only, after draining the lane.  An external block holds the particle
+ *  scratch and, where it is large enough, the y field after it (without that
+ *  the fused pass runs one block per column: the same bits). */
 void ensure_scratch(BatchSolver::Impl *m, Lane &ln, int64_t npart, void *external,
                     size_t external_bytes) {
   int nb_need = 0;
   for (auto const &h : m->sys) nb_need += h.nbricks;
   int const nsys = static_cast<int>(m->sys.size());
   size_t const need = scratch_bytes(npart);
+  size_t const field = ln.plan.field_bytes;
   bool const grow_own = !external && need > ln.own_bytes;
-  bool const grow = grow_own || nb_need > ln.counts_cap || nb_need + nsys > ln.offsets_cap ||
+  bool const grow_field = !external && field > ln.own_ybuf_bytes;
+  bool const grow = grow_own || grow_field || nb_need > ln.counts_cap || nb_need + nsys > ln.offsets_cap ||
                     nsys * 16 > ln.sums_cap;
   if (grow) hip_check(hipStreamSynchronize(ln.stream), "sync before realloc"); // queued work
   if (external) {
     if (external_bytes < need) throw std::invalid_argument("P3M: scratch block too small");
     carve(ln, external, npart);
+    ln.ybuf = (field > 0 && external_bytes >= need + field)
+                  ? static_cast<char *>(external) + need
+                  : nullptr;
   } else {
     if (grow_own) {
       if (ln.own) (void)hipFree(ln.own);
@@ -3092,6 +3121,18 @@ void ensure_scratch(BatchSolver::Impl *m, Lane &ln, int64_t npart, void *externa
       ln.own_bytes = cap;
     }
     carve(ln, ln.own, npart);
+    if (grow_field) {
+      // at least twice the last size: a free waits for the whole device, and
+      // selections that vary must not pay for one each (at most 8 MB: 128
+      // planes of 64 KB)
+      size_t const cap = std::max(field, 2 * ln.own_ybuf_bytes);
+      if (ln.own_ybuf) (void)hipFree(ln.own_ybuf);
+      ln.own_ybuf = nullptr;
+      ln.own_ybuf_bytes = 0;
+      hip_check(hipMalloc(&ln.own_ybuf, cap), "hipMalloc y field");
+      ln.own_ybuf_bytes = cap;
+    }
+    ln.ybuf = field > 0 ? ln.own_ybuf : nullptr;
   }
   if (nb_need > ln.counts_cap) {
     dfree(ln.counts);
@@ -3164,7 +3205,7 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
   free_plan(p);
   p.sel = sel;
   p.nsel = static_cast<int>(sel.size());
-  size_t const csz = (prec == MeshPrecision::FP64) ? 16 : 8;
+  size_t const csz = mesh_complex_bytes(prec);
   // split y/x passes: sizes over the systems that use them; z passes: all
   int max_mx = 1, max_my = 1, max_mz = 1;
   for (int s : sel) {
@@ -3260,13 +3301,13 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
     return h.desc.kzmajor ? 0 : ((h.desc.g.Kz + ncyi - 1) / ncyi) * h.desc.g.M[0];
   });
   auto const ff = push_prefix([](HostSys const &h) { return h.desc.kzmajor ? h.desc.g.Kz : 0; });
-  // y field of the wide fused pass (not in the fixed scratch): at most
-  // kWideColumns planes
-  p.wide = !ln.fixed && ff.second > 0 && ff.second <= kWideColumns;
-  auto const yc = push_prefix([&p](HostSys const &h) {
+  // y field of the wide fused pass (not in the fixed scratch)
+  bool const wide = !ln.fixed && wide_elements(m, sel) > 0;
+  auto const yc = push_prefix([wide](HostSys const &h) {
     DevGeo const &g = h.desc.g;
-    return p.wide && h.desc.kzmajor ? g.Kz * g.M[0] * g.M[1] : 0;
+    return wide && h.desc.kzmajor ? g.Kz * g.M[0] * g.M[1] : 0;
   });
+  p.field_bytes = align256(static_cast<size_t>(yc.second) * csz);
   struct GH {
     int cao, sel_start, nsel, wt_start, blocks, wsp_start, blocks_sp, nshare;
   };
@@ -3378,14 +3419,6 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
               "hipMalloc bin partials");
     ln.bin_cap = p.blocks_bin;
   }
-  size_t const ybytes = static_cast<size_t>(yc.second) * csz;
-  if (ybytes > ln.ybuf_bytes) {
-    if (ln.ybuf) (void)hipFree(ln.ybuf); // the stream is idle (synchronised above)
-    ln.ybuf = nullptr;
-    ln.ybuf_bytes = 0;
-    hip_check(hipMalloc(&ln.ybuf, ybytes), "hipMalloc y field");
-    ln.ybuf_bytes = ybytes;
-  }
   int const conv_blocks = p.blocks_x + p.blocks_f; // split partials, then fused
   if (conv_blocks > ln.conv_cap) {
     dfree(ln.conv_part);
@@ -3405,7 +3438,7 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
   bool const want_sums = (flags & 6u) != 0; // energy or virial (P3M_ENERGY | P3M_PRESSURE)
   int const ns = p.nsel;
   C const *tw = static_cast<C const *>(m->d_tw);
-  C *const ybuf = p.wide ? static_cast<C *>(ln.ybuf) : nullptr;
+  C *const ybuf = static_cast<C *>(ln.ybuf); // null: one block per column
   SysDesc const *sys = m->d_sys;
   // the stage's start time, from its first launch
   unsigned stamped = 0;
@@ -3500,7 +3533,7 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
   if (p.blocks_f > 0) {
     double *fpart = ln.conv_part + 8 * static_cast<size_t>(p.blocks_x);
     unsigned long long *const f_stamp = p.blocks_x > 0 ? nullptr : ln.stamps + 3;
-    if (p.wide)
+    if (ybuf)
       k_fft_yx_conv_wide<MT><<<p.blocks_f * (want_force ? 3 : 1), kWideBlock, p.lds_f, st>>>(
           sys, p.d_sel, p.wt_f, ns, tw, want_force ? 1 : 0, want_sums ? 1 : 0, fpart, ybuf,
           p.ycol, f_stamp);

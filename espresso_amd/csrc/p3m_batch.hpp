@@ -138,15 +138,17 @@ public:
   int add_lane();
   int num_lanes() const;
   hipStream_t lane_stream(int lane) const;
-  /** Enqueue a solve of `sel` on `lane` (no system of `sel` may be in another
-   *  lane's unfinished solve).  With `scratch`, the particle scratch of the
-   *  solve is taken from that device block of scratch_size >=
-   *  working_bytes(sel) bytes (it must stay untouched until the solve ends)
-   *  instead of the lane's own memory. */
   /** Energy and virial of system s from the last solve on the lane,
    *  computed on the device into d_energy (1 double) and d_virial (9),
    *  either may be null, in stream order. */
   void device_results(int lane, int s, double *d_energy, double *d_virial);
+  /** Enqueue a solve of `sel` on `lane` (no system of `sel` may be in another
+   *  lane's unfinished solve).  With `scratch`, the particle scratch of the
+   *  solve is taken from that device block of scratch_size >=
+   *  working_bytes(sel) bytes (it must stay untouched until the solve ends)
+   *  instead of the lane's own memory, and so is the field of a small
+   *  selection where scratch_size leaves field_bytes(sel) more; without that
+   *  room the solve takes longer and gives the same forces. */
   void solve_on(int lane, std::vector<int> const &sel, ParticleArrays const &pa, unsigned flags,
                 bool sync, std::vector<SolveResult> *out, void *scratch = nullptr,
                 size_t scratch_size = 0);
@@ -158,6 +160,9 @@ public:
   /** Device working memory a solve of `sel` needs beyond the resident
    *  systems (particle scratch). */
   size_t working_bytes(std::vector<int> const &sel) const;
+  /** Field that a solve of a small selection (few kz columns) uses on top of
+   *  working_bytes(sel), at most 8 MB; 0 for other selections. */
+  size_t field_bytes(std::vector<int> const &sel) const;
 
   /** Set-up of allocation-free solves (solve_fixed): looks up this device's
    *  copy of the library's fixed scratch array, uploads the descriptors and

@@ -170,7 +170,15 @@ ServeStats Server::run(std::vector<ServeRequest> const &reqs, double *pos, doubl
         for (int s : f.sel) in_batch[s] = 0;
         size_t offset = SIZE_MAX;
         size_t bytes = 0;
-        while (!f.sel.empty()) {
+        if (!f.sel.empty()) {
+          // the field of a small batch, while that leaves half the arena to
+          // later batches: nothing waits for room that only speeds a batch up
+          size_t const field = m_batch.field_bytes(f.sel);
+          bytes = m_batch.working_bytes(f.sel) + field;
+          if (field > 0 && bytes + m_cfg.budget_bytes / 2 <= free_total)
+            offset = arena.allocate(bytes);
+        }
+        while (offset == SIZE_MAX && !f.sel.empty()) {
           bytes = m_batch.working_bytes(f.sel);
           offset = arena.allocate(bytes);
           if (offset != SIZE_MAX) break;

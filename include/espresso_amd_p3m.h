@@ -473,7 +473,8 @@ int p3m_batch_add_system(p3m_batch *b, const p3m_params *p, int64_t n, int *sys_
 int p3m_batch_particle_offset(const p3m_batch *b, int sys_id, int64_t *offset);
 int p3m_batch_system_bytes(const p3m_batch *b, int sys_id, int64_t *bytes);
 /* Device working memory (particle scratch) of a solve of the selection,
- * beyond the resident systems. */
+ * beyond the resident systems.  Selections of few systems use a field of up
+ * to 8 MB more where there is room for it. */
 int p3m_batch_working_bytes(const p3m_batch *b, int nsel, const int *sys_ids, int64_t *bytes);
 /* Solve the selected systems: flags P3M_FORCES / P3M_ENERGY / P3M_PRESSURE,
  * P3M_ASYNC (enqueue only).  energy[nsel] and virial[9*nsel] may be NULL. */
@@ -512,7 +513,8 @@ const char *p3m_batch_last_error(const p3m_batch *b);
  * counterpart in the reference.  Requests (arrival time, system, seed) are
  * admitted into batches as lanes (streams) and working memory free up; the
  * particle scratch of every batch in flight comes from one device arena of
- * budget_bytes.  Per request the system's positions get a Gaussian
+ * budget_bytes, and so does the field of a batch of few systems while half of
+ * the arena stays free.  Per request the system's positions get a Gaussian
  * displacement of width sigma (counter-based draws keyed by the seed, folded
  * into the box), its forces are cleared and recomputed.  A server keeps the
  * batch's solver alive: the batch handle may be destroyed before it.

@@ -134,3 +134,46 @@ def test_admission_by_working_memory():
     small = _server(b, lanes=1, budget_bytes=4096, max_batch=8, sigma=0.)
     with pytest.raises(ValueError, match="exceeds the budget"):
         small.run([0.], [ids[3]], [1], pos, q, force)
+
+
+@pytest.mark.parametrize("single", [False, True])
+def test_field_of_small_batches_comes_from_the_arena(single):
+    """A batch of few kz columns keeps one field component beside its
+    particle scratch.  With half the arena to spare the field is part of the
+    batch's working memory, for two batches at once too; in an arena for the
+    particle scratch alone the batch runs without it.  The arithmetic is the
+    same: FP64 forces equal bit for bit, FP32 ones to the rounding of the
+    spread."""
+    import torch
+    from espresso_amd import P3MBatch
+    n, L, meshes = 700, 8., [(32, 30, 28), (24, 40, 36)]
+    b = P3MBatch(single_precision=single)
+    for mesh in meshes:
+        b.add_system([L] * 3, n, 1.3, mesh, 5, 0.9, 2.)
+    rng = np.random.default_rng(61)
+    pos = torch.tensor(rng.uniform(0., L, (2 * n, 3)), device="cuda")
+    q = torch.tensor(np.where(np.arange(2 * n) % 2 == 0, 1., -1.), device="cuda")
+    ref = torch.zeros_like(pos)
+    for k in (0, 1):
+        b.solve(pos, q, ref, systems=[k])
+    scratch = [b.working_bytes_of(k) for k in (0, 1)]
+    field = [-(-(x * y * (z // 2 + 1) * (8 if single else 16)) // 256) * 256 for x, y, z in meshes]
+
+    def served(ids, budget):
+        srv = _server(b, lanes=2, budget_bytes=budget, max_batch=1, sigma=0.)
+        f = torch.zeros_like(pos)
+        res = srv.run([0.] * len(ids), ids, [1] * len(ids), pos, q, f)
+        rows = [slice(k * n, (k + 1) * n) for k in ids]
+        for r in rows:
+            if single:
+                assert S.rel_rms(f[r].cpu().numpy(), ref[r].cpu().numpy()) <= 1e-5
+            else:
+                assert torch.equal(f[r], ref[r])
+        return res
+
+    for k in (0, 1):
+        assert served([k], 8 << 20)["peak_bytes"] == scratch[k] + field[k]
+        assert served([k], 2 * (scratch[k] + field[k]) - 512)["peak_bytes"] == scratch[k]
+        assert served([k], scratch[k])["peak_bytes"] == scratch[k]
+    both = served([0, 1], 8 << 20)
+    assert both["peak_lanes"] == 2 and both["peak_bytes"] == sum(scratch) + sum(field)
