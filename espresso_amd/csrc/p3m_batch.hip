@@ -3077,6 +3077,7 @@ void upload_descs(BatchSolver::Impl *m, hipStream_t st) {
   size_t const need = m->sys.size();
   if (need > m->d_sys_cap) {
     dfree(m->d_sys);
+    m->d_sys_cap = 0; // of a null pointer, should the allocation fail
     hip_check(hipMalloc(&m->d_sys, sizeof(SysDesc) * need), "hipMalloc sys");
     m->d_sys_cap = need;
   }
@@ -3136,20 +3137,24 @@ void ensure_scratch(BatchSolver::Impl *m, Lane &ln, int64_t npart, void *externa
   }
   if (nb_need > ln.counts_cap) {
     dfree(ln.counts);
+    ln.counts_cap = 0;
     hip_check(hipMalloc(&ln.counts, sizeof(int) * kCountCopies * std::max(nb_need, 1)),
               "hipMalloc counts");
     ln.counts_cap = nb_need;
   }
   if (nb_need + nsys > ln.offsets_cap) {
     dfree(ln.offsets);
+    ln.offsets_cap = 0;
     hip_check(hipMalloc(&ln.offsets, sizeof(int) * std::max(nb_need + nsys, 1)),
               "hipMalloc offsets");
     ln.offsets_cap = nb_need + nsys;
   }
   if (nsys * 16 > ln.sums_cap) {
     dfree(ln.sums);
+    ln.sums_cap = 0;
     hip_check(hipMalloc(&ln.sums, sizeof(double) * std::max(nsys * 16, 16)), "hipMalloc sums");
     if (ln.h_sums) (void)hipHostFree(ln.h_sums);
+    ln.h_sums = nullptr;
     hip_check(hipHostMalloc(&ln.h_sums, sizeof(double) * (std::max(nsys * 16, 16) + 1 + kStamps)),
               "hipHostMalloc sums");
     ln.sums_cap = nsys * 16;
@@ -3373,6 +3378,7 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
     dfree(ln.tables);
     if (ln.h_tables) (void)hipHostFree(ln.h_tables);
     ln.h_tables = nullptr;
+    ln.tables_cap = 0;
     size_t const cap = host.size() + host.size() / 2 + 64;
     hip_check(hipMalloc(&ln.tables, sizeof(int) * cap), "hipMalloc plan");
     hip_check(hipHostMalloc(&ln.h_tables, sizeof(int) * cap), "hipHostMalloc plan");
@@ -3411,10 +3417,13 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
   for (auto const &g : gh)
     p.groups.push_back({g.cao, g.nsel, p.dbuf + g.sel_start, p.dbuf + g.wt_start, g.blocks,
                         p.dbuf + g.wsp_start, g.blocks_sp, g.nshare});
-  p.version = m->version;
-  if (ln.fixed) return; // partial-sum buffers carved above
+  if (ln.fixed) { // partial-sum buffers carved above
+    p.version = m->version;
+    return;
+  }
   if (p.blocks_bin > ln.bin_cap) {
     dfree(ln.bin_part); // the stream is idle (synchronised above)
+    ln.bin_cap = 0;
     hip_check(hipMalloc(&ln.bin_part, sizeof(double) * 8 * std::max(p.blocks_bin, 1)),
               "hipMalloc bin partials");
     ln.bin_cap = p.blocks_bin;
@@ -3422,10 +3431,12 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
   int const conv_blocks = p.blocks_x + p.blocks_f; // split partials, then fused
   if (conv_blocks > ln.conv_cap) {
     dfree(ln.conv_part);
+    ln.conv_cap = 0;
     hip_check(hipMalloc(&ln.conv_part, sizeof(double) * 8 * std::max(conv_blocks, 1)),
               "hipMalloc conv partials");
     ln.conv_cap = conv_blocks;
   }
+  p.version = m->version; // from here on the plan is complete
 }
 
 template <typename MT>
@@ -3845,6 +3856,7 @@ void BatchSolver::prepare_on(int lane, std::vector<int> const &sel, double *pos,
     dfree(ln.seeds);
     if (ln.h_seeds) (void)hipHostFree(ln.h_seeds);
     ln.h_seeds = nullptr;
+    ln.seeds_cap = 0;
     hip_check(hipMalloc(&ln.seeds, sizeof(unsigned long long) * ns), "hipMalloc seeds");
     hip_check(hipHostMalloc(&ln.h_seeds, sizeof(unsigned long long) * ns), "hipHostMalloc");
     ln.seeds_cap = ns;

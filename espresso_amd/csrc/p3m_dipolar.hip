@@ -750,8 +750,9 @@ __global__ __launch_bounds__(kDpBlock) void k_dp_pairs(int64_t n, double const *
   }
 }
 
-void dp_free(void *p) {
+template <typename T> void dp_free(T *&p) {
   if (p) (void)hipFree(p);
+  p = nullptr;
 }
 
 double sinc_pi(double x) {
@@ -968,14 +969,10 @@ void DipolarSolver::configure(DipolarParams const &p) {
   for (int s = 0; s < 16; ++s) m->plan.radix[s] = fp.radix[s];
   // buffers
   if (M != m->M) {
-    for (auto *&x : m->mesh) {
-      dp_free(x);
-      x = nullptr;
-    }
-    for (auto *&x : m->rmesh) {
-      dp_free(x);
-      x = nullptr;
-    }
+    m->configured = false; // until every mesh is there again
+    m->M = 0;
+    for (auto *&x : m->mesh) dp_free(x);
+    for (auto *&x : m->rmesh) dp_free(x);
     dp_free(m->tw);
     dp_free(m->Ge);
     dp_free(m->Gf);
@@ -1146,6 +1143,7 @@ void DipolarSolver::solve(int64_t n, double const *pos, double const *dip, doubl
   if (need > m->cap_part) {
     hip_check(hipStreamSynchronize(st), "sync");
     dp_free(m->part);
+    m->cap_part = 0; // of a null pointer, should the allocation fail
     hip_check(hipMalloc(&m->part, sizeof(double) * need), "hipMalloc dp3m partials");
     m->cap_part = need;
   }
@@ -1167,10 +1165,9 @@ void DipolarSolver::solve(int64_t n, double const *pos, double const *dip, doubl
   if (n > m->cap_sort || nk > m->cap_keys) {
     hip_check(hipStreamSynchronize(st), "sync");
     if (n > m->cap_sort) {
-      for (void *x : {static_cast<void *>(m->spos), static_cast<void *>(m->sdip),
-                      static_cast<void *>(m->key), static_cast<void *>(m->rank),
-                      static_cast<void *>(m->perm)})
-        dp_free(x);
+      for (double **x : {&m->spos, &m->sdip}) dp_free(*x);
+      for (int **x : {&m->key, &m->rank, &m->perm}) dp_free(*x);
+      m->cap_sort = 0;
       hip_check(hipMalloc(&m->spos, sizeof(double) * 3 * n), "hipMalloc dp3m sort");
       hip_check(hipMalloc(&m->sdip, sizeof(double) * 3 * n), "hipMalloc dp3m sort");
       hip_check(hipMalloc(&m->key, sizeof(int) * n), "hipMalloc dp3m sort");
@@ -1182,6 +1179,7 @@ void DipolarSolver::solve(int64_t n, double const *pos, double const *dip, doubl
       dp_free(m->counts);
       dp_free(m->offsets);
       dp_free(m->total);
+      m->cap_keys = 0;
       hip_check(hipMalloc(&m->counts, sizeof(int) * nk * kDpCopies), "hipMalloc dp3m sort");
       hip_check(hipMalloc(&m->offsets, sizeof(int) * nk), "hipMalloc dp3m sort");
       hip_check(hipMalloc(&m->total, sizeof(int) * nk), "hipMalloc dp3m sort");
@@ -1317,6 +1315,7 @@ void DipolarSolver::short_range(int64_t n, double const *pos, double const *dip,
   if (static_cast<size_t>(nb) > m->cap_part) {
     hip_check(hipStreamSynchronize(st), "sync");
     dp_free(m->part);
+    m->cap_part = 0; // of a null pointer, should the allocation fail
     hip_check(hipMalloc(&m->part, sizeof(double) * nb), "hipMalloc dp3m partials");
     m->cap_part = static_cast<size_t>(nb);
   }

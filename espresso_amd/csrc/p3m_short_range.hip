@@ -754,6 +754,7 @@ template <typename T> void sr_grow(T *&p, size_t &cap, size_t need, char const *
   if (need <= cap) return;
   if (p) (void)hipFree(p);
   p = nullptr;
+  cap = 0; // of a null pointer, should the allocation fail
   size_t const n = need + need / 4 + 64;
   hip_check(hipMalloc(&p, sizeof(T) * n), what);
   cap = n;
