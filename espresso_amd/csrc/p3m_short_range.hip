@@ -14,7 +14,7 @@ namespace espresso_amd {
 namespace {
 using namespace dev;
 
-constexpr int kSRMaxCells = 64; // cells per dimension at most
+constexpr int kSRMaxCells = 64; // cells per dimension at most (z bins of columns: 4 x)
 constexpr int kColWaves = 4;    // waves per block of k_sr_columns
 constexpr int kSortedSlack = 8; // particles k_sr_columns may read past the sorted ones
 
@@ -281,7 +281,7 @@ __device__ __forceinline__ void tile_pairs(double4 const *tile, int cnt, double4
       displacement<MI>(pi, pj, g, dx, dy, dz);
       double const r2 = dx * dx + dy * dy + dz * dz;
       pair_term<EV>(dx, dy, dz, r2, qpi * pj.w, alpha, two_a, fx, fy, fz, ev);
-      if (im.on)
+      if (!MI || im.on) // cells are searched with images only
         image_terms<EV>(im, pi.z, pj.z - sz, dx, dy, g.L[2], qpi * pj.w, rc2, alpha, two_a, fx,
                         fy, fz, ev);
     }
@@ -814,42 +814,25 @@ void ShortRange::compute(hipStream_t st, ShortRangeParams const &p, int64_t n, d
   if (n > INT32_MAX) throw std::invalid_argument("P3M: too many particles for the short range");
   if (n == 0) return;
   hip_check(hipSetDevice(m->device), "hipSetDevice");
-  // cells of edge >= r_cut / nsub: two per r_cut when the box is wide enough
-  // for 5 distinct neighbour cells (one from 128 charges per r_cut^3 on), one
-  // when it allows 3, else all pairs
+  // cells of edge >= r_cut / nsub, two per r_cut or one with subdivision 1, in
+  // boxes that hold 2 nsub + 1 distinct ones along every axis; else all pairs
+  // (a box too narrow for five of r_cut/2 does not hold three of r_cut either)
   if (p.subdivision < 0 || p.subdivision > 2)
     throw std::invalid_argument("P3M: short-range subdivision must be 0, 1 or 2");
   int nsub = (p.subdivision == 1) ? 1 : 2;
-  if (p.subdivision == 0 && !p.elc_images &&
-      static_cast<double>(n) * p.r_cut * p.r_cut * p.r_cut / (p.box[0] * p.box[1] * p.box[2]) >=
-          128.)
-    nsub = 1;
   int nc[3];
-  auto fit = [&](int s) {
-    bool ok = true;
-    for (int d = 0; d < 3; ++d) {
-      nc[d] = std::min(kSRMaxCells, static_cast<int>(std::floor(p.box[d] * s / p.r_cut)));
-      if (nc[d] < 2 * s + 1) ok = false;
-    }
-    return ok;
-  };
-  if (!fit(nsub)) {
-    if (nsub == 1 && p.subdivision == 0 && fit(2)) {
-      nsub = 2; // too narrow for three cells of r_cut, wide enough for five of r_cut/2
-    } else {
-      nsub = 1;
-      if (!fit(1)) {
-        nsub = 0;
-        nc[0] = nc[1] = nc[2] = 1;
-      }
-    }
+  for (int d = 0; d < 3; ++d)
+    nc[d] = std::min(kSRMaxCells, static_cast<int>(std::floor(p.box[d] * nsub / p.r_cut)));
+  if (std::min({nc[0], nc[1], nc[2]}) < 2 * nsub + 1) {
+    nsub = 0;
+    nc[0] = nc[1] = nc[2] = 1;
   }
   CellGrid g;
   for (int d = 0; d < 3; ++d) {
     m->nc[d] = g.nc[d] = nc[d];
     g.L[d] = p.box[d];
   }
-  // without ELC images the pairs run over columns
+  // without ELC images the pairs run over columns of merged cells
   bool const columns = nsub != 0 && !p.elc_images;
   Columns cols{};
   if (columns) {

@@ -16,7 +16,7 @@ struct ShortRangeParams {
   double prefactor = 0.;
   double alpha = 0.;
   double r_cut = 0.;
-  int subdivision = 0; // cells per r_cut: 0 = automatic (2 when the box allows), 1 or 2
+  int subdivision = 0; // cells per r_cut: 0 or 2 = two, 1 = one
   // ELC dielectric contrasts: each pair within r_cut also gets the terms of
   // add_pair_force_corrections / pair_energy_correction (elc.hpp:250-296),
   // particle i against the image of itself in the layer it sits in
@@ -54,8 +54,10 @@ public:
   void compute(hipStream_t st, ShortRangeParams const &p, int64_t n, double const *pos,
                double const *q, double *force, ShortRangeResult *out);
 
-  /** Cells of edge >= r_cut / s that the box of the last call holds per
-   *  dimension (1 1 1: all pairs); the column search merges them in x and y. */
+  /** Cells of edge >= r_cut / s, s = 1 with subdivision 1, else 2, that the
+   *  box of the last call holds per dimension (1 1 1: all pairs).  The search
+   *  with ELC images runs over these; the column search has a grid of its own
+   *  and goes by them only for whether the box is wide enough. */
   void cells(int out[3]) const;
 
   /** Dipolar real space (DipolarP3M::pair_force / pair_energy,

@@ -537,12 +537,15 @@ class _P3MBase:
         return force
 
     def set_short_range_subdivision(self, cells_per_cutoff):
-        """Cells per r_cut of the short-range cell lists (0: automatic)."""
+        """Cells per r_cut of the short-range cell lists: 1, or 2 (0 is 2).
+        Boxes narrower than 3 r_cut (2.5 r_cut) along an axis take all pairs;
+        the cells themselves are searched with ELC images only."""
         _lib.raise_for(_lib.load().p3m_set_short_range_subdivision(
             self._ctx, int(cells_per_cutoff)), self._ctx)
 
     def short_range_cells(self):
-        """Cells per dimension of the last short-range call."""
+        """Cells of the chosen edge that the box of the last short-range call
+        holds per dimension (1 1 1: all pairs)."""
         c = (C.c_int * 3)()
         _lib.raise_for(_lib.load().p3m_short_range_cells(self._ctx, c), self._ctx)
         return list(c)

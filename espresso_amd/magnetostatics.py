@@ -247,7 +247,8 @@ class DipolarP3M:
         return e.value if energy else None
 
     def set_short_range_subdivision(self, cells_per_cutoff):
-        """Cells per r_cut of the real space: 0 (automatic), 1 or 2."""
+        """Cells per r_cut of the real space: 1, or 2 (0 is 2).  Boxes narrower
+        than 3 r_cut (2.5 r_cut) take all pairs."""
         _lib.raise_for(_lib.load().p3m_dipolar_set_short_range_subdivision(
             self._ctx, int(cells_per_cutoff)), dipolar=self._ctx)
 

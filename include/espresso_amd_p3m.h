@@ -225,11 +225,11 @@ int p3m_real_space_error(double prefactor, double r_cut_iL, int n_c_part, double
  * (p3m.hpp:167-180), P3M_PRESSURE sets virial[9] to sum_pairs F (x) d. */
 int p3m_short_range(p3m_context *ctx, int64_t n, const double *pos, const double *q,
                     unsigned flags, double *force, double *energy, double *virial);
-/* Cells per r_cut of the short-range cell lists: 0 = automatic, 1 or 2
- * (falls back to fewer cells, then all pairs, in narrow boxes).  Without ELC
- * images the pair search runs over columns of these cells merged to edge
- * r_cut, and the value only decides how narrow a box may be before all pairs
- * are taken: 3 r_cut with 1, else 2.5 r_cut. */
+/* Cells per r_cut of the short-range cell lists: 1, or 2 (0, the default, is
+ * 2).  The value decides how narrow a box may be before all pairs are taken
+ * (3 r_cut along every axis with 1, else 2.5 r_cut) and the cells of the pair
+ * search with ELC images; without images the search runs over columns of edge
+ * r_cut with either value (of r_cut/2 along an axis under 3 r_cut). */
 int p3m_set_short_range_subdivision(p3m_context *ctx, int cells_per_cutoff);
 
 /* Force convention of p3m_solve.  P3M_CONV_GPU gives the forces of the
@@ -344,9 +344,9 @@ int p3m_dipolar_solve(p3m_dipolar *ctx, int64_t n, const double *pos, const doub
  * below half the box): forces and torques added, energy with P3M_ENERGY. */
 int p3m_dipolar_short_range(p3m_dipolar *ctx, int64_t n, const double *pos, const double *dip,
                             double *force, double *torque, unsigned flags, double *energy);
-/* Cells per r_cut of p3m_dipolar_short_range: 0 = automatic, 1 or 2; as for
- * p3m_set_short_range_subdivision, all pairs are taken in boxes narrower than
- * 3 r_cut with 1, else 2.5 r_cut. */
+/* Cells per r_cut of p3m_dipolar_short_range: 1, or 2 (0, the default, is 2).
+ * As for p3m_set_short_range_subdivision, all pairs are taken in boxes narrower
+ * than 3 r_cut with 1, else 2.5 r_cut; that is all the value decides. */
 int p3m_dipolar_set_short_range_subdivision(p3m_dipolar *ctx, int cells_per_cutoff);
 int p3m_dipolar_get_stream(const p3m_dipolar *ctx, void **stream);
 int p3m_dipolar_wait_stream(p3m_dipolar *ctx, void *producer); /* as p3m_wait_stream */
@@ -359,8 +359,9 @@ int p3m_dipolar_synchronize(p3m_dipolar *ctx);
  * each trial (r_cut, alpha), for callers whose pair loop runs there;
  * P3M_TUNE_RS_MODEL (default) models a host loop at 1 ns per pair. */
 int p3m_set_tuning_real_space(p3m_context *ctx, int mode);
-/* Cells of the chosen edge that the box of the last p3m_short_range call holds
- * per dimension (0 0 0 before the first; 1 1 1 for all pairs). */
+/* Cells of edge r_cut, with subdivision 1, or r_cut/2 that the box of the last
+ * p3m_short_range call holds per dimension, at most 64 (0 0 0 before the first;
+ * 1 1 1 for all pairs). */
 int p3m_short_range_cells(const p3m_context *ctx, int cells[3]);
 
 /* Real-space pair forces of CoulombP3M::pair_force (p3m.hpp:146-165, A&S

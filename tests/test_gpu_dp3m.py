@@ -80,8 +80,8 @@ def test_kspace_clustered_and_partial_outputs():
 
 @pytest.mark.parametrize("subdiv", [0, 1, 2])
 def test_short_range_cell_lists_match_oracle(subdiv):
-    """Cell lists of edge r_cut (subdivision 1) and r_cut/2 (2), and the
-    occupancy choice (0), against the oracle's all-pairs sum."""
+    """Every number of cells per cutoff in a box wide enough for all of them
+    (the column search) against the oracle's all-pairs sum."""
     from espresso_amd.magnetostatics import DipolarP3M
     from oracle import dp3m as D
     L = 20.
@@ -120,13 +120,32 @@ def test_particle_count_beyond_int32_rejected():
             _lib.raise_for(rc, dipolar=dp._ctx)
 
 
-# r_cut 3.5: 125 cells of about 27 dipoles (block queue); r_cut 6.5: 27 cells
-# of about 126 dipoles (per-wave queues, home passes of more than 64 lanes)
+@pytest.mark.parametrize("box", [5.6, 5.4])
+def test_narrow_boxes_match_oracle(box):
+    """Boxes of 2.5 to 3 cutoffs go by columns with two cells per cutoff and by
+    all pairs with one, narrower ones by all pairs."""
+    from espresso_amd.magnetostatics import DipolarP3M
+    from oracle import dp3m as D
+    n, r_cut = 700, 2.2
+    pos, dip = _system(n, box, 15)
+    fr, tr, er = D.pair_terms(pos - box * np.floor(pos / box), dip, box, 1.3, 0.9, r_cut, 1e-4)
+    dp = DipolarP3M(prefactor=1.3, accuracy=1e-4, mesh=16, cao=4, alpha=0.9, r_cut=r_cut,
+                    tune=False)
+    dp.activate(pos, dip, box_l=box)
+    for subdiv in (0, 1, 2):
+        dp.set_short_range_subdivision(subdiv)
+        f, t = np.zeros((n, 3)), np.zeros((n, 3))
+        e = dp.add_short_range_forces(pos, dip, f, t, energy=True)
+        assert S.rel_rms(f, fr) <= 1e-12 and S.rel_rms(t, tr) <= 1e-12
+        assert abs(e - er) <= 1e-12 * abs(er)
+
+
+# r_cut 3.5: columns with z bins of r_cut/2 (16 dipoles per r_cut^3 on average);
+# r_cut 6.5: three columns along x and y, z bins of r_cut/4
 @pytest.mark.parametrize("subdiv,r_cut", [(1, 3.5), (2, 3.5), (1, 6.5)])
 def test_short_range_dense_cluster_matches_oracle(subdiv, r_cut):
-    """400 dipoles packed into one cell among 3000 sparse ones: a home cell
-    of more than 256 dipoles (two home passes), candidate tables of more
-    than one window and many queue drains."""
+    """400 dipoles packed into one place among 3000 sparse ones: several full
+    home groups in one z bin, and lists that fill and drain many times."""
     from espresso_amd.magnetostatics import DipolarP3M
     from oracle import dp3m as D
     L = 20.

@@ -4,8 +4,10 @@ reference's pair_force/pair_energy with the A&S erfc, p3m.hpp:146-180).
 
 Forces rel-rms <= 1e-12, energy and virial <= 1e-12 relative: both sides
 evaluate the same FP64 pair terms and differ only in summation order.  The
-cases cover cells of edge r_cut/2 and r_cut, the all-pairs path of narrow
-boxes, non-cubic boxes, uncharged particles and positions outside the box.
+cases cover the column search, the all-pairs path of narrow boxes and where
+the cells per cutoff draw the line between them, non-cubic boxes, uncharged
+particles and positions outside the box; the cell search of ELC images is
+covered with ELC.
 The total device force (k-space + short range) is checked against exact
 Ewald on the C3 fixture subset.
 """
@@ -72,6 +74,47 @@ def test_short_range_matches_oracle(box, r_cut, subdiv, cells):
     p3m.add_short_range_forces(tp, tq, tf2, sync=False)
     p3m.synchronize()
     assert S.rel_rms(tf2.cpu().numpy(), f_ref) <= 1e-12
+
+
+@pytest.mark.parametrize("box,cells", [
+    ((5.6, 5.7, 5.8), (5, 5, 5)),    # 2.5 to 3 cutoffs along every axis
+    ((9., 5.6, 12.), (8, 5, 10)),    # along one
+    ((5.4, 9., 9.), None),           # too narrow for either
+])
+def test_cells_per_cutoff_decide_when_all_pairs_are_taken(box, cells):
+    """A box of 2.5 to 3 cutoffs is searched by columns with two cells per
+    cutoff and takes all pairs with one; the same sums either way, at any
+    density (500 charges, and 5000: more than 128 per cubed cutoff in the
+    smallest box)."""
+    import torch
+    from oracle import oracle as O
+    r_cut = 2.2
+    p3m = _actor(box, r_cut, 1.1)
+    for n in (500, 5000):
+        pos, q = _system(n, box, n)
+        e_ref, f_ref = O.real_space(pos, q, box, 1.3, 1.1, r_cut)
+        for subdiv in (0, 1, 2):
+            p3m.set_short_range_subdivision(subdiv)
+            tf = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
+            e = p3m.add_short_range_forces(torch.tensor(pos, device="cuda"),
+                                           torch.tensor(q, device="cuda"), tf, energy=True)
+            pairs = subdiv == 1 or cells is None
+            assert tuple(p3m.short_range_cells()) == ((1, 1, 1) if pairs else cells)
+            assert S.rel_rms(tf.cpu().numpy(), f_ref) <= 1e-12
+            assert abs(e - e_ref) <= 1e-12 * abs(e_ref)
+
+
+def test_cells_per_cutoff_do_not_depend_on_the_density():
+    """Cells of r_cut/2 by default, from sparse to 128 charges per r_cut^3 and
+    more."""
+    import torch
+    p3m = _actor((9., 9., 9.), 2.2, 1.1)
+    for n in (300, 8700, 9000):
+        pos, q = _system(n, (9., 9., 9.), n)
+        f = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
+        p3m.add_short_range_forces(torch.tensor(pos, device="cuda"),
+                                   torch.tensor(q, device="cuda"), f)
+        assert tuple(p3m.short_range_cells()) == (8, 8, 8)
 
 
 def test_short_range_host_arrays_and_errors():
