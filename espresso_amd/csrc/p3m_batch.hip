@@ -67,15 +67,20 @@ constexpr int kCountCopies = 8; // brick counter copies (one per XCD-sized share
 constexpr int kBrick = 8;    // first-stencil points per brick edge
 constexpr int kFill = 8192;  // mesh elements zeroed per block
 // systems of up to this many particles and bins are binned by one block of
-// kSmallBlock threads (bin_system): 13.8 us at 1000 particles against 23 for
-// the four launches otherwise, 35 against 26 at 10^4
+// kSmallBlock threads (bin_system), others in four launches.  FP64 solves,
+// one block against four launches: 1000 particles 59 against 68 us at mesh 32
+// and 57 against 69 at mesh 16, 4000 66 against 71 and 63 against 81; at mesh
+// 32 the two meet between 6000 (75, 75) and 8000 (77, 75), with fewer bins
+// later (mesh 16, 8000: 73, 98); eight systems at once and FP32 meshes alike
 constexpr int kSmallSystem = 4096, kSmallBins = 4096, kSmallBlock = 1024;
 constexpr int kStamps = 8;   // stage start times of a solve
 constexpr int kWideBlock = 512;    // threads of a k_fft_yx_conv_wide block
 // kz columns of a selection up to which that kernel runs: 384 blocks, three
 // component blocks to every two CUs (mesh 32 FP64: 13.1 against 22.8 us, mesh
-// 64 FP32: 19.7 against 44.8; with the chip filled by whole columns, 256
-// systems, the one-block pass does 7 line passes where this one does 12)
+// 64 FP32: 19.7 against 44.8; solves near the limit, 119 columns of mesh 32
+// FP64 77 against 82 us, 125 of mesh 48 106 against 122; with the chip filled
+// by whole columns, 256 systems, the one-block pass does 7 line passes where
+// this one does 12)
 constexpr int kWideColumns = 128;
 
 /** Per-system state read by every kernel. */
@@ -851,7 +856,7 @@ __global__ __launch_bounds__(NTH, SEGMAX == 64 ? 8 : 1) void k_spread(SysDesc co
                                                int const *__restrict__ offsets,
                                                double4 const *__restrict__ spos, int chunk,
                                                double const *__restrict__ sums, int int_mesh,
-    int nshare, unsigned long long *stamp) {
+                                               int nshare, unsigned long long *stamp) {
   stamp_start(stamp);
   using GR = GroupRows<P, NTH, SX, SY, SZ>;
   constexpr int TY = GR::TY, TZ = GR::TZ;
@@ -977,7 +982,7 @@ __global__ __launch_bounds__(kBlock) void k_fft_z_r2c(SysDesc const *__restrict_
                                                       int const *__restrict__ wt, int nsel,
                                                       cx_t<MT> const *__restrict__ tw, int nlp,
                                                       double const *__restrict__ sums, int det,
-    unsigned long long *stamp) {
+                                                      unsigned long long *stamp) {
   stamp_start(stamp);
   using C = cx_t<MT>;
   extern __shared__ double smem_d[];
@@ -1080,7 +1085,7 @@ __global__ __launch_bounds__(kBlock) void k_fft_x_conv(SysDesc const *__restrict
                                                        cx_t<MT> const *__restrict__ tw, int ncol,
                                                        int want_fields, int want_energy,
                                                        double *partials,
-    unsigned long long *stamp) {
+                                                       unsigned long long *stamp) {
   stamp_start(stamp);
   using C = cx_t<MT>;
   extern __shared__ double smem_d[];
@@ -1174,7 +1179,7 @@ __global__ __launch_bounds__(kBlock) void k_fft_y_inv(SysDesc const *__restrict_
                                                       int const *__restrict__ sel,
                                                       int const *__restrict__ wt, int nsel,
                                                       cx_t<MT> const *__restrict__ tw, int ncol,
-    unsigned long long *stamp) {
+                                                      unsigned long long *stamp) {
   stamp_start(stamp);
   using C = cx_t<MT>;
   extern __shared__ double smem_d[];
@@ -1260,7 +1265,7 @@ __global__ __launch_bounds__(kBlock) void k_fft_yx_conv(SysDesc const *__restric
                                                         cx_t<MT> const *__restrict__ tw,
                                                         int want_fields, int want_energy,
                                                         double *partials,
-    unsigned long long *stamp) {
+                                                        unsigned long long *stamp) {
   stamp_start(stamp);
   using C = cx_t<MT>;
   extern __shared__ double smem_d[];
@@ -1511,7 +1516,7 @@ __global__ __launch_bounds__(kBlock) void k_fft_z_c2r(SysDesc const *__restrict_
                                                       cx_t<MT> const *__restrict__ tw, int nlp,
                                                       cx_t<MT> const *__restrict__ ybuf,
                                                       int const *__restrict__ ycol,
-    unsigned long long *stamp) {
+                                                      unsigned long long *stamp) {
   stamp_start(stamp);
   using C = cx_t<MT>;
   extern __shared__ double smem_d[];
@@ -2099,7 +2104,7 @@ __global__ __launch_bounds__(256) void k_spread_col(SysDesc const *__restrict__ 
                                                    int const *__restrict__ soff,
                                                    int const *__restrict__ offsets,
                                                    double4 const *__restrict__ spos, int chunk,
-    unsigned long long *stamp) {
+                                                   unsigned long long *stamp) {
   stamp_start(stamp);
   using G = ColGeo<P, W>;
   constexpr int IP = G::IP;
@@ -3103,8 +3108,8 @@ void ensure_scratch(BatchSolver::Impl *m, Lane &ln, int64_t npart, void *externa
   size_t const field = ln.plan.field_bytes;
   bool const grow_own = !external && need > ln.own_bytes;
   bool const grow_field = !external && field > ln.own_ybuf_bytes;
-  bool const grow = grow_own || grow_field || nb_need > ln.counts_cap || nb_need + nsys > ln.offsets_cap ||
-                    nsys * 16 > ln.sums_cap;
+  bool const grow = grow_own || grow_field || nb_need > ln.counts_cap ||
+                    nb_need + nsys > ln.offsets_cap || nsys * 16 > ln.sums_cap;
   if (grow) hip_check(hipStreamSynchronize(ln.stream), "sync before realloc"); // queued work
   if (external) {
     if (external_bytes < need) throw std::invalid_argument("P3M: scratch block too small");
@@ -3346,10 +3351,13 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
       g.blocks_sp = acc;
     }
     // few, crowded bricks are shared by several blocks (each reads or flushes
-    // the whole tile), until every CU has one or a share would hold fewer
-    // particles than a chunk.  64 bricks of 156 particles in 4 shares: gather
-    // 15.4 -> 7.6 us, spread 10.3 -> 7.6; 216 bricks of 139 in 2: gather 16.6
-    // -> 17.4, spread 14.2 -> 20.8, so not beyond 256 blocks
+    // the whole tile): twice as many while there are at most 128 blocks and
+    // more than 48 particles to each, so up to 256 blocks of 25 particles or
+    // more.  64 bricks of 156 particles in 4 shares: gather 15.4 -> 7.6 us,
+    // spread 10.3 -> 7.6; 216 bricks of 139 in 2: gather 16.6 -> 17.4, spread
+    // 14.2 -> 20.8, so not beyond 256 blocks.  FP64 solves, unshared -> shared:
+    // 27 bricks of 56 (cao 5) 61 -> 59 us, 64 of 78 76 -> 72, 125 of 80 in 2
+    // 81 -> 78 (cao 3 77 -> 74, cao 7 90 -> 83), 125 of 320 114 -> 100
     int64_t np = 0;
     for (int s : gs) np += m->sys[s].n;
     if (shape.column == 0)
@@ -3505,10 +3513,11 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
                                sizeof(typename SpreadWord<MT>::type);
         auto const args = std::make_tuple(sys, g.d_sel, g.wt_sp, g.nsel, p.soff, ln.offsets,
                                           static_cast<double4 const *>(ln.spos), shape.chunk,
-                                          static_cast<double const *>(ln.sums), det ? 1 : 0, g.nshare,
-                                          stamp(1));
+                                          static_cast<double const *>(ln.sums), det ? 1 : 0,
+                                          g.nshare, stamp(1));
         auto launch = [&](auto kern) {
-          std::apply([&](auto... a) { kern<<<g.blocks_sp * g.nshare, NT.value, lds, st>>>(a...); }, args);
+          int const blocks = g.blocks_sp * g.nshare;
+          std::apply([&](auto... a) { kern<<<blocks, NT.value, lds, st>>>(a...); }, args);
         };
         if (shape.group == 4)
           launch(k_spread<P.value, MT, 64, NT.value, 2, 2, 1>);
@@ -3598,7 +3607,8 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
                               static_cast<double const *>(ln.sums), shape.chunk, g.nshare,
                               stamp(5));
           auto launch = [&](auto kern) {
-            std::apply([&](auto... a) { kern<<<g.blocks * g.nshare, NT.value, lds, st>>>(a...); }, args);
+            int const blocks = g.blocks * g.nshare;
+            std::apply([&](auto... a) { kern<<<blocks, NT.value, lds, st>>>(a...); }, args);
           };
           if (shape.gather == kGatherPlane8)
             launch(k_gather_plane<P.value, MT, 8, NT.value>);

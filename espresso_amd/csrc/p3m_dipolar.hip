@@ -322,9 +322,10 @@ __global__ __launch_bounds__(kDpPlaneBlock) void k_dp_fft_plane(double *const *r
  *  meshes in one pass over the half spectrum (Nyquist wave number 0): with
  *  the transformed dipole components A_d (table entries 0..2) and the
  *  integer wave numbers D, z = sum_d D_d A_d gives the energy partials
- *  G_e |z|^2, twice where -k lies in the other half.  With back != 0 the field meshes T_d = D_d G_e z overwrite
- *  A_d, and with forces != 0 the six force meshes F_ab = D_a D_b (-i G_f z)
- *  (xx xy xz yy yz zz, table entries 3..8) are written. */
+ *  G_e |z|^2, twice where -k lies in the other half.  With back != 0 the
+ *  field meshes T_d = D_d G_e z overwrite A_d, and with forces != 0 the six
+ *  force meshes F_ab = D_a D_b (-i G_f z) (xx xy xz yy yz zz, table entries
+ *  3..8) are written. */
 __global__ __launch_bounds__(kDpBlock) void k_dp_kspace(C2 *const *T, C2 *const *F,
                                                         double const *__restrict__ Ge,
                                                         double const *__restrict__ Gf, int M,

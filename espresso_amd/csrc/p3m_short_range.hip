@@ -56,10 +56,8 @@ __global__ __launch_bounds__(256) void k_sr_bin(int64_t n, double const *__restr
   p_rank[i] = atomicAdd(&counts[cell], 1);
 }
 
-/** Exclusive scan of the cell counts (one block, four cells per thread and
- *  pass); offsets[ncells] = total.  With goff, the cells are the z bins of
- *  columns of nz bins: goff[c] = 64-particle home groups in the columns before c (a
- *  group never crosses a column), goff[ncol] = all of them. */
+/** Exclusive scan of one value per thread of a 1024-thread block, and the sum
+ *  of all. */
 __device__ __forceinline__ int block_scan_1024(int v, int *wsum, int &total) {
   int const lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   int s = v;
@@ -81,6 +79,11 @@ __device__ __forceinline__ int block_scan_1024(int v, int *wsum, int &total) {
   total = all;
   return before + s - v;
 }
+
+/** Exclusive scan of the cell counts (one block, four cells per thread and
+ *  pass); offsets[ncells] = total.  With goff, the cells are the z bins of
+ *  columns of nz bins: goff[c] = 64-particle home groups in the columns
+ *  before c (a group never crosses a column), goff[ncol] = all of them. */
 __global__ __launch_bounds__(1024) void k_sr_scan(int const *counts, int ncells, int *offsets,
                                                   int nz, int *goff, int *arrived) {
   __shared__ int wsum[16];
@@ -456,9 +459,9 @@ __device__ __forceinline__ void dip_pair(double dx, double dy, double dz, double
 
 /** Pair terms over columns: Coulomb without ELC images, or dipolar (DIP, sdip
  *  the sorted dipoles).  The cells are columns of edge >= r_cut / rx (x) and
- *  r_cut / ry (y), cut into z bins of edge >= r_cut / rz, z fastest, so that the candidates of a column within reach of a home
- *  group are one contiguous run of the sorted particles (split at the
- *  periodic boundary).  One block of W waves per home group of 64 sorted
+ *  r_cut / ry (y), cut into z bins of edge >= r_cut / rz, z fastest, so that
+ *  the candidates of a column within reach of a home group are one contiguous
+ *  run of the sorted particles (split at the periodic boundary).  One block of W waves per home group of 64 sorted
  *  particles of one column: lane = home particle, position and force in
  *  registers; the waves share the runs of the (2 rx + 1)(2 ry + 1) columns,
  *  U candidates at a time, and their forces are added through LDS at the end.
@@ -728,9 +731,10 @@ Columns make_columns(ShortRangeParams const &p, int64_t n) {
   c.max_groups =
       static_cast<int>(std::min<int64_t>(n, n / 64 + c.ncol)); // one partial group per column
   // Few groups are shared by several blocks, each taking every split-th batch
-  // of candidates.  Up to 4096 blocks, four rounds of what the chip holds, as
-  // long as the lists of one wave still fill: its candidates must be a
-  // twentieth of the number of blocks.  Dipolar and Coulomb kernel, at that
+  // of candidates: twice as many while there are fewer than 4096 blocks, four
+  // rounds of what the chip holds (so fewer than 8192 in the end), as long as
+  // the lists of one wave still fill: its candidates must be a twentieth of the
+  // number of blocks.  Dipolar and Coulomb kernel, at that
   // split against twice and half of it: 1006 groups of 980 candidates each
   // 84 us in 2 blocks, 103 in 4, 111 in 1; 40 groups of 1900 32 us in 8, 36 in
   // 16; 321 groups of 16,700 0.62 ms in 16, 0.71 in 8.
