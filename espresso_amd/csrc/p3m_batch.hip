@@ -147,22 +147,24 @@ __device__ __forceinline__ Slot locate(int const *wt, int const *sel, int nsel) 
   return r;
 }
 
-/** locate() for kernels that share a brick among nshare blocks: the brick's
- *  slot and this block's share of it. */
-__device__ __forceinline__ Slot locate_share(int const *wt, int const *sel, int nsel, int nshare,
+/** locate() for kernels that share a brick among 2^lgshare blocks: the brick's
+ *  slot and this block's share of it.  Shifts, not divisions: selections of
+ *  many light bricks pay for this in every block (6912 bricks of 46 particles,
+ *  cao 1: spread 31.2 us without shares, 34.9 with divisions, 32.3 so). */
+__device__ __forceinline__ Slot locate_share(int const *wt, int const *sel, int nsel, int lgshare,
                                              int &share) {
   Slot r;
   int const v = xcd_block();
-  r.vb = v / nshare;
-  share = v - r.vb * nshare;
+  r.vb = v >> lgshare;
+  share = v - (r.vb << lgshare);
   r.slot = find_slot(wt, nsel, r.vb);
   r.s = sel[r.slot];
   r.lb = r.vb - wt[r.slot];
   return r;
 }
-/** Narrows the particles [beg, end) of a brick to one of nshare shares. */
-__device__ __forceinline__ void take_share(int nshare, int share, int &beg, int &end) {
-  int const per = (end - beg + nshare - 1) / nshare;
+/** Narrows the particles [beg, end) of a brick to one of 2^lgshare shares. */
+__device__ __forceinline__ void take_share(int lgshare, int share, int &beg, int &end) {
+  int const per = (end - beg + (1 << lgshare) - 1) >> lgshare;
   beg = min(end, beg + share * per);
   end = min(end, beg + per);
 }
@@ -856,7 +858,7 @@ __global__ __launch_bounds__(NTH, SEGMAX == 64 ? 8 : 1) void k_spread(SysDesc co
                                                int const *__restrict__ offsets,
                                                double4 const *__restrict__ spos, int chunk,
                                                double const *__restrict__ sums, int int_mesh,
-                                               int nshare, unsigned long long *stamp) {
+                                               int lgshare, unsigned long long *stamp) {
   stamp_start(stamp);
   using GR = GroupRows<P, NTH, SX, SY, SZ>;
   constexpr int TY = GR::TY, TZ = GR::TZ;
@@ -873,7 +875,7 @@ __global__ __launch_bounds__(NTH, SEGMAX == 64 ? 8 : 1) void k_spread(SysDesc co
 
   // the block's group of SX x SY x SZ bricks and their particle runs
   int share;
-  Slot const L = locate_share(wt, sel, nsel, nshare, share);
+  Slot const L = locate_share(wt, sel, nsel, lgshare, share);
   SysDesc const &d = sys[L.s];
   int const nb0 = d.g.nb[0], nb1 = d.g.nb[1], nb2 = d.g.nb[2];
   int const ng2 = (nb2 + SZ - 1) / SZ, ng1 = (nb1 + SY - 1) / SY;
@@ -889,7 +891,7 @@ __global__ __launch_bounds__(NTH, SEGMAX == 64 ? 8 : 1) void k_spread(SysDesc co
       int const b = (bx * nb1 + by) * nb2 + bz;
       rb[u] = offsets[d.off_off + b];
       re[u] = offsets[d.off_off + b + 1];
-      take_share(nshare, share, rb[u], re[u]);
+      take_share(lgshare, share, rb[u], re[u]);
     }
     ntot += re[u] - rb[u];
   }
@@ -1658,7 +1660,7 @@ __global__ __launch_bounds__(NTH) void k_gather_plane(
     int nsel, int const *__restrict__ soff, int const *__restrict__ offsets,
     double4 const *__restrict__ spos, int const *__restrict__ sidx, double *__restrict__ force,
     double const *__restrict__ sums, int chunk,
-    int nshare, unsigned long long *stamp) {
+    int lgshare, unsigned long long *stamp) {
   stamp_start(stamp);
   constexpr int T = kBrick + P - 1;
   constexpr int TYZ = T * T;
@@ -1673,12 +1675,12 @@ __global__ __launch_bounds__(NTH) void k_gather_plane(
   MT *tz = ty + tile_n;
 
   int share;
-  Slot const L = locate_share(wt, sel, nsel, nshare, share);
+  Slot const L = locate_share(wt, sel, nsel, lgshare, share);
   SysDesc const &d = sys[L.s];
   int const tyz = d.g.T[1] * d.g.T[2]; // == TYZ (bricks), read at run time
   int const b = L.lb;
   int beg = offsets[d.off_off + b], end = offsets[d.off_off + b + 1];
-  take_share(nshare, share, beg, end);
+  take_share(lgshare, share, beg, end);
   if (beg == end) return;
   int o0, o1, o2;
   brick_origin<P>(d, b, o0, o1, o2);
@@ -1775,7 +1777,7 @@ __global__ __launch_bounds__(NTH, (NTH == 512 && sizeof(MT) == 4) ? 8 : 1) void 
     int nsel, int const *__restrict__ soff, int const *__restrict__ offsets,
     double4 const *__restrict__ spos, int const *__restrict__ sidx, double *__restrict__ force,
     double const *__restrict__ sums, int chunk,
-    int nshare, unsigned long long *stamp) {
+    int lgshare, unsigned long long *stamp) {
   stamp_start(stamp);
   constexpr int T = kBrick + P - 1;
   constexpr int TYZ = T * T;
@@ -1792,11 +1794,11 @@ __global__ __launch_bounds__(NTH, (NTH == 512 && sizeof(MT) == 4) ? 8 : 1) void 
   MT *tz = ty + tile_n;
 
   int share;
-  Slot const L = locate_share(wt, sel, nsel, nshare, share);
+  Slot const L = locate_share(wt, sel, nsel, lgshare, share);
   SysDesc const &d = sys[L.s];
   int const b = L.lb;
   int beg = offsets[d.off_off + b], end = offsets[d.off_off + b + 1];
-  take_share(nshare, share, beg, end);
+  take_share(lgshare, share, beg, end);
   if (beg == end) return;
   int o0, o1, o2;
   brick_origin<P>(d, b, o0, o1, o2);
@@ -2425,7 +2427,7 @@ struct Plan {
     int blocks;
     int *wt_sp;    // spread work table (brick groups of LaunchShape::group)
     int blocks_sp;
-    int nshare;    // blocks per brick of the spread and gather
+    int lgshare;   // log2 of the blocks per brick of the spread and gather
   };
   std::vector<Group> groups;
   int nlp_z = 1, nlp_zc = 1, c2r_comps = 3, ncol_y = 1, ncol_x = 1, ncol_yi = 1;
@@ -3319,7 +3321,7 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
   });
   p.field_bytes = align256(static_cast<size_t>(yc.second) * csz);
   struct GH {
-    int cao, sel_start, nsel, wt_start, blocks, wsp_start, blocks_sp, nshare;
+    int cao, sel_start, nsel, wt_start, blocks, wsp_start, blocks_sp, lgshare;
   };
   int const gsx = 2, gsy = 2, gsz = 1; // brick groups of the spread (LaunchShape::group 4)
   std::vector<GH> gh;
@@ -3328,7 +3330,7 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
     for (int s : sel)
       if (m->sys[s].desc.cao == cao) gs.push_back(s);
     if (gs.empty()) continue;
-    GH g{cao, static_cast<int>(host.size()), static_cast<int>(gs.size()), 0, 0, 0, 0, 1};
+    GH g{cao, static_cast<int>(host.size()), static_cast<int>(gs.size()), 0, 0, 0, 0, 0};
     host.insert(host.end(), gs.begin(), gs.end());
     g.wt_start = static_cast<int>(host.size());
     int acc = 0;
@@ -3361,8 +3363,9 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
     int64_t np = 0;
     for (int s : gs) np += m->sys[s].n;
     if (shape.column == 0)
-      while (g.blocks * g.nshare <= 128 && np > 48 * static_cast<int64_t>(g.blocks) * g.nshare)
-        g.nshare *= 2;
+      while ((g.blocks << g.lgshare) <= 128 &&
+             np > (48 * static_cast<int64_t>(g.blocks) << g.lgshare))
+        ++g.lgshare;
     gh.push_back(g);
   }
   // per-system offsets of the selection's particles in the lane scratch
@@ -3424,7 +3427,7 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
   p.npart = npart;
   for (auto const &g : gh)
     p.groups.push_back({g.cao, g.nsel, p.dbuf + g.sel_start, p.dbuf + g.wt_start, g.blocks,
-                        p.dbuf + g.wsp_start, g.blocks_sp, g.nshare});
+                        p.dbuf + g.wsp_start, g.blocks_sp, g.lgshare});
   if (ln.fixed) { // partial-sum buffers carved above
     p.version = m->version;
     return;
@@ -3514,9 +3517,9 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
         auto const args = std::make_tuple(sys, g.d_sel, g.wt_sp, g.nsel, p.soff, ln.offsets,
                                           static_cast<double4 const *>(ln.spos), shape.chunk,
                                           static_cast<double const *>(ln.sums), det ? 1 : 0,
-                                          g.nshare, stamp(1));
+                                          g.lgshare, stamp(1));
         auto launch = [&](auto kern) {
-          int const blocks = g.blocks_sp * g.nshare;
+          int const blocks = g.blocks_sp << g.lgshare;
           std::apply([&](auto... a) { kern<<<blocks, NT.value, lds, st>>>(a...); }, args);
         };
         if (shape.group == 4)
@@ -3604,10 +3607,10 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
               std::make_tuple(sys, g.d_sel, g.wt, g.nsel, p.soff, ln.offsets,
                               static_cast<double4 const *>(ln.spos),
                               static_cast<int const *>(ln.sidx), pa.force,
-                              static_cast<double const *>(ln.sums), shape.chunk, g.nshare,
+                              static_cast<double const *>(ln.sums), shape.chunk, g.lgshare,
                               stamp(5));
           auto launch = [&](auto kern) {
-            int const blocks = g.blocks * g.nshare;
+            int const blocks = g.blocks << g.lgshare;
             std::apply([&](auto... a) { kern<<<blocks, NT.value, lds, st>>>(a...); }, args);
           };
           if (shape.gather == kGatherPlane8)
