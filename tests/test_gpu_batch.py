@@ -326,3 +326,31 @@ def test_wide_fused_pass_matches_the_one_block_pass(single):
             assert e[0] == e_all[k] and np.array_equal(v[0], v_all[k])
         e_only, _ = b.solve(tp, tq, None, systems=[k], energy=True)
         assert abs(e_only[0] - e[0]) <= (2e-6 if single else 1e-12) * (abs(e[0]) + len(q[k]))
+
+
+@pytest.mark.parametrize("mesh,cao,n,others", [
+    (32, 7, 12000, 2),   # 64 bricks in 4 shares, 192 bricks unshared
+    (16, 7, 5000, 16),   # 8 bricks in 16 shares, 136 bricks unshared
+    (40, 6, 25000, 1),   # 125 bricks in 2 shares, 250 bricks unshared
+    (24, 3, 4999, 4),    # 27 bricks in 4 shares, 135 bricks unshared
+])
+def test_shared_bricks_give_the_bits_of_unshared_ones(mesh, cao, n, others):
+    """A system alone, its bricks shared by several blocks, against the same
+    system in a selection of more than 128 bricks, which shares none: equal
+    FP64 forces bit for bit (fixed-point spread, per-particle gather)."""
+    import torch
+    from espresso_amd import P3MBatch
+    L = 11.
+    b = P3MBatch(single_precision=False)
+    for _ in range(1 + others):
+        b.add_system([L] * 3, n, 1.1, mesh, cao, 0.9, 2.)
+    rng = np.random.default_rng(mesh + cao)
+    pos = rng.uniform(0., L, (n * (1 + others), 3))
+    pos[: n // 4] *= 0.4  # one corner is more crowded
+    pos = torch.tensor(pos, device="cuda")
+    q = torch.tensor(np.where(np.arange(len(pos)) % 2 == 0, 1., -1.), device="cuda")
+    alone, mix = torch.zeros_like(pos), torch.zeros_like(pos)
+    b.solve(pos, q, alone, systems=[0])
+    b.solve(pos, q, mix)
+    assert float(alone[:n].abs().max()) > 0.
+    assert torch.equal(alone[:n], mix[:n])
