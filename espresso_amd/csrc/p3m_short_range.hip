@@ -17,6 +17,8 @@ using namespace dev;
 constexpr int kSRMaxCells = 64; // cells per dimension at most (z bins of columns: 4 x)
 constexpr int kColWaves = 4;    // waves per block of k_sr_columns
 constexpr int kSortedSlack = 8; // particles k_sr_columns may read past the sorted ones
+constexpr int kColBatch = 4;    // candidates tested before the lists are looked at
+constexpr int kColRuns = 75;    // runs of candidates of a home group: 25 columns, 3 box images
 
 /** Cell grid: nc cells per dimension of edge L / nc >= r_cut / nsub. */
 struct CellGrid {
@@ -464,7 +466,7 @@ __device__ __forceinline__ void dip_pair(double dx, double dy, double dz, double
  *  run of the sorted particles (split at the periodic boundary).  One block of W waves per home group of 64 sorted
  *  particles of one column: lane = home particle, position and force in
  *  registers; the waves share the runs of the (2 rx + 1)(2 ry + 1) columns,
- *  U candidates at a time, and their forces are added through LDS at the end.
+ *  kColBatch candidates at a time, and their forces are added through LDS at the end.
  *
  *  What bounds it: FP64 VALU issue, first of the distance tests, then of the
  *  pair terms.  A candidate is the same for all lanes, so its position comes
@@ -488,12 +490,14 @@ __global__ __launch_bounds__(kColWaves * 64, DIP ? 3 : EV ? 4 : 5) void k_sr_col
     int const *__restrict__ sidx, double prefactor, double alpha, double rc2,
     double *__restrict__ force, double *__restrict__ torque, double *__restrict__ shares,
     int *__restrict__ arrived, double *__restrict__ partials) {
-  constexpr int W = kColWaves, U = 4, CAP = 24; // waves, candidates per batch, list length
+  constexpr int W = kColWaves, U = kColBatch, CAP = 24; // CAP: list length
   constexpr int NV = DIP ? 6 : 3, NE = DIP ? 1 : 7; // force (and torque); reduced terms
   static_assert(CAP >= 2 * U && CAP * 64 * sizeof(int) >= NV * 64 * sizeof(double));
   __shared__ __align__(16) int list[W][CAP * 64];
   __shared__ double red[8 * 16];
   __shared__ int last;
+  __shared__ int4 runs[kColRuns];
+  __shared__ int nruns;
   int const ngroups = goff[g.nc[0] * g.nc[1]];
   int const b = blockIdx.x, nblocks = ngroups * split;
   if (b >= nblocks) {
@@ -514,6 +518,7 @@ __global__ __launch_bounds__(kColWaves * 64, DIP ? 3 : EV ? 4 : 5) void k_sr_col
   int const me = share * W + wave, all = split * W; // of the group's waves (a power of two)
   bool const home = lane < nh;
   double4 hp = spos[h0 + min(lane, nh - 1)];
+  int64_t const row = 3 * static_cast<int64_t>(sidx[h0 + min(lane, nh - 1)]);
   double const qpi = prefactor * hp.w;
   double4 hm{0., 0., 0., 0.};
   if constexpr (DIP) hm = sdip[h0 + min(lane, nh - 1)];
@@ -589,43 +594,66 @@ __global__ __launch_bounds__(kColWaves * 64, DIP ? 3 : EV ? 4 : 5) void k_sr_col
     slot += (r2 < lim) ? 256 : 0;
   };
 
-  // `sweeps` passes over all columns, each over every sweeps-th batch of a
-  // column's run, the columns out of order: lanes at different corners of the
-  // group then fill their lists at about the same rate
+  // Runs of candidates: first and end particle of every column and box image
+  // along z in reach, and the image.  One lane of the first wave looks up one
+  // of them and the empty ones are dropped: with the look-ups in the loop they
+  // are a chain of loads (100 dipoles 17.1 us, so 14.6; 50,000 77.6 and 73.0)
   int const ncy = 2 * ry + 1, ncols = (2 * rx + 1) * ncy;
+  if (wave == 0) {
+    int n = 0;
+    for (int r0 = 0; r0 < 3 * ncols; r0 += 64) {
+      int const r = r0 + lane, q = r / 3, k = r - 3 * q - 1;
+      int const c = (4 * q) % ncols; // 9, 15 or 25 columns: all of them once
+      int nx = cx + c / ncy - rx, ny = cy + c % ncy - ry, ix = 0, iy = 0;
+      if (nx < 0) { nx += g.nc[0]; ix = -1; } else if (nx >= g.nc[0]) { nx -= g.nc[0]; ix = 1; }
+      if (ny < 0) { ny += g.nc[1]; iy = -1; } else if (ny >= g.nc[1]) { ny -= g.nc[1]; iy = 1; }
+      int const *const off = offsets + (nx * g.nc[1] + ny) * nz;
+      int const lo = max(b0 - rz - k * nz, 0), hi = min(b1 + rz - k * nz, nz - 1);
+      int jb = 0, je = 0;
+      if (r < 3 * ncols && lo <= hi) {
+        jb = off[lo];
+        je = off[hi + 1];
+      }
+      uint64_t const some = __ballot(jb < je);
+      if (jb < je)
+        runs[n + __popcll(some & ((1ull << lane) - 1ull))] =
+            int4{jb, je, ix + 1 + 4 * (iy + 1), k};
+      n += __popcll(some);
+    }
+    if (lane == 0) nruns = n;
+  }
+  __syncthreads();
+
+  // `sweeps` passes over all runs, each over every sweeps-th batch of a run,
+  // the columns out of order: lanes at different corners of the group then fill
+  // their lists at about the same rate
+  int const nr = __builtin_amdgcn_readfirstlane(nruns);
   int turn = 0; // batches so far: batch t goes to wave t % all
   for (int sweep = 0; sweep < sweeps; ++sweep) {
-    for (int q = 0; q < ncols; ++q) {
-      int const c = (4 * q) % ncols; // 9, 15 or 25 columns: all of them once
-      int nx = cx + c / ncy - rx, ny = cy + c % ncy - ry;
-      double sx = 0., sy = 0.;
-      if (nx < 0) { nx += g.nc[0]; sx = -g.L[0]; } else if (nx >= g.nc[0]) { nx -= g.nc[0]; sx = g.L[0]; }
-      if (ny < 0) { ny += g.nc[1]; sy = -g.L[1]; } else if (ny >= g.nc[1]) { ny -= g.nc[1]; sy = g.L[1]; }
-      double const hx = hp.x - sx, hy = hp.y - sy;
-      int const *const off = offsets + (nx * g.nc[1] + ny) * nz;
-      for (int k = -1; k <= 1; ++k) { // box images along z
-        int const lo = max(b0 - rz - k * nz, 0), hi = min(b1 + rz - k * nz, nz - 1);
-        if (hi < lo) continue;
-        int const jb = off[lo] + sweep * U, je = off[hi + 1];
-        double const hz = hp.z - k * g.L[2];
-        int const nb = max(0, (je - jb + sweeps * U - 1) / (sweeps * U));
-        for (int t = (me - turn) & (all - 1); t < nb; t += all) {
-          int const j0 = jb + t * (sweeps * U);
-          // the last batch of a run reads past it, never past the allocation
-          // (kSortedSlack), and lists nothing from there
-          double4 const *const cj = spos + j0;
-          if (j0 + U <= je) {
+    for (int r = 0; r < nr; ++r) {
+      int4 const run = runs[r];
+      int const jb = __builtin_amdgcn_readfirstlane(run.x) + sweep * U;
+      int const je = __builtin_amdgcn_readfirstlane(run.y);
+      int const xy = __builtin_amdgcn_readfirstlane(run.z);
+      int const nb = max(0, (je - jb + sweeps * U - 1) / (sweeps * U));
+      double const hx = hp.x - ((xy & 3) - 1) * g.L[0], hy = hp.y - ((xy >> 2) - 1) * g.L[1],
+                   hz = hp.z - __builtin_amdgcn_readfirstlane(run.w) * g.L[2];
+      for (int t = (me - turn) & (all - 1); t < nb; t += all) {
+        int const j0 = jb + t * (sweeps * U);
+        // the last batch of a run reads past it, never past the allocation
+        // (kSortedSlack), and lists nothing from there
+        double4 const *const cj = spos + j0;
+        if (j0 + U <= je) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) test(hx, hy, hz, cj[u], j0 + u, rc2);
-          } else {
+          for (int u = 0; u < U; ++u) test(hx, hy, hz, cj[u], j0 + u, rc2);
+        } else {
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-              test(hx, hy, hz, cj[u], j0 + u, (j0 + u < je) ? rc2 : -1.);
-          }
-          if (__any(slot > full)) drain(false);
+          for (int u = 0; u < U; ++u)
+            test(hx, hy, hz, cj[u], j0 + u, (j0 + u < je) ? rc2 : -1.);
         }
-        turn += nb;
+        if (__any(slot > full)) drain(false);
       }
+      turn += nb;
     }
   }
   drain(true);
@@ -638,6 +666,21 @@ __global__ __launch_bounds__(kColWaves * 64, DIP ? 3 : EV ? 4 : 5) void k_sr_col
     f[4] = prefactor * (hm.z * h[0] - hm.x * h[2]);
     f[5] = prefactor * (hm.x * h[1] - hm.y * h[0]);
     ev[0] *= prefactor;
+  }
+  // the caller's rows, in flight while the sums are added (nobody else writes
+  // them before this group's last block does)
+  double was[NV] = {};
+  if (wave == 0 && home) {
+    if (!DIP || force) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) was[k] = force[row + k];
+    }
+    if constexpr (DIP) {
+      if (torque) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) was[3 + k] = torque[row + k];
+      }
+    }
   }
   // the waves' sums, in wave order
   double *const own = reinterpret_cast<double *>(list[wave]);
@@ -683,15 +726,14 @@ __global__ __launch_bounds__(kColWaves * 64, DIP ? 3 : EV ? 4 : 5) void k_sr_col
     }
   }
   if (add) {
-    int64_t const i = 3 * static_cast<int64_t>(sidx[h0 + lane]);
     if (!DIP || force) {
 #pragma unroll
-      for (int k = 0; k < 3; ++k) force[i + k] += f[k];
+      for (int k = 0; k < 3; ++k) force[row + k] = was[k] + f[k];
     }
     if constexpr (DIP) {
       if (torque) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) torque[i + k] += f[3 + k];
+        for (int k = 0; k < 3; ++k) torque[row + k] = was[3 + k] + f[3 + k];
       }
     }
   }
@@ -711,7 +753,7 @@ struct Columns {
   int reach[3];
   int ncol, max_groups, split, sweeps;
 };
-Columns make_columns(ShortRangeParams const &p, int64_t n) {
+Columns make_columns(ShortRangeParams const &p, int64_t n, bool exact_erfc = false) {
   Columns c;
   double const per_cut = static_cast<double>(n) * p.r_cut * p.r_cut * p.r_cut /
                          (p.box[0] * p.box[1] * p.box[2]);
@@ -734,18 +776,23 @@ Columns make_columns(ShortRangeParams const &p, int64_t n) {
   // of candidates: twice as many while there are fewer than 4096 blocks, four
   // rounds of what the chip holds (so fewer than 8192 in the end), as long as
   // the lists of one wave still fill: its candidates must be a twentieth of the
-  // number of blocks.  Dipolar and Coulomb kernel, at that
+  // number of blocks, and two batches (a little more with the exact erfc,
+  // whose registers leave three waves per SIMD instead of four: 225 groups of
+  // 800 candidates 33 us in 2 blocks, 35 in 4).  Dipolar and Coulomb kernel, at that
   // split against twice and half of it: 1006 groups of 980 candidates each
   // 84 us in 2 blocks, 103 in 4, 111 in 1; 40 groups of 1900 32 us in 8, 36 in
-  // 16; 321 groups of 16,700 0.62 ms in 16, 0.71 in 8.
+  // 16; 321 groups of 16,700 0.62 ms in 16, 0.71 in 8.  Few candidates, dipoles:
+  // 20 groups of 300 15 us in 8, 16 in 4, 20 in 2; 31 of 230 15 in 4, 17 in 2;
+  // 115 of 120 14.5 in 2, 14.9 in 1.
   double const columns = (2. * c.reach[0] + 1.) * (2. * c.reach[1] + 1.);
   double const in_reach = per_cut / (c.g.nc[0] * c.g.nc[1]) * p.box[0] * p.box[1] /
                           (p.r_cut * p.r_cut); // candidates of one column per r_cut of z
   double const tests = columns * (std::min(64., static_cast<double>(n) / c.ncol) +
                                   2. * in_reach * (1. + 1. / c.reach[2]));
+  double const per_block = exact_erfc ? 0.06 : 0.05;
   c.split = 1;
   while (c.split < 16 && c.max_groups * c.split < 4096 &&
-         tests / (2 * c.split * kColWaves) >= std::max(32., 0.05 * c.max_groups * 2 * c.split))
+         tests / (2 * c.split * kColWaves) >= std::max(2. * kColBatch, per_block * c.max_groups * 2 * c.split))
     c.split *= 2;
   // one pass over the columns per 16 candidates (four batches) that a wave
   // takes of each: with 4 against 16 passes, 200,000 dipoles of 4300 partners
@@ -925,7 +972,7 @@ bool ShortRange::compute_dipolar(hipStream_t st, ShortRangeParams const &p, bool
       return false;
   if (n == 0) return true;
   hip_check(hipSetDevice(m->device), "hipSetDevice");
-  Columns const cols = make_columns(p, n);
+  Columns const cols = make_columns(p, n, exact_erfc);
   CellGrid const &g = cols.g;
   int const ncells = cols.ncol * g.nc[2];
   sr_grow(m->counts, m->cap_cells, static_cast<size_t>(ncells), "hipMalloc cell counts");
