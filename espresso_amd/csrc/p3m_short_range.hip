@@ -475,13 +475,14 @@ __device__ __forceinline__ void dip_pair(double dx, double dy, double dz, double
  *  miss is overwritten by the next candidate), and the pair terms run when a
  *  list is nearly full, with most lanes busy (85 % of them; 42 % when every
  *  list is emptied each time and the columns are swept once, in order).
- *  Measured (250,000 charges, 311 partners each): 0.60 ms, 73 % VALU issue,
+ *  Measured (250,000 charges, 311 partners each): 0.57 ms, 73 % VALU issue,
  *  against 2.94 ms with lanes over the home particles of one r_cut/2 cell,
- *  which kept 10 of 64 lanes busy; 1000 charges: 32 against 89 us.  50,000
- *  dipoles, 66 partners each: 84 us, against 144 with lanes over the home
+ *  which kept 10 of 64 lanes busy; 1000 charges: 27 against 89 us.  50,000
+ *  dipoles, 66 partners each: 77 us, against 144 with lanes over the home
  *  particles of one r_cut cell and a queue of hits per block; 200,000 dipoles
- *  with 105, 420 and 4300 partners (calls): 0.39, 0.91 and 6.9 ms against 0.71,
- *  1.9 and 20. */
+ *  with 100, 420 and 4300 partners (calls): 0.36, 0.86 and 6.8 ms against 0.71,
+ *  1.9 and 20.  Few sparse dipoles are latency: 300 16 against 11 us, 8000 of 33
+ *  partners 26 against 23. */
 template <bool DIP, bool EV, bool EXACT>
 __global__ __launch_bounds__(kColWaves * 64, DIP ? 3 : EV ? 4 : 5) void k_sr_columns(
     CellGrid g, int rx, int ry, int rz, int split, int sweeps, int const *__restrict__ offsets,
