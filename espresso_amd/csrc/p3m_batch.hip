@@ -465,85 +465,111 @@ __global__ __launch_bounds__(kBlock) void k_scatter(SysDesc const *__restrict__ 
 struct BinLds {
   int count[kSmallBins]; // particles per bin, then the start of the bin
   int key[kSmallSystem]; // bin << 14 | rank of every particle, -1 if uncharged
-  double red[8 * 16];
+  double red[7][kSmallSystem / 64]; // sums over 64 consecutive particles
+  double qmax[16];
   int wsum[16];
 };
 
+/** wave_sum of eight values at once, the sum of v[k] in lanes of k = 4 (lane >>
+ *  5 & 1) + 2 (lane >> 4 & 1) + (lane >> 3 & 1): each step sends half of the
+ *  values that are left, 10 exchanges instead of 48.  The same pairs are added
+ *  as by wave_sum, so the sums have its bits. */
+__device__ __forceinline__ double wave_sums8(double const (&v)[8], int lane) {
+  auto step = [lane](double a, double b, int off) { // a in the low lanes, b in the high ones
+    bool const high = lane & off;
+    return (high ? b : a) + __shfl_xor(high ? a : b, off, 64);
+  };
+  double const a0 = step(v[0], v[4], 32), a1 = step(v[1], v[5], 32), a2 = step(v[2], v[6], 32),
+               a3 = step(v[3], v[7], 32);
+  double const b0 = step(a0, a2, 16), b1 = step(a1, a3, 16);
+  double t = step(b0, b1, 8);
+#pragma unroll
+  for (int off = 4; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+  return t;
+}
+
 /** Sorts one system into its bins with one block: bins and ranks from LDS
  *  counters, the scan of the counts, then the sorted arrays; and the system's
- *  sums (n_q, sum q, sum q^2, dipole, sum |q|, max |q|) in a fixed order.  The
- *  work of k_bin, k_scan and k_scatter, which for a small system are three
- *  launches of little else than latency.  Four particles per thread and turn,
- *  their loads in flight together. */
+ *  sums (n_q, sum q, sum q^2, dipole, sum |q|, max |q|), added as k_bin and
+ *  k_scan add them (64 particles, four of those, then all), so that a system
+ *  has the same bits whichever bins it.  The work of k_bin, k_scan and
+ *  k_scatter, which for a small system are three launches of little else than
+ *  latency.  Four particles per thread, their loads in flight together. */
 __device__ void bin_system(SysDesc const &d, int s, int64_t soff, ParticleArrays const &pa,
                            int *p_nmp, int *offsets, double4 *spos, int *sidx, double *sums,
                            int *err_flag, int epoch, BinLds &m) {
-  constexpr int U = 4;
+  constexpr int U = kSmallSystem / kSmallBlock;
+  static_assert(kBlock == 256 && U * kSmallBlock == kSmallSystem);
   int const n = d.n, nb = d.nbricks, tid = threadIdx.x;
+  int const lane = tid & 63, wid = tid >> 6;
   for (int e = tid; e < nb; e += kSmallBlock) m.count[e] = 0;
   __syncthreads();
-  double v[8] = {0., 0., 0., 0., 0., 0., 0., 0.}; // v[7]: max |q|
+  double4 r[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    int const li = tid + u * kSmallBlock;
+    int64_t const i = d.part_off + li;
+    r[u] = li < n ? double4{pa.pos[3 * i], pa.pos[3 * i + 1], pa.pos[3 * i + 2], pa.q[i]}
+                  : double4{0., 0., 0., 0.};
+  }
+  double qmax = 0.;
   bool bad = false;
-  for (int l0 = tid; l0 < n; l0 += U * kSmallBlock) {
-    double4 r[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      int64_t const i = d.part_off + min(l0 + u * kSmallBlock, n - 1);
-      r[u] = double4{pa.pos[3 * i], pa.pos[3 * i + 1], pa.pos[3 * i + 2], pa.q[i]};
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      int const li = l0 + u * kSmallBlock;
-      int nmp[3] = {-1, -1, -1}, key = -1;
-      double const q = r[u].w;
-      if (li < n && q != 0.) {
-        int gi[3];
-        double dist[3];
-        double const x[3] = {r[u].x, r[u].y, r[u].z};
-        if (!particle_coordinates_rt(d.g, d.cao, x, nmp, gi, dist)) bad = true;
-        int const b = particle_bin(d.g, gi);
-        key = (b << 14) | atomicAdd(&m.count[b], 1);
-        double px = x[0], py = x[1], pz = x[2];
-        if (pa.upos) {
-          double const *up = pa.upos + 3 * (d.part_off + li);
-          px = up[0];
-          py = up[1];
-          pz = up[2];
-        }
-        v[0] += 1.;
-        v[1] += q;
-        v[2] += q * q;
-        v[3] += q * px;
-        v[4] += q * py;
-        v[5] += q * pz;
-        v[6] += fabs(q);
-        v[7] = fmax(v[7], fabs(q));
+  for (int u = 0; u < U; ++u) {
+    int const li = tid + u * kSmallBlock;
+    int nmp[3] = {-1, -1, -1}, key = -1;
+    double v[8] = {0., 0., 0., 0., 0., 0., 0., 0.};
+    double const q = r[u].w;
+    if (li < n && q != 0.) {
+      int gi[3];
+      double dist[3];
+      double const x[3] = {r[u].x, r[u].y, r[u].z};
+      if (!particle_coordinates_rt(d.g, d.cao, x, nmp, gi, dist)) bad = true;
+      int const b = particle_bin(d.g, gi);
+      key = (b << 14) | atomicAdd(&m.count[b], 1);
+      double px = x[0], py = x[1], pz = x[2];
+      if (pa.upos) {
+        double const *up = pa.upos + 3 * (d.part_off + li);
+        px = up[0];
+        py = up[1];
+        pz = up[2];
       }
-      if (li < n) {
-        m.key[li] = key;
-        if (p_nmp) {
-          p_nmp[3 * li] = nmp[0];
-          p_nmp[3 * li + 1] = nmp[1];
-          p_nmp[3 * li + 2] = nmp[2];
-        }
+      v[0] = 1.;
+      v[1] = q;
+      v[2] = q * q;
+      v[3] = q * px;
+      v[4] = q * py;
+      v[5] = q * pz;
+      v[6] = fabs(q);
+      qmax = fmax(qmax, v[6]);
+    }
+    if (li < n) {
+      m.key[li] = key;
+      if (p_nmp) {
+        p_nmp[3 * li] = nmp[0];
+        p_nmp[3 * li + 1] = nmp[1];
+        p_nmp[3 * li + 2] = nmp[2];
       }
     }
+    double const t = (u * kSmallBlock < n) ? wave_sums8(v, lane) : 0.; // the same for the block
+    int const k = (lane >> 5 & 1) * 4 + (lane >> 4 & 1) * 2 + (lane >> 3 & 1);
+    if ((lane & 7) == 0 && k < 7) m.red[k][u * (kSmallBlock / 64) + wid] = t;
   }
   if (bad) atomicExch(err_flag, epoch);
-  int const lane = tid & 63, wid = tid >> 6;
 #pragma unroll
-  for (int k = 0; k < 7; ++k) v[k] = wave_sum(v[k]);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v[7] = fmax(v[7], __shfl_xor(v[7], off, 64));
-  if (lane == 0)
-#pragma unroll
-    for (int k = 0; k < 8; ++k) m.red[k * 16 + wid] = v[k];
+  for (int off = 32; off > 0; off >>= 1) qmax = fmax(qmax, __shfl_xor(qmax, off, 64));
+  if (lane == 0) m.qmax[wid] = qmax;
   __syncthreads(); // counts, keys and wave sums complete
-  if (tid < 8) {
+  if (wid < 7) {
+    double p = 0.; // of the 256 particles of a block of k_bin
+    if (lane < kSmallSystem / kBlock)
+      for (int w = 0; w < kBlock / 64; ++w) p += m.red[wid][lane * (kBlock / 64) + w];
+    p = wave_sum(p);
+    if (lane == 0) sums[s * 16 + wid] = p;
+  } else if (tid == 7 * 64) {
     double t = 0.;
-    for (int w = 0; w < kSmallBlock / 64; ++w)
-      t = (tid == 7) ? fmax(t, m.red[tid * 16 + w]) : t + m.red[tid * 16 + w];
-    sums[s * 16 + tid] = t;
+    for (int w = 0; w < kSmallBlock / 64; ++w) t = fmax(t, m.qmax[w]);
+    sums[s * 16 + 7] = t;
   }
   // exclusive scan of the counts, kSmallBins / kSmallBlock per thread
   constexpr int PER = kSmallBins / kSmallBlock;

@@ -160,3 +160,32 @@ def test_noalloc_rejects_oversize_and_missing_setup():
         assert S.rel_rms(f1, f_ref) <= 1e-12 and abs(e1 - e_ref) <= 1e-12 * abs(e_ref)
     finally:
         L.p3m_destroy(ctx)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 256, 257, 1000, 1025, 4095, 4096])
+def test_noalloc_energy_has_the_bits_of_solve(n):
+    """The allocation-free solve bins every system in several launches, the
+    other one bins systems of up to 4096 particles with one block: the same
+    sums, added in the same order (charges and a dipole term without short
+    binary fractions), so forces, energy and virial are equal bit for bit."""
+    import torch
+    from espresso_amd import _lib
+    L = _lib.load()
+    rng = np.random.default_rng(n)
+    Lb = 13.
+    pos = rng.uniform(0., Lb, (n, 3))
+    q = rng.uniform(0.3, 1.7, n) * np.where(np.arange(n) % 2 == 0, 1., -1.)
+    q[5::11] = 0.
+    upos = pos + Lb * rng.integers(-1, 2, (n, 3))
+    pos_t, q_t, upos_t = (torch.tensor(a, device="cuda") for a in (pos, q, upos))
+    pair = torch.tensor([[1., 1., 1.], [4., 5., 6.]], dtype=torch.float64, device="cuda")
+    neutral = torch.tensor([1., -1.], dtype=torch.float64, device="cuda")
+    ctx = _context(L, _lib, [Lb] * 3, pair, neutral, 16, 5, 1.1, 3.2, 0, 3.)
+    flags = _lib.P3M_FORCES | _lib.P3M_ENERGY | _lib.P3M_PRESSURE
+    try:
+        f, e, v = _solve(L, _lib, L.p3m_solve, ctx, pos_t, q_t, upos_t, n, flags)
+        f1, e1, v1 = _solve(L, _lib, L.p3m_solve_noalloc, ctx, pos_t, q_t, upos_t, n, flags)
+        assert np.array_equal(f, f1)
+        assert e == e1 and np.array_equal(v, v1)
+    finally:
+        L.p3m_destroy(ctx)
