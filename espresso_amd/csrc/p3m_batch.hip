@@ -66,8 +66,8 @@ constexpr int kCountCopies = 8; // brick counter copies (one per XCD-sized share
                                 // k_scan reads a brick's copies as two 16-byte words)
 constexpr int kBrick = 8;    // first-stencil points per brick edge
 constexpr int kFill = 4096;  // mesh elements zeroed per block (twice that beside bin_system)
-// systems of up to this many particles and bins are binned by one block of
-// kSmallBlock threads (bin_system), others in four launches.  FP64 solves,
+// selections of systems of up to this many particles and bins are binned by one
+// block of kSmallBlock threads per system (bin_system), others in four launches.  FP64 solves,
 // one block against four launches: 1000 particles 59 against 68 us at mesh 32
 // and 57 against 69 at mesh 16, 4000 66 against 71 and 63 against 81; at mesh
 // 32 the two meet between 6000 (75, 75) and 8000 (77, 75), with fewer bins
@@ -230,9 +230,9 @@ __global__ void k_influence(MT *G, int Mx, int My, int Mz, int Kz, double wx, do
 }
 
 // ---------------------------------------------------------------------------
-// particle binning: systems of up to kSmallSystem particles by one block each
-// (bin_system), larger ones by one block per 256 particles (k_bin, k_scan,
-// k_scatter)
+// particle binning: selections of systems of up to kSmallSystem particles by
+// one block per system (bin_system), others by one block per 256 particles
+// (k_bin, k_scan, k_scatter)
 // ---------------------------------------------------------------------------
 /** Brick (or column bin) of a particle with first stencil point gi. */
 __device__ __forceinline__ int particle_bin(DevGeo const &g, int const gi[3]) {
@@ -330,7 +330,6 @@ __global__ __launch_bounds__(1024) void k_scan(SysDesc const *__restrict__ sys,
   __shared__ int carry;
   __shared__ double red[16 * 8];
   int const slot = blockIdx.x;
-  if (wt_bin[slot] == wt_bin[slot + 1]) return; // binned by bin_system
   int const s = sel[slot];
   SysDesc const &d = sys[s];
   {
@@ -620,27 +619,26 @@ __device__ void bin_system(SysDesc const &d, int s, int64_t soff, ParticleArrays
   }
 }
 
-/** Start of a solve, one launch: nsmall blocks bin the small systems (SMALL),
- *  the others zero the charge mesh (unless it is kept), each block its share of
- *  the system's brick counters.  Selections without small systems take the
- *  instance without bin_system, whose registers leave one block of 1024
+/** Start of a solve, one launch: the first nsmall blocks bin the systems of a
+ *  small selection (SMALL), the others zero the charge mesh (unless it is
+ *  kept) and, for k_bin, each block its share of the system's brick counters.
+ *  Other selections take the instance without bin_system, whose registers leave one block of 1024
  *  threads on a CU, and a part of a mesh is zeroed by the XCD whose spread
  *  blocks add to it: 32 FP64 meshes of 48^3 6.9 us, 9.2 without either, 8.1
  *  without the second. */
 template <typename MT, bool SMALL>
 __global__ __launch_bounds__(SMALL ? kSmallBlock : kBlock) void k_begin(
     SysDesc const *__restrict__ sys, int const *__restrict__ sel, int const *__restrict__ wt,
-    int nsel, int const *__restrict__ small, int nsmall, int const *__restrict__ soff,
-    ParticleArrays pa, int *p_nmp, int *offsets, double4 *spos, int *sidx, double *sums,
-    int *counts, int *err_flag, int epoch, int clear_err, int zero_rho,
-    unsigned long long *stamps) {
+    int nsel, int nsmall, int const *__restrict__ soff, ParticleArrays pa, int *p_nmp,
+    int *offsets, double4 *spos, int *sidx, double *sums, int *counts, int *err_flag, int epoch,
+    int clear_err, int zero_rho, unsigned long long *stamps) {
   constexpr int NTH = SMALL ? kSmallBlock : kBlock, FILL = SMALL ? 2 * kFill : kFill;
   if (blockIdx.x == 0 && threadIdx.x < kStamps)
     stamps[threadIdx.x] = threadIdx.x ? 0ull : static_cast<unsigned long long>(wall_clock64());
   if constexpr (SMALL) {
     extern __shared__ double smem_d[];
     if (static_cast<int>(blockIdx.x) < nsmall) {
-      int const s = small[blockIdx.x];
+      int const s = sel[blockIdx.x];
       bin_system(sys[s], s, soff[s], pa, p_nmp, offsets, spos, sidx, sums, err_flag, epoch,
                  *reinterpret_cast<BinLds *>(smem_d));
       return;
@@ -655,9 +653,7 @@ __global__ __launch_bounds__(SMALL ? kSmallBlock : kBlock) void k_begin(
   SysDesc const &d = sys[sel[slot]];
   if (clear_err && vb == 0 && threadIdx.x == 0) *err_flag = 0;
   int const nblk = wt[slot + 1] - wt[slot];
-  int const nc = (d.n > kSmallSystem || d.nbricks > kSmallBins || clear_err)
-                     ? d.nbricks * kCountCopies
-                     : 0;
+  int const nc = SMALL ? 0 : d.nbricks * kCountCopies;
   int const per = (nc + nblk - 1) / nblk;
   int *c = counts + d.brick_off * kCountCopies;
   for (int e = lb * per + threadIdx.x; e < min(nc, (lb + 1) * per); e += NTH) c[e] = 0;
@@ -2450,8 +2446,7 @@ struct Plan {
       *wt_y = nullptr, *wt_x = nullptr, *wt_yi = nullptr, *wt_f = nullptr, *ycol = nullptr;
   int *wt_part = nullptr; // particle blocks of every system
   int blocks_part = 0;
-  int *d_small = nullptr; // systems binned by bin_system
-  int nsmall = 0;
+  bool small = false; // binned by bin_system
   size_t field_bytes = 0; // y field of the wide fused pass, 0: not for this selection
   int blocks_bin = 0, blocks_fill = 0, blocks_z = 0, blocks_zc = 0, blocks_y = 0, blocks_x = 0,
       blocks_yi = 0, blocks_f = 0;
@@ -3312,22 +3307,22 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
     return std::make_pair(start, acc);
   };
   host.insert(host.end(), sel.begin(), sel.end());
-  // small systems are binned by one block each; not on the fixed lane, whose
-  // error flag is cleared by the launch that would bin them
-  auto const small = [&ln](HostSys const &h) {
-    return !ln.fixed && h.n <= kSmallSystem && h.nbricks <= kSmallBins;
-  };
-  auto const bin = push_prefix([&small](HostSys const &h) {
-    return small(h) ? 0 : static_cast<int>(std::max<int64_t>((h.n + kBlock - 1) / kBlock, 1));
+  // a selection of small systems only is binned by one block per system;
+  // beside larger ones, whose launches are needed anyway, those blocks would
+  // only hold up the first launch (64 systems of 500 to 20,000 particles, FP32:
+  // 382 us, 367 so).  Not on the fixed lane, whose error flag is cleared by the
+  // launch that would bin them
+  p.small = !ln.fixed && std::all_of(sel.begin(), sel.end(), [m](int s) {
+    HostSys const &h = m->sys[s];
+    return h.n <= kSmallSystem && h.nbricks <= kSmallBins;
+  });
+  auto const bin = push_prefix([&p](HostSys const &h) {
+    return p.small ? 0 : static_cast<int>(std::max<int64_t>((h.n + kBlock - 1) / kBlock, 1));
   });
   auto const part = push_prefix([](HostSys const &h) {
     return static_cast<int>((h.n + kBlock - 1) / kBlock);
   });
-  int const small_start = static_cast<int>(host.size());
-  for (int s : sel)
-    if (small(m->sys[s])) host.push_back(s);
-  p.nsmall = static_cast<int>(host.size()) - small_start;
-  int const per_fill = p.nsmall > 0 ? 2 * kFill : kFill;
+  int const per_fill = p.small ? 2 * kFill : kFill;
   auto const fill = push_prefix([per_fill](HostSys const &h) {
     int64_t const R = (int64_t)h.desc.g.M[0] * h.desc.g.M[1] * h.desc.g.M[2];
     return static_cast<int>((R + per_fill - 1) / per_fill);
@@ -3443,7 +3438,6 @@ void build_plan(BatchSolver::Impl *m, Lane &ln, std::vector<int> const &sel, Mes
   p.d_sel = p.dbuf;
   p.wt_part = p.dbuf + part.first;
   p.blocks_part = part.second;
-  p.d_small = p.dbuf + small_start;
   p.wt_bin = p.dbuf + bin.first;
   p.blocks_bin = bin.second;
   p.wt_fill = p.dbuf + fill.first;
@@ -3512,16 +3506,15 @@ void enqueue(BatchSolver::Impl *m, Lane &ln, ParticleArrays const &pa, unsigned 
   bool const zero_rho = !(flags & kSolveAccumulate) && !no_spread;
   ln.epoch = ln.epoch % std::numeric_limits<int>::max() + 1;
   int const epoch = ln.epoch; // of the error flag
-  auto const begin = [&](auto kern, int threads, size_t lds) {
-    kern<<<((p.nsmall + 7) & ~7) + p.blocks_fill, threads, lds, st>>>(
-        sys, p.d_sel, p.wt_fill, ns, p.d_small, p.nsmall, p.soff, pa, p_nmp, ln.offsets, ln.spos,
-        ln.sidx, ln.sums, ln.counts, ln.err_flag, epoch, ln.fixed ? 1 : 0, zero_rho ? 1 : 0,
-        ln.stamps);
+  auto const begin = [&](auto kern, int nsmall, int threads, size_t lds) {
+    kern<<<((nsmall + 7) & ~7) + p.blocks_fill, threads, lds, st>>>(
+        sys, p.d_sel, p.wt_fill, ns, nsmall, p.soff, pa, p_nmp, ln.offsets, ln.spos, ln.sidx,
+        ln.sums, ln.counts, ln.err_flag, epoch, ln.fixed ? 1 : 0, zero_rho ? 1 : 0, ln.stamps);
   };
-  if (p.nsmall > 0)
-    begin(k_begin<MT, true>, kSmallBlock, sizeof(BinLds));
+  if (p.small)
+    begin(k_begin<MT, true>, ns, kSmallBlock, sizeof(BinLds));
   else
-    begin(k_begin<MT, false>, kBlock, 0);
+    begin(k_begin<MT, false>, 0, kBlock, 0);
   if (p.blocks_bin > 0) {
     k_bin<<<p.blocks_bin, kBlock, 0, st>>>(sys, p.d_sel, p.wt_bin, ns, p.soff, pa, ln.counts,
                                             ln.p_brick, ln.p_rank, p_nmp, ln.bin_part,
