@@ -311,13 +311,19 @@ __device__ __forceinline__ bool coordinate_1d(DevGeo const &g, int P, double x, 
   int const n = static_cast<int>(t);
   nmp = n;
   dist = ca_distance(t, n);
-  // an unconditional remainder: with periodic_index the 64 registers of the
-  // cao-3 FP64 gather became 65, three blocks on a CU instead of four (4 10^5
-  // charges, mesh 96: 48 -> 56 us), and column kernels lost waves too
-  int gg = n - g.marg[d];
-  gg %= g.M[d];
-  if (gg < 0) gg += g.M[d];
-  gi = gg;
+  // Up to order 5 an unconditional remainder: with periodic_index the 64
+  // registers of the cao-3 FP64 gather became 65, three blocks on a CU instead
+  // of four (4 10^5 charges, mesh 96: 47 -> 56 us), and gathers in 256-thread
+  // blocks at cao 5 and column kernels lost waves too.  Orders 6 and 7 lose
+  // none and take the shorter form (10^6 charges, cao 7: call 788 -> 785 us)
+  if (P >= 6) {
+    gi = periodic_index(n - g.marg[d], g.M[d]);
+  } else {
+    int gg = n - g.marg[d];
+    gg %= g.M[d];
+    if (gg < 0) gg += g.M[d];
+    gi = gg;
+  }
   return ok;
 }
 
